@@ -127,6 +127,7 @@ def _load_lib():
         "mm_run_bare": (C.c_int64, [vp, C.c_uint64]),
         "mm_push": (C.c_int, [vp]),
         "mm_plan": (C.c_int, [vp, C.POINTER(PlanInfo)]),
+        "mm_step_kernel": (C.c_int, [vp]),
         "mm_free_memory": (C.c_uint64, [vp]),
         "mm_cu_count": (C.c_int, [vp]),
         "mm_max_lds": (C.c_uint64, [vp]),
@@ -344,6 +345,12 @@ class Hip(Backend):
         return {"global": bool(p.global_), "threads": p.threads, "lds_bytes": p.lds_bytes,
                 "slots_per_wg": p.slots_per_wg, "kernel": p.kernel, "tuned": bool(p.tuned),
                 "tile": p.tile, "slots_per_cu": p.slots_per_cu}
+
+    @staticmethod
+    def step_kernel(batch):
+        """The kernel that run() steps the batch with: 32 (matrix cores), 8 or 4 (transforms, as
+        plan_of describes them)."""
+        return lib.mm_step_kernel(batch.state)
 
     @staticmethod
     def run_bare(batch, bits):

@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "../../include/montmul_hip.h"
+#include "mm_mx.h"
 #include "mm_slot_steps.h"
 
 // Device scratch of the allocation-free product (mm_mul_noalloc): the spectrum of one factor and
@@ -608,6 +609,10 @@ struct State {
     F1 *d_nphat1 = nullptr, *d_nhat1 = nullptr, *d_work1 = nullptr;
     F2 *d_nphat2 = nullptr, *d_nhat2 = nullptr, *d_work2 = nullptr;
     F1* d_iwc1 = nullptr;  // unweighting times base (register-transform step)
+    // The matrix-core step (mm_mx.h) runs this batch's steps; its constants, the limbs of every
+    // slot's N', then of every slot's N.
+    bool mx = false;
+    uint32_t* d_nl = nullptr;
     uint32_t* d_coef = nullptr;  // n = 2^14 register step: coefficient staging, 6 n words per slot
     v2::S2* d_iwc2 = nullptr;
     // set_modulus staging (N' and N limbs, the half factors' work vectors), allocated on the
@@ -645,7 +650,7 @@ struct State {
         for (void* p : {(void*)d_x, (void*)d_exp, (void*)d_nbits, (void*)d_pos, (void*)d_err, (void*)d_lim,
                         (void*)d_nphat1, (void*)d_nhat1, (void*)d_work1, (void*)d_nphat2, (void*)d_nhat2, (void*)d_work2,
                         (void*)d_iwc1, (void*)d_iwc2, (void*)d_stage_lim, (void*)d_stage1, (void*)d_stage2, (void*)d_coef,
-                        (void*)d_ones, (void*)d_ones_list, (void*)d_ones_out})
+                        (void*)d_ones, (void*)d_ones_list, (void*)d_ones_out, (void*)d_nl})
             if (p) hipFree(p);
     }
     v2::VArgs vargs() const {
@@ -657,6 +662,17 @@ struct State {
         A.iwc1 = d_iwc1;
         A.iwc2 = d_iwc2;
         A.coef = d_coef;
+        return A;
+    }
+    mx::Args mx_args(bool bare) const {
+        mx::Args A{};
+        A.x = d_x;
+        A.np = d_nl;
+        A.n = d_nl + (size_t)slots * k;
+        A.exp = d_exp; A.nbits = d_nbits; A.pos = d_pos; A.err = d_err;
+        A.lim = bare && global ? d_lim : nullptr;
+        A.ew = ew ? ew : 1;
+        A.base = base;
         return A;
     }
     // The step kernel's arguments: args() plus the radix-4 kernel's LDS tile in global mode.
@@ -978,6 +994,7 @@ int64_t steps(State* S, uint64_t bits, bool bare) {
         float ms = 0;
         if (run_chunks(C, reps,
                        [&]() {
+                           if (S->mx) return mx::launch(S->mx_args(bare), S->k, S->slots, (uint32_t)s, bare, C->stream);
                            if (kern2)
                                hipLaunchKernelGGL(kern2, dim3(S->slots), dim3(S->threads), S->lds, C->stream, A2, 0u, (uint32_t)s);
                            else
@@ -1445,11 +1462,17 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
                         " is not a plan for L = " + std::to_string(st->len));
         set_plan(S.get(), p);
     }
+    // The matrix-core step runs every plan that names no transform kernel, mode or tile of its own
+    // (force_global at n >= 512 is the default plan). Its work grows as n^2: at L = 2,048 it does
+    // 25 M squarings/s against the transforms' 14.4 M; L = 4,096 would take 4.6 K matrix
+    // instructions a step, 37 K cycles of a CU at best against the 88 K that they take there.
+    S->mx = wrap && mx::fits(k, st->base) && !tune && !C->opts.prefer_lds && C->opts.tile == 0 && C->opts.slots_per_cu == 0 &&
+            (v2ok || (!C->opts.force_global && !(kenv && strcmp(kenv, "v1") == 0)));
     // Device memory: x, N'-hat, N-hat or A|B, work vectors and limbs in global mode, exponents
     // of up to k words, per-slot words, the two raw values of 1 with a list word and a flag,
     // tables (about 6n elements per field, twice), a margin.
     const uint64_t per_slot = 4ull * k + 48ull * n + (S->global || tune ? 24ull * n + 12ull * k : 0) + 16 + 4ull * k +
-                              (v2ok && n > 8192 ? 24ull * n : 0) + 8ull * k + 8;
+                              (v2ok && n > 8192 ? 24ull * n : 0) + 8ull * k + 8 + (S->mx ? 8ull * k : 0);
     const uint64_t need = (uint64_t)st->slots * per_slot + 300ull * n + 48ull * n * 2 + (64ull << 20);
     size_t freeb = 0, total = 0;
     if (hipMemGetInfo(&freeb, &total) != hipSuccess) return fail("hipMemGetInfo failed");
@@ -1467,6 +1490,7 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
     S->exp_cap = sl;
     if ((S->global || tune) && (dalloc(&S->d_work1, sl * n) || dalloc(&S->d_work2, sl * n) || dalloc(&S->d_lim, sl * 3 * k)))
         return 1;
+    if (S->mx && dalloc(&S->d_nl, sl * 2 * k)) return 1;
     if (v2ok) {
         if (dalloc(&S->d_iwc1, n) || dalloc(&S->d_iwc2, n)) return 1;
         if (n > 8192 && dalloc(&S->d_coef, sl * 6 * n)) return 1;
@@ -1482,13 +1506,14 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
     HIPCHK(hipMemsetAsync(S->d_exp, 0, sl * 4, sm));
     // Constants: N'-hat by a weighted forward transform; A|B (or N-hat) from N.
     {
-        uint32_t* limbs = nullptr;
-        if (dalloc(&limbs, sl * k)) return 1;
-        std::unique_ptr<uint32_t, void (*)(uint32_t*)> guard(limbs, [](uint32_t* p) { hipFree(p); });
+        uint32_t* limbs = S->d_nl;
+        if (!S->mx && dalloc(&limbs, sl * k)) return 1;
+        std::unique_ptr<uint32_t, void (*)(uint32_t*)> guard(S->mx ? nullptr : limbs, [](uint32_t* p) { hipFree(p); });
         const uint32_t tt = plan_threads(n);
         HIPCHK(hipMemcpyAsync(limbs, st->nprime, sl * k * 4, hipMemcpyHostToDevice, sm));
         hipLaunchKernelGGL(k_load_forward, dim3(st->slots), dim3(tt), 0, sm, S->tab->t, limbs, k, S->d_nphat1, S->d_nphat2);
         HIPCHK(hipGetLastError());
+        if (S->mx) limbs += sl * k;  // N' stays
         HIPCHK(hipMemcpyAsync(limbs, st->n, sl * k * 4, hipMemcpyHostToDevice, sm));
         if (wrap) {
             const uint32_t h = n / 2;
@@ -1569,6 +1594,10 @@ int mm_set_modulus(void* st, size_t i, const uint32_t* nl, const uint32_t* npl, 
     F2* t2 = S->d_stage2;
     HIPCHK(hipMemcpyAsync(lim, npl, (size_t)k * 4, hipMemcpyHostToDevice, sm));
     HIPCHK(hipMemcpyAsync(lim + k, nl, (size_t)k * 4, hipMemcpyHostToDevice, sm));
+    if (S->mx) {
+        HIPCHK(hipMemcpyAsync(S->d_nl + i * k, lim, 4ull * k, hipMemcpyDeviceToDevice, sm));
+        HIPCHK(hipMemcpyAsync(S->d_nl + ((size_t)S->slots + i) * k, lim + k, 4ull * k, hipMemcpyDeviceToDevice, sm));
+    }
     const uint32_t tt = plan_threads(n);
     hipLaunchKernelGGL(k_load_forward, dim3(1), dim3(tt), 0, sm, S->tab->t, lim, k, S->d_nphat1 + i * n, S->d_nphat2 + i * n);
     HIPCHK(hipGetLastError());
@@ -1762,6 +1791,11 @@ int mm_plan(void* st, mm_plan_info* out) {
                               : S->v1_tile;
     out->slots_per_cu = S->slots_per_cu;
     return 0;
+}
+
+int mm_step_kernel(void* st) {
+    const State* S = (const State*)st;
+    return S->mx ? 32 : S->v2 ? 8 : 4;
 }
 
 uint64_t mm_free_memory(void* self) {

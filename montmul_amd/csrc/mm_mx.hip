@@ -1,0 +1,41 @@
+// mm_mx.hip - the matrix-core step kernels of every length they run (L = 16 .. 2,048), in an
+// object of their own.
+
+#include "mm_mx.h"
+
+namespace mm {
+namespace mx {
+
+template <u32 NB, bool BARE>
+__global__ __launch_bounds__(64) void k_steps_mx(Args A, u32 bits) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    steps<NB, BARE>(A, blockIdx.x, bits, threadIdx.x, lds);
+}
+
+// k = 8 .. 1,024 limbs. The limb sums stay below BETA (2^32 - 1) while c n <= 2^20.
+bool fits(u32 k, u32 base) { return k >= 8 && k <= 1024 && (k & (k - 1)) == 0 && (u64)base * 4 * k <= (1u << 20); }
+
+template <u32 NB> static hipError_t go(const Args& A, u32 slots, u32 bits, bool bare, hipStream_t sm) {
+    if (bare)
+        hipLaunchKernelGGL((k_steps_mx<NB, true>), dim3(slots), dim3(64), Lay<NB>::bytes, sm, A, bits);
+    else
+        hipLaunchKernelGGL((k_steps_mx<NB, false>), dim3(slots), dim3(64), Lay<NB>::bytes, sm, A, bits);
+    return hipGetLastError();
+}
+
+hipError_t launch(const Args& A, u32 k, u32 slots, u32 bits, bool bare, hipStream_t sm) {
+    switch (k / 8) {
+        case 1: return go<1>(A, slots, bits, bare, sm);
+        case 2: return go<2>(A, slots, bits, bare, sm);
+        case 4: return go<4>(A, slots, bits, bare, sm);
+        case 8: return go<8>(A, slots, bits, bare, sm);
+        case 16: return go<16>(A, slots, bits, bare, sm);
+        case 32: return go<32>(A, slots, bits, bare, sm);
+        case 64: return go<64>(A, slots, bits, bare, sm);
+        case 128: return go<128>(A, slots, bits, bare, sm);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace mx
+}  // namespace mm
