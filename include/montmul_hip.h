@@ -176,10 +176,10 @@ int64_t mm_run_bare(void *state, uint64_t bits);
 int mm_push(void *state);
 /* Gpu::plan_of (gpu/mod.rs:102-104). */
 int mm_plan(void *state, mm_plan_info *out);
-/* The kernel that mm_run and mm_run_bare step this batch with: 32 = matrix cores (mm_options names
- * no transform plan, and the length and base fit it); else mm_plan's kernel, 4 or 8. mm_plan
- * describes the transform kernels, which run the mixed launch in every case. No reference
- * counterpart. */
+/* The kernel that mm_run and mm_run_bare step this batch with: 32 = matrix cores, 64 =
+ * double-precision transforms (mm_options names no transform plan, and the length and base fit
+ * them); else mm_plan's kernel, 4 or 8. mm_plan describes the modular transform kernels, which run
+ * the mixed launch in every case. No reference counterpart. */
 int mm_step_kernel(void* state);
 /* Gpu::free_memory, sm_count, max_dyn_smem, device_name (gpu/mod.rs:83-99). */
 uint64_t mm_free_memory(void *self);

@@ -348,8 +348,8 @@ class Hip(Backend):
 
     @staticmethod
     def step_kernel(batch):
-        """The kernel that run() steps the batch with: 32 (matrix cores), 8 or 4 (transforms, as
-        plan_of describes them)."""
+        """The kernel that run() steps the batch with: 32 (matrix cores), 64 (double-precision
+        transforms), 8 or 4 (modular transforms, as plan_of describes them)."""
         return lib.mm_step_kernel(batch.state)
 
     @staticmethod

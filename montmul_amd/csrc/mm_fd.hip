@@ -1,0 +1,107 @@
+// mm_fd.hip - the double-precision step kernels of every length they run (L = 4,096 .. 16,384), in an
+// object of their own, and their tables.
+
+#include "mm_fd.h"
+
+#include <algorithm>
+#include <cmath>
+
+namespace mm {
+namespace fd {
+
+// Four waves per SIMD (128 VGPRs): two 512-thread workgroups, or one of 1,024, on a CU.
+template <u32 LOGC, bool BARE>
+__global__ __launch_bounds__(Geo<LOGC>::T) __attribute__((amdgpu_waves_per_eu(4))) void k_steps_fd(Args A, u32 bits) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    steps<LOGC, BARE>(A, blockIdx.x, bits, lds);
+}
+
+template <u32 LOGC>
+__global__ __launch_bounds__(Geo<LOGC>::T) __attribute__((amdgpu_waves_per_eu(4))) void k_constants_fd(Args A, const u32* npl, const u32* nl,
+                                                                                                  double2* np, double2* nh) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    typedef Slot<LOGC> S;
+    const size_t v = blockIdx.x;
+    constants<LOGC>(A, npl + v * S::k, nl + v * S::k, np + v * S::C, nh + v * S::H, lds);
+}
+
+// k = 2,048 .. 8,192 limbs; c C <= 2^16 keeps the limb sums of T below BETA (2^32 - 1).
+bool fits(u32 k, u32 base) { return (k == 2048 || k == 4096 || k == 8192) && (u64)base * 2 * k <= 65536; }
+
+void make_tables(u32 C, double2* out) {
+    auto unit = [](u64 num, u64 den) {  // exp(2 pi i num / den), den a power of two >= 8
+        // The octant's sine and cosine, so that both are rounded from small angles.
+        num %= den;
+        const u64 q = num / (den / 4), r = num % (den / 4);
+        const bool flip = r > den / 8;
+        const long double a = 2 * 3.14159265358979323846264338327950288L * (long double)(flip ? den / 4 - r : r) / (long double)den;
+        double c = (double)cosl(a), s = (double)sinl(a);
+        if (flip) std::swap(c, s);
+        switch (q) {
+            case 0: return make_double2(c, s);
+            case 1: return make_double2(-s, c);
+            case 2: return make_double2(-c, -s);
+            default: return make_double2(s, -c);
+        }
+    };
+    const u32 T = C / 16, S1 = C / 256, S2 = C / 4096;
+    for (u32 a = 0; a < 4; a++)
+        for (u32 t = 0; t < T; t++) out[a * T + t] = unit((u64)t * (16 * a + 1), 4ull * C);
+    for (u32 b = 1; b < 4; b++)
+        for (u32 t = 0; t < T; t++) out[(3 + b) * T + t] = unit((u64)t * b, C);
+    out += 7 * T;
+    for (u32 m = 0; m < 16; m++)
+        for (u32 j = 0; j < S1; j++) out[m * S1 + j] = unit((u64)j * m, T);
+    out += C / 16;
+    for (u32 m = 0; m < 16; m++)
+        for (u32 j = 0; j < S2; j++) out[m * S2 + j] = unit((u64)j * m, S1);
+}
+
+template <u32 LOGC> static hipError_t limit() {
+    for (const void* k : {(const void*)k_steps_fd<LOGC, false>, (const void*)k_steps_fd<LOGC, true>, (const void*)k_constants_fd<LOGC>}) {
+        const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Geo<LOGC>::lds);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+hipError_t set_lds_limit() {
+    hipError_t e = limit<12>();
+    if (e == hipSuccess) e = limit<13>();
+    if (e == hipSuccess) e = limit<14>();
+    return e;
+}
+
+template <u32 LOGC> static hipError_t go(const Args& A, u32 slots, u32 bits, bool bare, hipStream_t sm) {
+    typedef Geo<LOGC> G;
+    if (bare)
+        hipLaunchKernelGGL((k_steps_fd<LOGC, true>), dim3(slots), dim3(G::T), G::lds, sm, A, bits);
+    else
+        hipLaunchKernelGGL((k_steps_fd<LOGC, false>), dim3(slots), dim3(G::T), G::lds, sm, A, bits);
+    return hipGetLastError();
+}
+hipError_t launch(const Args& A, u32 k, u32 slots, u32 bits, bool bare, hipStream_t sm) {
+    switch (k) {
+        case 2048: return go<12>(A, slots, bits, bare, sm);
+        case 4096: return go<13>(A, slots, bits, bare, sm);
+        case 8192: return go<14>(A, slots, bits, bare, sm);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+template <u32 LOGC>
+static hipError_t consts(const Args& A, u32 count, const u32* npl, const u32* nl, double2* np, double2* nh, hipStream_t sm) {
+    typedef Geo<LOGC> G;
+    hipLaunchKernelGGL((k_constants_fd<LOGC>), dim3(count), dim3(G::T), G::lds, sm, A, npl, nl, np, nh);
+    return hipGetLastError();
+}
+hipError_t launch_constants(const Args& A, u32 k, u32 count, const u32* npl, const u32* nl, double2* np, double2* nh, hipStream_t sm) {
+    switch (k) {
+        case 2048: return consts<12>(A, count, npl, nl, np, nh, sm);
+        case 4096: return consts<13>(A, count, npl, nl, np, nh, sm);
+        case 8192: return consts<14>(A, count, npl, nl, np, nh, sm);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace fd
+}  // namespace mm

@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "../../include/montmul_hip.h"
+#include "mm_fd.h"
 #include "mm_mx.h"
 #include "mm_slot_steps.h"
 
@@ -479,6 +480,16 @@ struct DevTables {
     }
 };
 
+// Twiddles of the double-precision transforms of one complex length.
+struct FdTables {
+    double2* p = nullptr;
+    int device = 0;
+    ~FdTables() {
+        hipSetDevice(device);
+        hipFree(p);
+    }
+};
+
 // A launch plan the autotuner can choose: kernel (register radix-8 or radix-4), mode (global or
 // LDS-resident), the register kernel's exchange tile in global mode (1: its default) and slots
 // per CU (0: as many as fit; 1: one, by padding the workgroup's LDS past half a CU's).
@@ -506,6 +517,7 @@ struct Ctx {
     std::string name;
     std::mutex mu;
     std::map<uint32_t, std::shared_ptr<DevTables>> tabs;
+    std::map<uint32_t, std::shared_ptr<FdTables>> fd_tabs;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // This device's copy of the fixed product scratch (null, with scratch_err, if its address
     // could not be taken).
@@ -595,6 +607,22 @@ int get_tables(Ctx* C, uint32_t n, std::shared_ptr<DevTables>* out) {
     return 0;
 }
 
+// The double-precision transforms' twiddles at complex length len, built and uploaded on first use.
+int get_fd_tables(Ctx* C, uint32_t len, std::shared_ptr<FdTables>* out) {
+    std::lock_guard<std::mutex> g(C->mu);
+    auto it = C->fd_tabs.find(len);
+    if (it != C->fd_tabs.end()) { *out = it->second; return 0; }
+    auto D = std::make_shared<FdTables>();
+    D->device = C->device;
+    std::vector<double2> h(fd::table_elems(len));
+    fd::make_tables(len, h.data());
+    HIPCHK(hipMalloc((void**)&D->p, h.size() * sizeof(double2)));
+    HIPCHK(hipMemcpy(D->p, h.data(), h.size() * sizeof(double2), hipMemcpyHostToDevice));
+    C->fd_tabs[len] = D;
+    *out = D;
+    return 0;
+}
+
 struct State {
     Ctx* C = nullptr;
     int device = 0;  // C's device, kept so that a state can be freed after its context is closed
@@ -613,6 +641,10 @@ struct State {
     // slot's N', then of every slot's N.
     bool mx = false;
     uint32_t* d_nl = nullptr;
+    // The double-precision step (mm_fd.h) runs them; the spectra of N' and N.
+    bool fd = false;
+    std::shared_ptr<FdTables> fd_tab;
+    double2 *d_fnp = nullptr, *d_fn = nullptr;
     uint32_t* d_coef = nullptr;  // n = 2^14 register step: coefficient staging, 6 n words per slot
     v2::S2* d_iwc2 = nullptr;
     // set_modulus staging (N' and N limbs, the half factors' work vectors), allocated on the
@@ -650,7 +682,8 @@ struct State {
         for (void* p : {(void*)d_x, (void*)d_exp, (void*)d_nbits, (void*)d_pos, (void*)d_err, (void*)d_lim,
                         (void*)d_nphat1, (void*)d_nhat1, (void*)d_work1, (void*)d_nphat2, (void*)d_nhat2, (void*)d_work2,
                         (void*)d_iwc1, (void*)d_iwc2, (void*)d_stage_lim, (void*)d_stage1, (void*)d_stage2, (void*)d_coef,
-                        (void*)d_ones, (void*)d_ones_list, (void*)d_ones_out, (void*)d_nl})
+                        (void*)d_ones, (void*)d_ones_list, (void*)d_ones_out, (void*)d_nl,
+                        (void*)d_fnp, (void*)d_fn})
             if (p) hipFree(p);
     }
     v2::VArgs vargs() const {
@@ -671,6 +704,18 @@ struct State {
         A.n = d_nl + (size_t)slots * k;
         A.exp = d_exp; A.nbits = d_nbits; A.pos = d_pos; A.err = d_err;
         A.lim = bare && global ? d_lim : nullptr;
+        A.ew = ew ? ew : 1;
+        A.base = base;
+        return A;
+    }
+    fd::Args fd_args() const {
+        fd::Args A{};
+        A.w = fd::tables_at(fd_tab->p, len);
+        A.x = d_x;
+        A.np = d_fnp;
+        A.n = d_fn;
+        A.exp = d_exp; A.nbits = d_nbits; A.pos = d_pos; A.err = d_err;
+        A.lim = d_lim;
         A.ew = ew ? ew : 1;
         A.base = base;
         return A;
@@ -794,6 +839,7 @@ int set_lds_limit(Ctx* C) {
         }
         C->max_dyn_lds_v2 = std::min(C->max_dyn_lds_v2 ? C->max_dyn_lds_v2 : dyn, dyn);
     }
+    HIPCHK(fd::set_lds_limit());
     HIPCHK(mix_lds_limit<512>(C->max_lds, &C->max_dyn_lds_mix[0]));
     HIPCHK(mix_lds_limit<1024>(C->max_lds, &C->max_dyn_lds_mix[1]));
     C->max_dyn_lds = dyn_max;
@@ -995,6 +1041,7 @@ int64_t steps(State* S, uint64_t bits, bool bare) {
         if (run_chunks(C, reps,
                        [&]() {
                            if (S->mx) return mx::launch(S->mx_args(bare), S->k, S->slots, (uint32_t)s, bare, C->stream);
+                           if (S->fd) return fd::launch(S->fd_args(), S->k, S->slots, (uint32_t)s, bare, C->stream);
                            if (kern2)
                                hipLaunchKernelGGL(kern2, dim3(S->slots), dim3(S->threads), S->lds, C->stream, A2, 0u, (uint32_t)s);
                            else
@@ -1415,6 +1462,7 @@ void mm_hip_close(mm_backend* be) {
     if (!C) return;
     hipSetDevice(C->device);
     C->tabs.clear();
+    C->fd_tabs.clear();
     if (C->mix_buf) hipFree(C->mix_buf);
     if (C->ev0) hipEventDestroy(C->ev0);
     if (C->ev1) hipEventDestroy(C->ev1);
@@ -1462,17 +1510,20 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
                         " is not a plan for L = " + std::to_string(st->len));
         set_plan(S.get(), p);
     }
-    // The matrix-core step runs every plan that names no transform kernel, mode or tile of its own
+    // The matrix-core step and the double-precision step run every plan that names no transform
+    // kernel, mode or tile of its own
     // (force_global at n >= 512 is the default plan). Its work grows as n^2: at L = 2,048 it does
     // 25 M squarings/s against the transforms' 14.4 M; L = 4,096 would take 4.6 K matrix
-    // instructions a step, 37 K cycles of a CU at best against the 88 K that they take there.
-    S->mx = wrap && mx::fits(k, st->base) && !tune && !C->opts.prefer_lds && C->opts.tile == 0 && C->opts.slots_per_cu == 0 &&
-            (v2ok || (!C->opts.force_global && !(kenv && strcmp(kenv, "v1") == 0)));
+    // instructions a step, 37 K cycles of a CU at best, where the double-precision step takes 39 K.
+    const bool unnamed = wrap && !tune && !C->opts.prefer_lds && C->opts.tile == 0 && C->opts.slots_per_cu == 0 &&
+                         (v2ok || (!C->opts.force_global && !(kenv && strcmp(kenv, "v1") == 0)));
+    S->mx = unnamed && mx::fits(k, st->base);
+    S->fd = unnamed && !S->mx && S->global && fd::fits(k, st->base);  // T goes through HBM
     // Device memory: x, N'-hat, N-hat or A|B, work vectors and limbs in global mode, exponents
     // of up to k words, per-slot words, the two raw values of 1 with a list word and a flag,
     // tables (about 6n elements per field, twice), a margin.
     const uint64_t per_slot = 4ull * k + 48ull * n + (S->global || tune ? 24ull * n + 12ull * k : 0) + 16 + 4ull * k +
-                              (v2ok && n > 8192 ? 24ull * n : 0) + 8ull * k + 8 + (S->mx ? 8ull * k : 0);
+                              (v2ok && n > 8192 ? 24ull * n : 0) + 8ull * k + 8 + (S->mx ? 8ull * k : 0) + (S->fd ? 48ull * n : 0);
     const uint64_t need = (uint64_t)st->slots * per_slot + 300ull * n + 48ull * n * 2 + (64ull << 20);
     size_t freeb = 0, total = 0;
     if (hipMemGetInfo(&freeb, &total) != hipSuccess) return fail("hipMemGetInfo failed");
@@ -1491,6 +1542,8 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
     if ((S->global || tune) && (dalloc(&S->d_work1, sl * n) || dalloc(&S->d_work2, sl * n) || dalloc(&S->d_lim, sl * 3 * k)))
         return 1;
     if (S->mx && dalloc(&S->d_nl, sl * 2 * k)) return 1;
+    if (S->fd && (get_fd_tables(C, st->len, &S->fd_tab) || dalloc(&S->d_fnp, sl * st->len) || dalloc(&S->d_fn, sl * (st->len / 2))))
+        return 1;
     if (v2ok) {
         if (dalloc(&S->d_iwc1, n) || dalloc(&S->d_iwc2, n)) return 1;
         if (n > 8192 && dalloc(&S->d_coef, sl * 6 * n)) return 1;
@@ -1507,14 +1560,15 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
     // Constants: N'-hat by a weighted forward transform; A|B (or N-hat) from N.
     {
         uint32_t* limbs = S->d_nl;
-        if (!S->mx && dalloc(&limbs, sl * k)) return 1;
+        if (!S->mx && dalloc(&limbs, sl * k * (S->fd ? 2 : 1))) return 1;
         std::unique_ptr<uint32_t, void (*)(uint32_t*)> guard(S->mx ? nullptr : limbs, [](uint32_t* p) { hipFree(p); });
         const uint32_t tt = plan_threads(n);
         HIPCHK(hipMemcpyAsync(limbs, st->nprime, sl * k * 4, hipMemcpyHostToDevice, sm));
         hipLaunchKernelGGL(k_load_forward, dim3(st->slots), dim3(tt), 0, sm, S->tab->t, limbs, k, S->d_nphat1, S->d_nphat2);
         HIPCHK(hipGetLastError());
-        if (S->mx) limbs += sl * k;  // N' stays
+        if (S->mx || S->fd) limbs += sl * k;  // N' stays
         HIPCHK(hipMemcpyAsync(limbs, st->n, sl * k * 4, hipMemcpyHostToDevice, sm));
+        if (S->fd) HIPCHK(fd::launch_constants(S->fd_args(), k, st->slots, limbs - sl * k, limbs, S->d_fnp, S->d_fn, sm));
         if (wrap) {
             const uint32_t h = n / 2;
             F1 c1 = cinv(F1{mod1(8 * h), 0});
@@ -1598,6 +1652,7 @@ int mm_set_modulus(void* st, size_t i, const uint32_t* nl, const uint32_t* npl, 
         HIPCHK(hipMemcpyAsync(S->d_nl + i * k, lim, 4ull * k, hipMemcpyDeviceToDevice, sm));
         HIPCHK(hipMemcpyAsync(S->d_nl + ((size_t)S->slots + i) * k, lim + k, 4ull * k, hipMemcpyDeviceToDevice, sm));
     }
+    if (S->fd) HIPCHK(fd::launch_constants(S->fd_args(), k, 1, lim, lim + k, S->d_fnp + i * S->len, S->d_fn + i * (S->len / 2), sm));
     const uint32_t tt = plan_threads(n);
     hipLaunchKernelGGL(k_load_forward, dim3(1), dim3(tt), 0, sm, S->tab->t, lim, k, S->d_nphat1 + i * n, S->d_nphat2 + i * n);
     HIPCHK(hipGetLastError());
@@ -1795,7 +1850,7 @@ int mm_plan(void* st, mm_plan_info* out) {
 
 int mm_step_kernel(void* st) {
     const State* S = (const State*)st;
-    return S->mx ? 32 : S->v2 ? 8 : 4;
+    return S->mx ? 32 : S->fd ? 64 : S->v2 ? 8 : 4;
 }
 
 uint64_t mm_free_memory(void* self) {
