@@ -247,7 +247,7 @@ def to_limbs(x, k=None):
 
 
 def from_limbs(buf):
-    return int.from_bytes(bytes(buf), "little")
+    return int.from_bytes(buf, "little")
 
 
 def _sign(x):

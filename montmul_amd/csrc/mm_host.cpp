@@ -33,18 +33,28 @@ struct Mpz {
     ~Mpz() { mpz_clear(v); }
 };
 
+// GMP's limbs are pairs of ours in memory order (64-bit, little-endian), so conversions are copies;
+// mpz_import and mpz_export go word by word.
+static_assert(sizeof(mp_limb_t) == 8 && GMP_NAIL_BITS == 0, "64-bit GMP limbs");
+
 void from_signed_limbs(mpz_t z, int sign, const uint32_t* l, size_t nl) {
-    mpz_import(z, nl, -1, 4, 0, 0, l);
-    if (sign < 0) mpz_neg(z, z);
+    const mp_size_t n = (mp_size_t)((nl + 1) / 2);
+    if (n == 0) { mpz_set_ui(z, 0); return; }
+    mp_limb_t* d = mpz_limbs_write(z, n);
+    d[n - 1] = 0;
+    memcpy(d, l, nl * 4);
+    mpz_limbs_finish(z, sign < 0 ? -n : n);
 }
 
 // to_limbs (batch.rs:34-39): k little-endian limbs; fails when the value does not fit.
 bool to_limbs(const mpz_t z, uint32_t* out, size_t k) {
-    memset(out, 0, k * 4);
-    if (mpz_sgn(z) < 0 || mpz_sizeinbase(z, 2) > 32 * k) return false;
-    if (mpz_sgn(z) == 0) return true;
-    size_t cnt = 0;
-    mpz_export(out, &cnt, -1, 4, 0, 0, z);
+    if (mpz_sgn(z) < 0 || (mpz_sgn(z) && mpz_sizeinbase(z, 2) > 32 * k)) {
+        memset(out, 0, k * 4);
+        return false;
+    }
+    const size_t bytes = std::min(k * 4, mpz_size(z) * 8);
+    if (bytes) memcpy(out, mpz_limbs_read(z), bytes);
+    memset((unsigned char*)out + bytes, 0, k * 4 - bytes);
     return true;
 }
 
@@ -286,10 +296,13 @@ int mm_modbatch_load(mm_modbatch* b, size_t i, int sign, const uint32_t* limbs, 
     const MmModulus& m = b->moduli[i];
     Mpz x;
     from_signed_limbs(x.v, sign, limbs, nl);
-    mpz_mul(x.v, x.v, m.r.v);
-    mpz_mod(x.v, x.v, m.n.v);
+    const bool one = mpz_cmp_ui(x.v, 1) == 0;  // 1 R mod N is at hand (Fermat tests start there)
+    if (!one) {
+        mpz_mul(x.v, x.v, m.r.v);
+        mpz_mod(x.v, x.v, m.n.v);
+    }
     std::vector<uint32_t> l(b->k);
-    to_limbs(x.v, l.data(), b->k);
+    to_limbs(one ? m.r.v : x.v, l.data(), b->k);
     if (b->be.load(b->state, i, l.data())) return fail(b->be.last_error());
     return 0;
 }
@@ -314,9 +327,11 @@ int mm_modbatch_set_exponent(mm_modbatch* b, size_t i, int sign, const uint32_t*
     Mpz e;
     from_signed_limbs(e.v, sign, limbs, nl);
     size_t nbits = significant_bits(e.v);
+    // Bit nbits - 1 at the top of the first word: e shifted up to whole words, highest word first.
     std::vector<uint32_t> words((nbits + 31) / 32, 0);
-    for (size_t p = 0; p < nbits; p++)
-        if (mpz_tstbit(e.v, nbits - 1 - p)) words[p / 32] |= 1u << (31 - p % 32);
+    mpz_mul_2exp(e.v, e.v, 32 * words.size() - nbits);
+    to_limbs(e.v, words.data(), words.size());
+    std::reverse(words.begin(), words.end());
     if (b->be.set_exponent(b->state, i, words.data(), words.size(), nbits)) return fail(b->be.last_error());
     return 0;
 }
@@ -365,7 +380,7 @@ int mm_modbatch_read(mm_modbatch* b, size_t i, uint32_t* out) {  // batch.rs:173
     if (mm_modbatch_read_raw(b, i, out)) return 1;
     const MmModulus& m = b->moduli[i];
     Mpz x;
-    mpz_import(x.v, b->k, -1, 4, 0, 0, out);
+    from_signed_limbs(x.v, 1, out, b->k);
     mpz_mul(x.v, x.v, m.rinv.v);
     mpz_mod(x.v, x.v, m.n.v);
     to_limbs(x.v, out, b->k);
