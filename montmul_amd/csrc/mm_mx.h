@@ -6,8 +6,9 @@
 // row i0 of a 32-row Toeplitz matrix of a times column i1 of the matrix whose columns are the
 // 32-digit blocks of b. v_mfma_i32_32x32x32_i8 takes 32 values of j at a time: the a operand at
 // step kappa (j = -32 kappa .. -32 kappa + 31) is the Toeplitz block a[32 kappa + i0 - j'], the b
-// operand is the 32 consecutive blocks of b from i1 - kappa, 1 KiB contiguous in LDS. Sums are
-// exact in 32 bits (n 2^14 <= 2^26).
+// operand is the 32 consecutive blocks of b from i1 - kappa, which the LDS holds in two planes (the
+// blocks' first and second 16 bytes), each lane's 16 bytes next to its neighbour's: with whole blocks
+// 32 bytes apart every read took two cycles for one. Sums are exact in 32 bits (n 2^14 <= 2^26).
 //
 // One wave steps one slot: no barrier anywhere. A step (R = 2^(32k) = 256^n) is
 //     T = c x^2                              2n columns
@@ -25,10 +26,11 @@
 // them nonnegative through the carry.
 //
 // Measured against the transform kernels it replaces by default (4,096 slots unless said):
-// L = 1,024 30.6 -> 79 M squarings/s, 2,048 (2,048 slots) 14.4 -> 25 M; one step of a slot among 64
-// at L = 512 59 -> 6.4 us, of one among 16 at L = 256 53 -> 3.5 us (the radix-4 kernel's barriers).
-// At L = 1,024 LDS reads bind (77 % busy, a quarter of it bank conflicts), then the matrix cores
-// (52 %, at the 1.74 GHz that dense int8 products leave of the clock).
+// L = 1,024 30.6 -> 91 M squarings/s, 2,048 (2,048 slots) 14.4 -> 30 M; one step of a slot among 64
+// at L = 512 59 -> 5.6 us, of one among 16 at L = 256 53 -> 2.8 us (the radix-4 kernel's barriers).
+// At L = 1,024 power binds as much as issue: a loop of these instructions alone on random digits
+// runs at 1.64 of 2.4 GHz, this kernel with its matrix cores 60 % busy at 1.75. Before the planes, the
+// fragments loaded two steps ahead and eight waves a CU it was 79 M.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -61,15 +63,18 @@ struct Args {
 };
 
 // LDS of one slot in bytes, for NB blocks of 32 digits (k = 8 NB limbs). Operands stand between
-// 1 KiB of zeros, so that fragments past either end read zeros.
+// zeros, so that fragments past either end read zeros: 64 bytes for the Toeplitz operand, 32
+// blocks for the other one.
 template <u32 NB> struct Lay {
-    static constexpr u32 n = 32 * NB, k = 8 * NB, pad = 1024;
-    static constexpr u32 op = pad;           // x, T mod R and m in turn
-    static constexpr u32 np = op + n + pad;  // N'
-    static constexpr u32 nn = np + n + pad;  // N
-    static constexpr u32 st = nn + n + pad;  // limb sums, 9 words of 8 bytes per 8 limbs
-    static constexpr u32 th = st + 9 * k;    // floor(T / R), past the sums of k limbs
-    static constexpr u32 bytes = st + 18 * k;
+    static constexpr u32 n = 32 * NB, k = 8 * NB, pad = 512;
+    static constexpr u32 op = 64;                            // x, T mod R and m in turn, in order
+    static constexpr u32 pl = op + n + 64;                   // two planes of x, N' and N
+    static constexpr u32 plane = 4 * pad + 3 * (n / 2);
+    static constexpr u32 xb = pl + pad, np = xb + n / 2 + pad, nn = np + n / 2 + pad;
+    static constexpr u32 st = pl + 2 * plane;                // limb sums, 9 words of 8 bytes per 8 limbs
+    static constexpr u32 bytes = st + 9 * k;
+    // Limb q of the planes' operand at `area` (q = -1: zeros).
+    static __device__ __forceinline__ u32 at(u32 area, int q) { return area + plane * ((u32)q >> 2 & 1) + 16 * (u32)(q >> 3) + 4 * ((u32)q & 3); }
 };
 
 // Orders a wave's LDS accesses across lanes (the LDS pipeline itself is in order per wave).
@@ -94,7 +99,10 @@ __device__ __forceinline__ v4i perm_a(const FragA& f, u32 sel) {
     for (u32 u = 0; u < 4; u++) r[u] = (int)__builtin_amdgcn_perm(f.d[4 - u], f.d[3 - u], sel);
     return r;
 }
-__device__ __forceinline__ v4i load_b(const unsigned char* b, int delta) { return *(const v4i*)(b + 32 * delta); }
+__device__ __forceinline__ v4i load_b(const unsigned char* b, int delta) { return *(const v4i*)(b + 16 * delta); }
+// Keeps loads ahead of the matrix instructions that they are meant to overlap: the scheduler moves
+// them down to their first use.
+__device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
 __device__ __forceinline__ v16i mfma(v4i a, v4i b, v16i c) { return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0); }
 
 // Per-lane constants of the fragments.
@@ -104,8 +112,8 @@ struct Lane {
         const u32 r = j & 3;
         sel = 0x01020304u + 0x01010101u * r;
     }
-    __device__ __forceinline__ const u32* a(const unsigned char* p) const { return (const u32*)p + (j >> 2) - 4 * h - 4 + 0; }
-    __device__ __forceinline__ const unsigned char* b(const unsigned char* p) const { return p + 32 * j + 16 * h; }
+    __device__ __forceinline__ const u32* a(const unsigned char* p) const { return (const u32*)p + (j >> 2) - 4 * h - 4; }
+    __device__ __forceinline__ const unsigned char* b(const unsigned char* p, u32 plane) const { return p + 16 * j + plane * h; }
 };
 
 // Output tiles LO .. HI-1 (1,024 digits each) of the product of two n-digit strings, n >= 1,024.
@@ -117,7 +125,7 @@ template <u32 NB, u32 LO, u32 HI>
 __device__ __forceinline__ void product(const Lane& L, const unsigned char* A, const unsigned char* B, v16i* acc) {
     constexpr int Q = NB / 32;
     const u32* pa = L.a(A);
-    const unsigned char* pb = L.b(B);
+    const unsigned char* pb = L.b(B, Lay<NB>::plane);
 #pragma unroll
     for (u32 c = 0; c < HI - LO; c++)
 #pragma unroll
@@ -133,17 +141,32 @@ __device__ __forceinline__ void product(const Lane& L, const unsigned char* A, c
         for (int p = 0; p <= Q; p++)
             if (need(p, Q - 1)) F.b[p] = load_b(pb, 32 * p - (int)t);
     };
-    auto mult = [&](const Frags& F) {
+    // A step of the loop: the matrix instructions of t (its a fragments selected already), between
+    // them the loads of t + 2 and the selection of t + 1, whose loads came a step ago.
+    v4i s0[Q], s1[Q];
+    auto select = [&](v4i* s, const Frags& F) {
 #pragma unroll
         for (int q = 0; q < Q; q++)
-            if (need(q, Q)) {
-                const v4i a = perm_a(F.a[q], L.sel);
-#pragma unroll
-                for (int p = 0; p <= Q; p++)
-                    if (q + p >= (int)LO && q + p < (int)HI) acc[q + p - LO] = mfma(a, F.b[p], acc[q + p - LO]);
-            }
+            if (need(q, Q)) s[q] = perm_a(F.a[q], L.sel);
     };
-    Frags F0, F1;
+    auto mult = [&](const v4i* s, const Frags& F) {
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+#pragma unroll
+            for (int p = 0; p <= Q; p++)
+                if (q + p >= (int)LO && q + p < (int)HI) acc[q + p - LO] = mfma(s[q], F.b[p], acc[q + p - LO]);
+    };
+    constexpr int MFMAS = HI - LO == 2 * Q ? Q * (Q + 1) : Q * (Q + 1) / 2;
+    auto interleave = [] {
+#pragma unroll
+        for (int i = 0; i < MFMAS; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a matrix instruction
+            __builtin_amdgcn_sched_group_barrier(0x002, (4 * Q + MFMAS - 1) / MFMAS, 0);  // selections
+            __builtin_amdgcn_sched_group_barrier(0x100, (4 * Q + 1 + MFMAS - 1) / MFMAS, 0);  // LDS reads
+        }
+        fence();
+    };
+    Frags F0, F1, F2;
     // t = 0: the a fragments 0, 32, .. n / 32 against the b fragments 0, 32, .. (the one past
     // the end is zero).
 #pragma unroll
@@ -151,6 +174,7 @@ __device__ __forceinline__ void product(const Lane& L, const unsigned char* A, c
 #pragma unroll
     for (int p = 0; p < Q; p++) F0.b[p] = load_b(pb, 32 * p);
     load(F1, 1);
+    fence();
 #pragma unroll
     for (int q = 0; q <= Q; q++) {
         const v4i a = perm_a(F0.a[q], L.sel);
@@ -158,47 +182,76 @@ __device__ __forceinline__ void product(const Lane& L, const unsigned char* A, c
         for (int p = 0; p < Q; p++)
             if (q + p >= (int)LO && q + p < (int)HI) acc[q + p - LO] = mfma(a, F0.b[p], acc[q + p - LO]);
     }
+    load(F2, 2);
+    select(s0, F1);
+    fence();
+    // t = 1 .. 31, three at a time (three sets of fragments in turn; loads past t = 31 are not used, and
+    // read the operands' next blocks or zeros).
 #pragma nounroll
-    for (u32 t = 1; t < 31; t += 2) {
-        load(F0, t + 1);
-        mult(F1);
-        load(F1, t + 2);
-        mult(F0);
+    for (u32 t = 1; t < 31; t += 3) {
+        mult(s0, F1);
+        load(F0, t + 2);
+        select(s1, F2);
+        interleave();
+        mult(s1, F2);
+        load(F1, t + 3);
+        select(s0, F0);
+        interleave();
+        mult(s0, F0);
+        load(F2, t + 4);
+        select(s1, F1);
+        interleave();
+#pragma unroll
+        for (int q = 0; q < Q; q++) s0[q] = s1[q];
     }
-    mult(F1);
+    mult(s0, F1);
 }
 
-// The same for n < 1,024: one tile, whose column 0 is b's block `shift`.
+// The same for n < 1,024: one tile, whose column 0 is b's block `shift`. Four steps' loads at a time,
+// ahead of the four before them.
 template <u32 NB>
 __device__ __forceinline__ v16i product1(const Lane& L, const unsigned char* A, const unsigned char* B, int shift) {
     const u32* pa = L.a(A);
-    const unsigned char* pb = L.b(B);
-    v16i acc, acc2;
+    const unsigned char* pb = L.b(B, Lay<NB>::plane) + 16 * shift;
+    v16i acc[2];
 #pragma unroll
-    for (u32 i = 0; i < 16; i++) acc[i] = acc2[i] = 0;
+    for (u32 i = 0; i < 16; i++) acc[0][i] = acc[1][i] = 0;
+    struct Frags { FragA a[4]; v4i b[4]; };
+    auto load = [&](Frags& F, u32 g) {
 #pragma unroll
-    for (u32 kappa = 0; kappa <= NB; kappa++) {
-        const v4i a = perm_a(load_a(pa, kappa), L.sel);
-        const v4i b = load_b(pb, shift - (int)kappa);
-        if (kappa & 1)
-            acc2 = mfma(a, b, acc2);
-        else
-            acc = mfma(a, b, acc);
+        for (u32 i = 0; i < 4; i++)
+            if (g + i <= NB) {
+                F.a[i] = load_a(pa, g + i);
+                F.b[i] = load_b(pb, -(int)(g + i));
+            }
+        fence();
+    };
+    Frags F[2];
+    load(F[0], 0);
+#pragma unroll
+    for (u32 g = 0; g <= NB; g += 4) {
+        if (g + 4 <= NB) load(F[g / 4 + 1 & 1], g + 4);
+#pragma unroll
+        for (u32 i = 0; i < 4; i++)
+            if (g + i <= NB) acc[i & 1] = mfma(perm_a(F[g / 4 & 1].a[i], L.sel), F[g / 4 & 1].b[i], acc[i & 1]);
+        fence();
     }
 #pragma unroll
-    for (u32 i = 0; i < 16; i++) acc[i] += acc2[i];
-    return acc;
+    for (u32 i = 0; i < 16; i++) acc[0][i] += acc[1][i];
+    return acc[0];
 }
 
 // Columns of a tile into limb sums: lane (j, h) holds rows 8 g + 4 h + (0 .. 3) of column j, the
-// four digits of limb 8 j + 2 g + h of the tile.
-__device__ __forceinline__ void stage(i64* st, u32 tile, const v16i& acc, const Lane& L, u32 cols) {
-    if (L.j < cols) {
+// four digits of limb 8 j + 2 g + h of the tile. Columns from `first`, `cols` of them.
+__device__ __forceinline__ void stage(i64* st, u32 tile, const v16i& acc, const Lane& L, u32 first, u32 cols) {
+    const u32 j = L.j - first;
+    i64 b8 = 1 << 8, b16 = 1 << 16, b24 = 1 << 24;
+    asm("" : "+s"(b8), "+s"(b16), "+s"(b24));  // products: three multiply-adds, not shifts and adds
+    if (j < cols) {
 #pragma unroll
-        for (u32 g = 0; g < 4; g++) {
-            const i64 v = (i64)acc[4 * g] + ((i64)acc[4 * g + 1] << 8) + ((i64)acc[4 * g + 2] << 16) + ((i64)acc[4 * g + 3] << 24);
-            st[288 * tile + 9 * L.j + 2 * g + L.h] = v;
-        }
+        for (u32 g = 0; g < 4; g++)
+            st[288 * tile + 9 * j + 2 * g + L.h] =
+                acc[4 * g] + (i64)acc[4 * g + 1] * (int)b8 + (i64)acc[4 * g + 2] * (int)b16 + (i64)acc[4 * g + 3] * (int)b24;
     }
 }
 template <u32 E> __device__ __forceinline__ u32 stage_pos(u32 lane, u32 i) {
@@ -211,44 +264,35 @@ template <u32 E> __device__ __forceinline__ u32 stage_pos(u32 lane, u32 i) {
 // Carries E limb sums per lane over ACT lanes (lane 0 lowest; the sums of other lanes are 0): limbs
 // in l, returns the carry out. Sums < 2^60.
 template <u32 E, u32 ACT> __device__ __forceinline__ u32 carry(const u64* v, u32* l, u32 lane) {
-    u64 c = 0;
+    u32 c = 0;
 #pragma unroll
     for (u32 i = 0; i < E; i++) {
-        const u64 s = v[i] + c;
-        l[i] = (u32)s;
-        c = s >> 32;
+        const bool o = __builtin_add_overflow((u32)v[i], c, &l[i]);
+        c = (u32)(v[i] >> 32) + o;
     }
-    const u32 C = (u32)c;
+    const u32 C = c;
     const u32 in = (u32)__builtin_amdgcn_update_dpp(0, (int)C, 0x138, 0xf, 0xf, false);  // wave_shr:1
-    u64 s = (u64)l[0] + in;
-    l[0] = (u32)s;
-    u32 c1 = (u32)(s >> 32);
-    bool ones = l[0] == 0xffffffffu;
+    bool c1 = __builtin_add_overflow(l[0], in, &l[0]);
+    u32 ones = l[0];
 #pragma unroll
     for (u32 i = 1; i < E; i++) {
-        s = (u64)l[i] + c1;
-        l[i] = (u32)s;
-        c1 = (u32)(s >> 32);
-        ones &= l[i] == 0xffffffffu;
+        c1 = __builtin_add_overflow(l[i], (u32)c1, &l[i]);
+        ones &= l[i];
     }
     constexpr u64 mask = ACT == 64 ? ~0ull : (1ull << ACT) - 1;
-    const u64 g = __ballot(c1 != 0) & mask, p = __ballot(ones) & mask;
+    const u64 g = __ballot(c1) & mask, p = __ballot(ones == 0xffffffffu) & mask;
     const u64 a = g | p, sum = a + g, cm = sum ^ a ^ g;  // bit i: a carry into lane i
     const u32 out = ACT == 64 ? (sum < a ? 1u : 0u) : (u32)(cm >> ACT) & 1;
     if (cm & mask) {
-        c1 = (u32)(cm >> lane) & 1;
+        c1 = (cm >> lane) & 1;
 #pragma unroll
-        for (u32 i = 0; i < E; i++) {
-            s = (u64)l[i] + c1;
-            l[i] = (u32)s;
-            c1 = (u32)(s >> 32);
-        }
+        for (u32 i = 0; i < E; i++) c1 = __builtin_add_overflow(l[i], (u32)c1, &l[i]);
     }
     return rdlane(C, ACT - 1) + out;
 }
 
-// Whether a number given as limbs + 0x80..80 is negative.
-template <u32 E, u32 ACT> __device__ __forceinline__ u32 negative(const u32* l, u32 lane) {
+// Sign of a number given as limbs + 0x80..80: 1 negative, 0 positive, 2 zero.
+template <u32 E, u32 ACT> __device__ __forceinline__ u32 sign_of(const u32* l, u32 lane) {
     const u32 top = rdlane(l[E - 1], ACT - 1);
     if (top != SGN) return top < SGN;
     bool gt = false, lt = false;
@@ -260,7 +304,7 @@ template <u32 E, u32 ACT> __device__ __forceinline__ u32 negative(const u32* l, 
     }
     constexpr u64 mask = ACT == 64 ? ~0ull : (1ull << ACT) - 1;
     const u64 g = __ballot(gt) & mask, t = __ballot(lt) & mask;
-    return t > g;
+    return g | t ? t > g : 2;
 }
 
 // Sum over the wave (in every lane's copy of the returned scalar).
@@ -278,132 +322,161 @@ __device__ __forceinline__ int wave_sum(int v) {
 template <u32 NB> struct Slot {
     typedef Lay<NB> Y;
     static constexpr u32 k = Y::k, Q = NB / 32;
-    static constexpr u32 ET = 2 * k >= 64 ? 2 * k / 64 : 1, AT = 2 * k / ET;  // limbs per lane and lanes of T
-    static constexpr u32 EK = k >= 64 ? k / 64 : 1, AK = k / EK;              // and of one residue
+    static constexpr u32 EK = k >= 64 ? k / 64 : 1, AK = k / EK;  // limbs per lane of a residue, and lanes
     const Lane L;
     unsigned char* const lds;
     u32 ex = 0, en = 0;  // x = x' + ex R, N = N'' + en R over the signed digits
 
     __device__ __forceinline__ Slot(u32 lane, unsigned char* base) : L(lane), lds(base) {}
 
-    __device__ __forceinline__ u32* words(u32 off) const { return (u32*)(lds + off); }
+    __device__ __forceinline__ u32* word(u32 off) const { return (u32*)(lds + off); }
     __device__ __forceinline__ i64* sums() const { return (i64*)(lds + Y::st); }
 
-    // A residue's limbs (k words at src) as signed digits at `area`; returns the flag.
-    __device__ __forceinline__ u32 digits_in(const u32* src, u32 area) {
-        u64 v[EK];
-        u32 l[EK];
-#pragma unroll
-        for (u32 i = 0; i < EK; i++) v[i] = L.id < AK ? (u64)src[EK * L.id + i] + SGN : 0;
-        const u32 e = carry<EK, AK>(v, l, L.id);
-        put(area, l);
-        return e;
-    }
-    // Biased limbs as signed digits at `area`.
-    __device__ __forceinline__ void put(u32 area, const u32* l) {
+    // Limb i of this lane's limbs as signed digits, biased limbs l: to the Toeplitz operand, or to the
+    // planes at `area`.
+    __device__ __forceinline__ void put(const u32* l) {
         if (L.id < AK)
 #pragma unroll
-            for (u32 i = 0; i < EK; i++) words(area)[EK * L.id + i] = l[i] ^ SGN;
+            for (u32 i = 0; i < EK; i++) word(Y::op)[EK * L.id + i] = l[i] ^ SGN;
     }
-    // The signed value of limb q of the digits at `area`.
-    __device__ __forceinline__ i64 limb_at(u32 area, u32 q) const { return (i64)(words(area)[q] ^ SGN) - (i64)SGN; }
+    __device__ __forceinline__ void put_planes(u32 area, const u32* l) {
+        if (L.id < AK)
+#pragma unroll
+            for (u32 i = 0; i < EK; i++) *word(Y::at(area, EK * L.id + i)) = l[i] ^ SGN;
+    }
+    // The signed value of four digits.
+    static __device__ __forceinline__ i64 value(u32 digits) { return (i64)(digits ^ SGN) - (i64)SGN; }
 
+    // A residue's limbs (k words at src), biased; returns the flag.
+    __device__ __forceinline__ u32 digits_in(const u32* src, u32* l) {
+        u64 v[EK];
+#pragma unroll
+        for (u32 i = 0; i < EK; i++) v[i] = L.id < AK ? (u64)src[EK * L.id + i] + SGN : 0;
+        return carry<EK, AK>(v, l, L.id);
+    }
     __device__ void init(const u32* x, const u32* np, const u32* n) {
         for (u32 o = 16 * L.id; o < Y::st; o += 1024) *(v4i*)(lds + o) = v4i{0, 0, 0, 0};
         wsync();
-        digits_in(np, Y::np);
-        en = digits_in(n, Y::nn);
-        ex = digits_in(x, Y::op);
+        u32 l[EK];
+        digits_in(np, l);
+        put_planes(Y::np, l);
+        en = digits_in(n, l);
+        put_planes(Y::nn, l);
+        ex = digits_in(x, l);
+        put(l);
+        put_planes(Y::xb, l);
         wsync();
     }
-
+    // Biased limbs to the number itself (in: 1, or the carry of the limbs below).
+    __device__ __forceinline__ u32 unbias(u32* l, u32 in) {
+        u64 v[EK];
+#pragma unroll
+        for (u32 i = 0; i < EK; i++) v[i] = L.id < AK ? (u64)l[i] + (0xffffffffu - SGN) + (EK * L.id + i == 0 ? in : 0) : 0;
+        return carry<EK, AK>(v, l, L.id);
+    }
+    __device__ __forceinline__ void out(u32* dst, const u32* l) {
+        if (L.id < AK)
+#pragma unroll
+            for (u32 i = 0; i < EK; i++) dst[EK * L.id + i] = l[i];
+    }
     // x's limbs, from its digits.
     __device__ void store_x(u32* x) {
-        u64 v[EK];
         u32 l[EK];
         wsync();
 #pragma unroll
-        for (u32 i = 0; i < EK; i++)
-            v[i] = L.id < AK ? (u64)(words(Y::op)[EK * L.id + i] ^ SGN) + (0xffffffffu - SGN) + (EK * L.id + i == 0) : 0;
-        carry<EK, AK>(v, l, L.id);
-        if (L.id < AK)
-#pragma unroll
-            for (u32 i = 0; i < EK; i++) x[EK * L.id + i] = l[i];
+        for (u32 i = 0; i < EK; i++) l[i] = L.id < AK ? word(Y::op)[EK * L.id + i] ^ SGN : 0;
+        unbias(l, 1);
+        out(x, l);
     }
 
-    // T = c x^2 as biased limbs, ET per lane; returns what stands above them (in units of R^2).
-    __device__ __forceinline__ u32 square(u32 c, u32* l) {
-        const unsigned char* X = lds + Y::op;
+    // The staged limb sum i of this lane (0 past the last lane).
+    __device__ __forceinline__ i64 staged(u32 i) const { return L.id < AK ? sums()[stage_pos<EK>(L.id, i)] : 0; }
+    // c times the staged sums, biased, through the carry; `in` joins limb 0.
+    __device__ __forceinline__ u32 carry_staged(u32 c, u64 in, u32* l) {
+        u64 v[EK];
+#pragma unroll
+        for (u32 i = 0; i < EK; i++) {
+            i64 s = staged(i);
+            if (c != 1) s *= (i64)c;
+            v[i] = L.id < AK ? (u64)s + BIAS + SGN + (EK * L.id + i == 0 ? in : 0) : 0;
+        }
+        return carry<EK, AK>(v, l, L.id);
+    }
+
+    // T = c x^2 as biased limbs, low and high half; returns what stands above them (in units of
+    // R^2). The halves are carried one after the other, so that the sums of one half are staged.
+    __device__ __forceinline__ u32 square(u32 c, u32* lo, u32* hi) {
+        const unsigned char *X = lds + Y::op, *XB = lds + Y::xb;
+        u32 mid;
         if constexpr (NB >= 32) {
             v16i acc[2 * Q];
-            product<NB, 0, 2 * Q>(L, X, X, acc);
+            product<NB, 0, 2 * Q>(L, X, XB, acc);
 #pragma unroll
-            for (u32 t = 0; t < 2 * Q; t++) stage(sums(), t, acc[t], L, 32);
+            for (u32 t = 0; t < Q; t++) stage(sums(), t, acc[t], L, 0, 32);
+            wsync();
+            mid = carry_staged(c, BETA, lo);
+            wsync();
+#pragma unroll
+            for (u32 t = 0; t < Q; t++) stage(sums(), t, acc[Q + t], L, 0, 32);
         } else {
-            stage(sums(), 0, product1<NB>(L, X, X, 0), L, 2 * NB);
+            const v16i acc = product1<NB>(L, X, XB, 0);
+            stage(sums(), 0, acc, L, 0, NB);
+            wsync();
+            mid = carry_staged(c, BETA, lo);
+            wsync();
+            stage(sums(), 0, acc, L, NB, NB);
         }
         wsync();
-        u64 v[ET];
-#pragma unroll
-        for (u32 i = 0; i < ET; i++) {
-            i64 s = L.id < AT ? sums()[stage_pos<ET>(L.id, i)] : 0;
-            if (c != 1) s *= (i64)c;
-            v[i] = L.id < AT ? (u64)s + BIAS + SGN + (ET * L.id + i == 0 ? BETA : 0) : 0;
-        }
-        u32 e = 0;
+        u32 top;
         if (ex) {  // + c (2 x' R + R^2)
+            u64 v[EK];
 #pragma unroll
-            for (u32 i = 0; i < ET; i++) {
-                const u32 q = ET * L.id + i;
-                if (L.id < AT && q >= k) v[i] += (u64)(2 * (i64)c * limb_at(Y::op, q - k));
+            for (u32 i = 0; i < EK; i++) {
+                const u32 q = EK * L.id + i;
+                v[i] = L.id < AK ? (u64)((i64)c * (staged(i) + 2 * value(word(Y::op)[q]))) + BIAS + SGN + (q == 0 ? mid : 0) : 0;
             }
-            e = c;
+            top = carry<EK, AK>(v, hi, L.id) + c;
+        } else {
+            top = carry_staged(c, mid, hi);  // mid holds the low half's BETA
         }
-        e += carry<ET, AT>(v, l, L.id) - (u32)BETA;
-        return e;
+        wsync();
+        return top - (u32)BETA;
+    }
+    // The part of a nonzero square() that stands for a number: 1 for T' < 0 (T = T' + R^2), else 0.
+    __device__ __forceinline__ u32 borrowed(const u32* lo, const u32* hi) const {
+        const u32 s = sign_of<EK, AK>(hi, L.id);
+        return (s == 2 ? sign_of<EK, AK>(lo, L.id) : s) & 1;
     }
 
     // One step; returns nonzero on a carry that must vanish but does not.
     __device__ __forceinline__ u32 step(u32 c) {
-        u32 bad = 0, lt[ET];
-        u32 et = square(c, lt);
-        if (et) {  // T = T' + et R^2: only T' < 0, et = 1 stands for a number below R^2
-            const u32 neg = negative<ET, AT>(lt, L.id);
+        u32 bad = 0;
+        u32 l[EK], hi[EK];
+        u32 et = square(c, l, hi);
+        if (et) {
+            const u32 neg = borrowed(l, hi);
             bad |= et != neg;
             et = neg;
         }
         // T's top limb below R, for q.
-        const i64 tlow = (i64)rdlane(lt[ET - 1], AT / 2 - 1) - (i64)SGN;
-        wsync();
-        if (L.id < AT / 2) {
-#pragma unroll
-            for (u32 i = 0; i < ET; i++) words(Y::op)[ET * L.id + i] = lt[i] ^ SGN;
-        } else if (L.id < AT) {
-#pragma unroll
-            for (u32 i = 0; i < ET; i++) words(Y::th)[ET * L.id + i - k] = lt[i];
-        }
+        const i64 tlow = (i64)rdlane(l[EK - 1], AK - 1) - (i64)SGN;
+        put(l);
         wsync();
         // m = (T mod R) N' mod R.
-        u64 v[EK];
-        u32 l[EK];
         low_product();
         wsync();
-#pragma unroll
-        for (u32 i = 0; i < EK; i++)
-            v[i] = L.id < AK ? (u64)sums()[stage_pos<EK>(L.id, i)] + BIAS + SGN + (EK * L.id + i == 0 ? BETA : 0) : 0;
-        carry<EK, AK>(v, l, L.id);
-        const u32 em = negative<EK, AK>(l, L.id);
-        put(Y::op, l);
+        carry_staged(1, BETA, l);
+        const u32 em = sign_of<EK, AK>(l, L.id) & 1;
+        put(l);
         wsync();
         // The last four low columns of m N, and with T's digits there q = (L + T mod R) / R.
         int g0 = 0, g1 = 0, g2 = 0, g3 = 0;
-        const u32 *mw = words(Y::op), *nw = words(Y::nn);
 #pragma unroll
         for (u32 r = 0; r < (k + 63) / 64; r++) {
             const u32 w = 64 * r + L.id;
-            const int md = w < k ? (int)mw[w] : 0;
-            const u32 W = w < k ? k - 1 - w : 0;
-            const u32 hi = nw[W], lo = nw[(int)W - 1];
+            const int md = w < k ? (int)word(Y::op)[w] : 0;
+            const int W = w < k ? (int)(k - 1 - w) : 0;
+            const u32 hi = *word(Y::at(Y::nn, W)), lo = *word(Y::at(Y::nn, W - 1));
             g0 = __builtin_amdgcn_sdot4(md, (int)__builtin_amdgcn_perm(hi, lo, 0x01020304u), g0, false);
             g1 = __builtin_amdgcn_sdot4(md, (int)__builtin_amdgcn_perm(hi, lo, 0x02030405u), g1, false);
             g2 = __builtin_amdgcn_sdot4(md, (int)__builtin_amdgcn_perm(hi, lo, 0x03040506u), g2, false);
@@ -414,26 +487,28 @@ template <u32 NB> struct Slot {
         // x = floor(T / R) + the high columns of m N + q + e_m N + e_N m.
         high_product();
         wsync();
+        u64 v[EK];
 #pragma unroll
         for (u32 i = 0; i < EK; i++) {
             const u32 j = EK * L.id + i;
-            v[i] = L.id < AK ? (u64)sums()[stage_pos<EK>(L.id, i)] + BIAS + words(Y::th)[j] + (j == 0 ? (u64)((i64)BETA + q) : 0) : 0;
-            if (em && L.id < AK) v[i] += (u64)limb_at(Y::nn, j);
+            v[i] = L.id < AK ? (u64)staged(i) + BIAS + hi[i] + (j == 0 ? (u64)((i64)BETA + q) : 0) : 0;
+            if (em && L.id < AK) v[i] += (u64)value(*word(Y::at(Y::nn, j)));
         }
         u32 f = et + (em & en);
         if (en) {
 #pragma unroll
             for (u32 i = 0; i < EK; i++)
-                if (L.id < AK) v[i] += (u64)limb_at(Y::op, EK * L.id + i);
+                if (L.id < AK) v[i] += (u64)value(word(Y::op)[EK * L.id + i]);
         }
         f += carry<EK, AK>(v, l, L.id) - (u32)BETA;
         ex = 0;
         if (f) {
-            ex = negative<EK, AK>(l, L.id);
+            ex = sign_of<EK, AK>(l, L.id) & 1;
             bad |= f != ex;
         }
         wsync();
-        put(Y::op, l);
+        put(l);
+        put_planes(Y::xb, l);
         wsync();
         return bad;
     }
@@ -443,9 +518,9 @@ template <u32 NB> struct Slot {
             v16i acc[Q];
             product<NB, 0, Q>(L, lds + Y::op, lds + Y::np, acc);
 #pragma unroll
-            for (u32 t = 0; t < Q; t++) stage(sums(), t, acc[t], L, 32);
+            for (u32 t = 0; t < Q; t++) stage(sums(), t, acc[t], L, 0, 32);
         } else {
-            stage(sums(), 0, product1<NB>(L, lds + Y::op, lds + Y::np, 0), L, NB);
+            stage(sums(), 0, product1<NB>(L, lds + Y::op, lds + Y::np, 0), L, 0, NB);
         }
     }
     __device__ __forceinline__ void high_product() {
@@ -453,9 +528,9 @@ template <u32 NB> struct Slot {
             v16i acc[Q];
             product<NB, Q, 2 * Q>(L, lds + Y::op, lds + Y::nn, acc);
 #pragma unroll
-            for (u32 t = 0; t < Q; t++) stage(sums(), t, acc[t], L, 32);
+            for (u32 t = 0; t < Q; t++) stage(sums(), t, acc[t], L, 0, 32);
         } else {
-            stage(sums(), 0, product1<NB>(L, lds + Y::op, lds + Y::nn, (int)NB), L, NB);
+            stage(sums(), 0, product1<NB>(L, lds + Y::op, lds + Y::nn, (int)NB), L, 0, NB);
         }
     }
 };
@@ -475,19 +550,14 @@ __device__ __forceinline__ void steps(const Args& A, u32 slot, u32 bits, u32 lan
     for (u32 it = 0; it < bits && pos < nb; it++, pos++) {
         const u32 c = (ex[pos >> 5] >> (31 - (pos & 31))) & 1 ? A.base : 1;
         if constexpr (BARE) {
-            u32 l[S::ET];
-            const u32 e = s.square(c, l);
-            bad |= e != 0 && e != negative<S::ET, S::AT>(l, lane);
+            u32 lo[S::EK], hi[S::EK];
+            const u32 e = s.square(c, lo, hi);
+            bad |= e != 0 && e != s.borrowed(lo, hi);
             if (A.lim) {
-                u64 v[S::ET];
-#pragma unroll
-                for (u32 i = 0; i < S::ET; i++) v[i] = lane < S::AT ? (u64)l[i] + (0xffffffffu - SGN) + (S::ET * lane + i == 0) : 0;
-                carry<S::ET, S::AT>(v, l, lane);
-                if (lane < S::AT)
-#pragma unroll
-                    for (u32 i = 0; i < S::ET; i++) A.lim[(size_t)slot * 3 * k + S::ET * lane + i] = l[i];
+                s.unbias(hi, s.unbias(lo, 1));
+                s.out(A.lim + (size_t)slot * 3 * k, lo);
+                s.out(A.lim + (size_t)slot * 3 * k + k, hi);
             }
-            wsync();
         } else {
             bad |= s.step(c);
         }
