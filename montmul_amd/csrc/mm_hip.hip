@@ -507,6 +507,10 @@ struct Ctx {
     size_t max_dyn_lds = 0;     // dynamic LDS every step kernel can take
     size_t max_dyn_lds_v2 = 0;  // the same for the register-transform kernels
     size_t max_dyn_lds_mix[2] = {0, 0};  // the mixed-length kernel, 512 and 1,024 threads
+    // Further streams of a mixed run (default priority), made on the first one, and the events that
+    // fork them from `stream` and join them to it.
+    hipStream_t side[3] = {nullptr, nullptr, nullptr};
+    hipEvent_t fork = nullptr, join[3] = {nullptr, nullptr, nullptr};
     // Mixed-length launches: head counter, length classes and work items in one device
     // buffer (grown on demand), and the latest launch's milliseconds per step.
     unsigned char* mix_buf = nullptr;
@@ -999,6 +1003,11 @@ template <class Launch> int run_chunks(Ctx* C, uint64_t reps, Launch&& launch, f
     return 0;
 }
 
+// Up to `s` steps of one batch by the kernel that steps it alone (matrix-core or double-precision).
+hipError_t launch_direct(State* S, uint32_t s, bool bare, hipStream_t sm) {
+    return S->mx ? mx::launch(S->mx_args(bare), S->k, S->slots, s, bare, sm) : fd::launch(S->fd_args(), S->k, S->slots, s, bare, sm);
+}
+
 // Runs up to `bits` steps on every slot with bits left (reference: Gpu::steps, gpu/mod.rs:113-158).
 int64_t steps(State* S, uint64_t bits, bool bare) {
     Ctx* C = S->C;
@@ -1037,8 +1046,7 @@ int64_t steps(State* S, uint64_t bits, bool bare) {
         float ms = 0;
         if (run_chunks(C, reps,
                        [&]() {
-                           if (S->mx) return mx::launch(S->mx_args(bare), S->k, S->slots, (uint32_t)s, bare, C->stream);
-                           if (S->fd) return fd::launch(S->fd_args(), S->k, S->slots, (uint32_t)s, bare, C->stream);
+                           if (S->mx || S->fd) return launch_direct(S, (uint32_t)s, bare, C->stream);
                            if (kern2)
                                hipLaunchKernelGGL(kern2, dim3(S->slots), dim3(S->threads), S->lds, C->stream, A2, 0u, (uint32_t)s);
                            else
@@ -1257,9 +1265,22 @@ int mix_class(State* S, uint32_t nt, MixClass* out, uint64_t* lds, uint32_t* gro
     return 0;
 }
 
-// Up to `bits` steps on every slot with bits left in every batch of the group, in launches of
-// the mixed-length kernel. Returns MM_OK, the first slot whose carry-out check failed (its
-// batch's index in *which), or MM_EFAULT.
+// The context's further streams and their events, on first use.
+int side_streams(Ctx* C) {
+    if (C->join[2]) return 0;
+    if (!C->fork) HIPCHK(hipEventCreateWithFlags(&C->fork, hipEventDisableTiming));
+    for (int i = 0; i < 3; i++) {
+        if (!C->side[i]) HIPCHK(hipStreamCreateWithFlags(&C->side[i], hipStreamNonBlocking));
+        if (!C->join[i]) HIPCHK(hipEventCreateWithFlags(&C->join[i], hipEventDisableTiming));
+    }
+    return 0;
+}
+
+// Up to `bits` steps on every slot with bits left in every batch of the group. The batches that the
+// matrix-core or the double-precision step runs keep their own kernels, side by side on up to four
+// streams: each takes the share of the CUs that its slots fill, and the run lasts as long as the
+// longest stream. The others share launches of the mixed-length kernel, on the context's stream. Returns
+// MM_OK, the first slot whose carry-out check failed (its batch's index in *which), or MM_EFAULT.
 int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which) {
     if (count == 0) return MM_OK;
     Ctx* C = G[0]->C;
@@ -1268,10 +1289,12 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
     if (hipSetDevice(C->device) != hipSuccess) { fail("hipSetDevice failed"); return MM_EFAULT; }
     uint64_t most = 0;
     uint32_t nt = 512;
+    std::vector<size_t> queued, direct;  // through the mixed-length kernel, by their own kernels
     for (size_t g = 0; g < count; g++) {
         const State* S = G[g];
+        (S->mx || S->fd ? direct : queued).push_back(g);
         for (uint32_t i = 0; i < S->slots; i++) most = std::max<uint64_t>(most, S->nbits[i] - S->pos[i]);
-        if (S->v2 && S->n <= 8192 && S->n / 8 > nt) nt = S->n / 8;
+        if (!S->mx && !S->fd && S->v2 && S->n <= 8192 && S->n / 8 > nt) nt = S->n / 8;
         G[g]->last_ms = 0;
         G[g]->last_launches = 0;
         G[g]->failed.clear();
@@ -1281,11 +1304,14 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
     std::vector<MixClass> cls(count);
     std::vector<uint32_t> groups(count, 1);
     uint64_t lds = 0;
-    for (size_t g = 0; g < count; g++) {
+    for (size_t g = 0; g < count; g++)
+        if (push(G[g])) return MM_EFAULT;
+    for (size_t g : queued) {
         uint64_t l = 0;
-        if (push(G[g]) || mix_class(G[g], nt, &cls[g], &l, &groups[g])) return MM_EFAULT;
+        if (mix_class(G[g], nt, &cls[g], &l, &groups[g])) return MM_EFAULT;
         lds = std::max(lds, l);
     }
+    if (direct.size() + !queued.empty() > 1 && side_streams(C)) return MM_EFAULT;
     const size_t lim = C->max_dyn_lds_mix[nt == 1024];
     if (lds > lim) {
         fail("mixed launch needs " + std::to_string(lds) + " bytes of LDS, " + std::to_string(lim) + " available");
@@ -1309,7 +1335,7 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
         items.clear();
         list.clear();
         cost.clear();
-        for (size_t g = 0; g < count; g++) {
+        for (size_t g : queued) {
             const State* S = G[g];
             const double per_step = (double)S->n * ilog2(S->n) * (S->v2 ? 1.0 : 3.0);
             std::vector<std::pair<uint64_t, uint32_t>> todo;  // (steps, slot)
@@ -1325,6 +1351,25 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
                 cost.push_back((double)todo[a].first * per_step);
             }
         }
+        // The direct batches' streams (0: the context's), the longest first and each to the least
+        // loaded: a step takes about as long as the modulus is long, times the rounds of slots.
+        std::vector<std::pair<double, size_t>> by_time;
+        for (size_t g : direct) {
+            const State* S = G[g];
+            uint64_t r = 0;
+            for (uint32_t i = 0; i < S->slots; i++) r = std::max<uint64_t>(r, S->nbits[i] - S->pos[i]);
+            const double per_cu = S->mx ? std::min(32.0, 4096.0 / S->k) : std::max(1.0, 8192.0 / S->k);
+            by_time.push_back({(double)std::min<uint64_t>(r, s) * S->k * std::max(1.0, S->slots / (per_cu * C->cus)), g});
+        }
+        std::stable_sort(by_time.begin(), by_time.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
+        std::vector<size_t> lane[4];
+        double load[4] = {0, 0, 0, 0};
+        for (double c : cost) load[0] += c / C->cus / 8;  // the mixed-length kernel's share
+        for (const auto& bt : by_time) {
+            const size_t l = std::min_element(load, load + 4) - load;
+            lane[l].push_back(bt.second);
+            load[l] += bt.first;
+        }
         std::vector<uint32_t> order(items.size());
         for (uint32_t i = 0; i < order.size(); i++) order[i] = i;
         std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return cost[a] > cost[b]; });
@@ -1333,7 +1378,7 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
         const size_t cls_off = 256, items_off = cls_off + ((count * sizeof(MixClass) + 255) & ~(size_t)255);
         const size_t list_off = items_off + ((queue.size() * sizeof(MixItem) + 255) & ~(size_t)255);
         const size_t need = list_off + list.size() * sizeof(uint32_t);
-        if (need > C->mix_cap) {
+        if (!queue.empty() && need > C->mix_cap) {
             if (hipStreamSynchronize(sm) != hipSuccess) { fail("stream synchronize failed"); return MM_EFAULT; }
             if (C->mix_buf) hipFree(C->mix_buf);
             C->mix_buf = nullptr;
@@ -1345,10 +1390,10 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
         const MixClass* dcls = (const MixClass*)(C->mix_buf + cls_off);
         const MixItem* ditems = (const MixItem*)(C->mix_buf + items_off);
         const uint32_t* dlist = (const uint32_t*)(C->mix_buf + list_off);
-        hipError_t ce = hipMemcpyAsync(C->mix_buf + cls_off, cls.data(), count * sizeof(MixClass), hipMemcpyHostToDevice, sm);
-        if (ce == hipSuccess)
+        hipError_t ce = queue.empty() ? hipSuccess : hipMemcpyAsync(C->mix_buf + cls_off, cls.data(), count * sizeof(MixClass), hipMemcpyHostToDevice, sm);
+        if (ce == hipSuccess && !queue.empty())
             ce = hipMemcpyAsync(C->mix_buf + items_off, queue.data(), queue.size() * sizeof(MixItem), hipMemcpyHostToDevice, sm);
-        if (ce == hipSuccess)
+        if (ce == hipSuccess && !queue.empty())
             ce = hipMemcpyAsync(C->mix_buf + list_off, list.data(), list.size() * sizeof(uint32_t), hipMemcpyHostToDevice, sm);
         if (ce != hipSuccess) { hip_fail("mixed launch upload", ce); return MM_EFAULT; }
         // The upload must land before a replayed graph reads it.
@@ -1360,11 +1405,28 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
         float ms = 0;
         if (run_chunks(C, reps,
                        [&]() {
-                           hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, sm, head, 1u, 0u);
-                           hipError_t fe = hipGetLastError();
-                           if (fe != hipSuccess) return fe;
-                           return nt == 1024 ? mix_launch<1024>(grid, lds, sm, dcls, ditems, dlist, (uint32_t)queue.size(), head)
-                                             : mix_launch<512>(grid, lds, sm, dcls, ditems, dlist, (uint32_t)queue.size(), head);
+                           hipError_t fe = hipSuccess;
+                           for (int l = 1; l < 4 && fe == hipSuccess; l++) {  // fork
+                               if (lane[l].empty()) continue;
+                               if ((fe = hipEventRecord(C->fork, sm)) != hipSuccess) break;
+                               fe = hipStreamWaitEvent(C->side[l - 1], C->fork, 0);
+                           }
+                           for (int l = 3; l >= 0 && fe == hipSuccess; l--)
+                               for (size_t i = 0; i < lane[l].size() && fe == hipSuccess; i++)
+                                   fe = launch_direct(G[lane[l][i]], (uint32_t)s, false, l ? C->side[l - 1] : sm);
+                           if (fe == hipSuccess && !queue.empty()) {
+                               hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, sm, head, 1u, 0u);
+                               if ((fe = hipGetLastError()) == hipSuccess)
+                                   fe = nt == 1024 ? mix_launch<1024>(grid, lds, sm, dcls, ditems, dlist, (uint32_t)queue.size(), head)
+                                                   : mix_launch<512>(grid, lds, sm, dcls, ditems, dlist, (uint32_t)queue.size(), head);
+                           }
+                           for (int l = 1; l < 4; l++) {  // join, also after an error: nothing runs on
+                               if (lane[l].empty()) continue;
+                               hipError_t je = hipEventRecord(C->join[l - 1], C->side[l - 1]);
+                               if (je == hipSuccess) je = hipStreamWaitEvent(sm, C->join[l - 1], 0);
+                               if (fe == hipSuccess) fe = je;
+                           }
+                           return fe;
                        },
                        &ms))
             return MM_EFAULT;
@@ -1461,6 +1523,10 @@ void mm_hip_close(mm_backend* be) {
     C->tabs.clear();
     C->fd_tabs.clear();
     if (C->mix_buf) hipFree(C->mix_buf);
+    for (hipStream_t sd : C->side)
+        if (sd) hipStreamDestroy(sd);
+    for (hipEvent_t e : {C->fork, C->join[0], C->join[1], C->join[2]})
+        if (e) hipEventDestroy(e);
     if (C->ev0) hipEventDestroy(C->ev0);
     if (C->ev1) hipEventDestroy(C->ev1);
     if (C->stream) hipStreamDestroy(C->stream);
