@@ -29,8 +29,8 @@
 // the later passes' twiddles, which stay in LDS.
 //
 // Measured against the modular transforms (mm_v2.h) that it replaces by default: L = 4,096 (1,024
-// slots) 7.0 -> 15.7 M squarings/s, 8,192 (4,096 slots) 3.6 -> 9.1 M, 16,384 (256 slots) 1.2 -> 1.84 M; one
-// slot alone at 8,192 92 -> 34 us a step.
+// slots) 7.0 -> 15.7 M squarings/s, 8,192 (4,096 slots) 3.6 -> 9.1 M, 16,384 (1,024 slots) 1.31 -> 3.7 M;
+// one slot alone at 8,192 92 -> 34 us a step.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -210,6 +210,8 @@ template <u32 R, bool INV> __device__ __forceinline__ void across(Z* v, u32 t) {
     }
     if constexpr (R == 4) {
         const double s2 = t & 2 ? -1.0 : 1.0;
+        // Selected by component: a choice between two Z went through scratch memory (1.84 M squarings/s
+        // at L = 16,384 and 256 slots against 3.5 M).
         const bool l3 = (t & 3) == 3;
 #pragma unroll
         for (u32 e = 0; e < 16; e++) {
@@ -217,12 +219,12 @@ template <u32 R, bool INV> __device__ __forceinline__ void across(Z* v, u32 t) {
             if constexpr (!INV) {
                 a = Z{__builtin_fma(s2, a.r, dpp<0x4E>(a.r)), __builtin_fma(s2, a.i, dpp<0x4E>(a.i))};
                 const Z b = rot<false>(a);
-                a = l3 ? b : a;
+                a = Z{l3 ? b.r : a.r, l3 ? b.i : a.i};
                 a = Z{__builtin_fma(s1, a.r, dpp<0xB1>(a.r)), __builtin_fma(s1, a.i, dpp<0xB1>(a.i))};
             } else {
                 a = Z{__builtin_fma(s1, a.r, dpp<0xB1>(a.r)), __builtin_fma(s1, a.i, dpp<0xB1>(a.i))};
                 const Z b = rot<true>(a);
-                a = l3 ? b : a;
+                a = Z{l3 ? b.r : a.r, l3 ? b.i : a.i};
                 a = Z{__builtin_fma(s2, a.r, dpp<0x4E>(a.r)), __builtin_fma(s2, a.i, dpp<0x4E>(a.i))};
             }
             v[e] = a;
