@@ -1,5 +1,5 @@
 // mm_fd.h - the Montgomery step on double-precision transforms (wraparound path, L = 4,096 ..
-// 16,384, k = L / 2 limbs).
+// 32,768, k = L / 2 limbs).
 //
 // A residue is C = L signed digits of 16 bits (-2^15 .. 2^15), in double precision, which issues one
 // multiply-add a cycle per lane where a product in GF(M61^2) takes sixteen 64-bit multiply-adds
@@ -12,7 +12,8 @@
 // 3.3 u (tables within u / 2), the last radix-2 or 4 stage 2 u: 49 u a transform. The two transforms
 // of a product, its pointwise step and the inverse make at most 150 u, and a coefficient of a b is
 // off by at most |a| |b| 150 u <= C 2^30 150 2^-53: 0.07, 0.15 and 0.29 at L = 4,096, 8,192 and
-// 16,384, below the 0.5 that rounding needs, for any digits. (Random digits err by 1e-4 or less.)
+// 16,384, below the 0.5 that rounding needs, for any digits (SplitSlot counts L = 32,768). (Random
+// digits err by 1e-4 or less.)
 //
 // A step, R = 2^(32k) = 2^(16 C):
 //     T = c x^2                  transform of length C, square, inverse
@@ -29,8 +30,8 @@
 // the later passes' twiddles, which stay in LDS.
 //
 // Measured against the modular transforms (mm_v2.h) that it replaces by default: L = 4,096 (1,024
-// slots) 7.0 -> 15.7 M squarings/s, 8,192 (4,096 slots) 3.6 -> 9.1 M, 16,384 (1,024 slots) 1.31 -> 3.7 M;
-// one slot alone at 8,192 92 -> 34 us a step.
+// slots) 7.0 -> 15.7 M squarings/s, 8,192 (4,096 slots) 3.6 -> 9.1 M, 16,384 (1,024 slots) 1.31 -> 3.7 M,
+// 32,768 (1,024 slots) 0.42 -> 1.18 M; one slot alone at 8,192 92 -> 34 us a step, at 32,768 560 -> 147 us.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -42,6 +43,7 @@ namespace fd {
 typedef uint32_t u32;
 typedef uint64_t u64;
 typedef int64_t i64;
+typedef uint16_t u16;
 
 constexpr u32 SGN = 0x80008000u;
 constexpr u64 BETA = 0x7fffffffu;  // |limb sums| < BETA (2^32 - 1): c C <= 2^16
@@ -56,13 +58,18 @@ struct Tables {
                         // exp(2 pi i t b / C) at (3 + b) T + t, b = 1 .. 3: element 4 a + b takes both
     const double2* t1;  // pass 1: exp(2 pi i j m / (C/16)) at m C/256 + j
     const double2* t2;  // pass 2: exp(2 pi i j m / (C/256)) at m C/4096 + j
+    // The split length 2C (see SplitSlot): t0's first four rows with the parts' weights, four rows for
+    // each part p, exp(2 pi i t (32 a + 4 p + 1) / 8C), then exp(2 pi i (4 p + 1) e / 128) at 16 p + e.
+    const double2* ts;
 };
 
 struct Args {
-    Tables w;           // length C = 2k
+    Tables w;           // length C = 2k (k = 16,384: C = k, the parts' length)
     u32* x;             // k limbs per slot
-    const double2* np;  // C per slot: spectrum of N', at e C/16 + t
-    const double2* n;   // C / 2 per slot: spectrum of N (length C / 2)
+    const double2* np;  // 2k per slot: spectrum of N', at e C/16 + t (k = 16,384: part after part)
+    const double2* n;   // k per slot: spectrum of N (length k)
+    double2* part;      // k = 16,384: k per slot, the first part's result
+    u32* dig;           // k = 16,384: k per slot, the digits that the second part loads again
     const u32* exp;     // ew words per slot, most significant bit first
     const u32* nbits;
     u32* pos;
@@ -244,11 +251,12 @@ __device__ __forceinline__ d2 ldg(u64 base, u32 off) {
 // of the butterfly, where sixteen have to be waited for in four groups.
 template <bool INV, u32 T, u32 SUB> struct Twiddle0 {
     d2 w[7];
-    __device__ __forceinline__ Twiddle0(const double2* t0, u32 t) {
-        u64 base = (u64)t0;
-        asm volatile("" : "+s"(base));  // or each step's row addresses stay in scalar registers
+    // t0: all rows; weighted: the first four, another length's weights in them or not.
+    __device__ __forceinline__ Twiddle0(const double2* t0, const double2* weighted, u32 t) {
+        u64 a = (u64)weighted, b = (u64)t0;
+        asm volatile("" : "+s"(a), "+s"(b));  // or each step's row addresses stay in scalar registers
 #pragma unroll
-        for (u32 r = 0; r < 7; r++) w[r] = ldg(base + 16 * SUB * T * r, 16 * SUB * t);
+        for (u32 r = 0; r < 7; r++) w[r] = ldg((r < 4 ? a : b) + 16 * SUB * T * r, 16 * SUB * t);
         fence();
     }
     __device__ __forceinline__ void apply(Z* v) const {
@@ -361,14 +369,15 @@ template <u32 LOGC, bool INV> __device__ __forceinline__ void last16(Z* v) {
 // Forward transform of weighted elements in pass-0 layout (the thread's own weights exp(i pi e / 32)
 // already applied); the spectrum ends in pass-2 layout. LOGF: the tables' length. The buffer must be
 // free (barrier before).
-template <u32 LOGF, u32 LOGC> __device__ __forceinline__ void forward(Z* v, const Tables& W, unsigned char* lds, bool on) {
+template <u32 LOGF, u32 LOGC>
+__device__ __forceinline__ void forward(Z* v, const Tables& W, unsigned char* lds, bool on, const double2* weighted) {
     typedef Geo<LOGC> G;
     typedef Geo<LOGF> F;
     typedef Pos<LOGC> P;
     constexpr u32 SUB = 1u << (LOGF - LOGC);
     double* X = (double*)lds;
     if (on) {
-        const Twiddle0<false, G::T, SUB> f(W.t0, tid());
+        const Twiddle0<false, G::T, SUB> f(W.t0, weighted, tid());
         dft16<false>(v);
         settle(v);
         f.apply(v);
@@ -398,7 +407,8 @@ template <u32 LOGF, u32 LOGC> __device__ __forceinline__ void forward(Z* v, cons
     }
 }
 // Its inverse up to the thread's own weights and the factor C: pass-2 layout in, pass-0 out.
-template <u32 LOGF, u32 LOGC> __device__ __forceinline__ void inverse(Z* v, const Tables& W, unsigned char* lds, bool on) {
+template <u32 LOGF, u32 LOGC>
+__device__ __forceinline__ void inverse(Z* v, const Tables& W, unsigned char* lds, bool on, const double2* weighted) {
     typedef Geo<LOGC> G;
     typedef Geo<LOGF> F;
     typedef Pos<LOGC> P;
@@ -424,7 +434,7 @@ template <u32 LOGF, u32 LOGC> __device__ __forceinline__ void inverse(Z* v, cons
         settle(v);
     }
     wsync();
-    const Twiddle0<true, G::T, SUB> f(W.t0, on ? tid() : 0);
+    const Twiddle0<true, G::T, SUB> f(W.t0, weighted, on ? tid() : 0);
     {
         const P p(tid());
         exchange<true, P::X1, P::X0>(v, X, p.x1, p.x0, on);
@@ -579,9 +589,9 @@ template <u32 LOGC> struct Slot {
     }
 
     // Whether T' (its biased halves at Tl) is negative; rare. Workgroup-uniform.
-    __device__ __forceinline__ u32 t_negative(const u32* Tl) {
+    __device__ __forceinline__ u32 t_negative(const u32* Tl, u32 K) {
         __syncthreads();  // every thread's halves written
-        if (tid() < 64) flag[1] = sign_of(Tl, 2 * k) & 1;
+        if (tid() < 64) flag[1] = sign_of(Tl, 2 * K) & 1;
         __syncthreads();
         const u32 neg = flag[1];
         __syncthreads();
@@ -597,11 +607,11 @@ template <u32 LOGC> struct Slot {
         load(v, ex);
         settle(v);
         __syncthreads();
-        forward<LOGC, LOGC>(v, A.w, lds, true);
+        forward<LOGC, LOGC>(v, A.w, lds, true, A.w.t0);
 #pragma unroll
         for (u32 e = 0; e < 16; e++) v[e] = Z{(v[e].r + v[e].i) * (v[e].r - v[e].i), 2.0 * v[e].r * v[e].i};
         settle(v);
-        inverse<LOGC, LOGC>(v, A.w, lds, true);
+        inverse<LOGC, LOGC>(v, A.w, lds, true, A.w.t0);
         __syncthreads();
         {
             const u32 x = G::at(tid());
@@ -632,6 +642,37 @@ template <u32 LOGC> struct Slot {
         return top - (u32)BETA + up;
     }
 
+    // x from the words (biased, carried; `top` stands above them) and the overflow check, for K limbs.
+    __device__ __forceinline__ u32 fix_x(u32 K, u32 top, u32 et, const u32* Tl) {
+        u32 bad = 0;
+        const u32 t = tid();
+        if (t < 64) {
+            u32* w = words();
+            if (t == 0) add_small(w, K, -(i64)(int)top);
+            wsync();
+            // X'' = words - bias is x, or x - (R + 1) where x > R / 2. A top word of zero leaves that open
+            // only if T / R is in the upper half itself (its top word is read then: x below R / 2
+            // is short of its bucket and has zeros there in every step).
+            u32 neg = w[K - 1] < SGN;
+            if (w[K - 1] == SGN && (et || Tl[2 * K - 1] - SGN >= 0x40000000u)) neg = sign_of(w, K) & 1;
+            ex = neg;
+            if (neg) {
+                if (t == 0) add_small(w, K, 1);
+                wsync();
+                if (sign_of(w, K) == 2) bad = 1;  // x = R stands as digits 0 and ex = 1
+            }
+            if (t == 0) flag[1] = neg;
+        }
+        __syncthreads();
+        // x is T / R + m N / R (within 1) with m N / R < N, or that less R + 1 if it passed R: the
+        // top limbs tell.
+        if (t == T - 1) {
+            const i64 d = (i64)words()[K - 1] - (i64)Tl[2 * K - 1] + ((i64)flag[1] << 32) - ((i64)et << 32);
+            bad |= d < -4;
+        }
+        return bad;
+    }
+
     // One step on the words; returns nonzero (in some thread) on a carry that must vanish but does not.
     __device__ __forceinline__ u32 step(u32 c, const double2* np, const double2* nh, u32* Tl) {
         u32 bad = 0, et;
@@ -640,7 +681,7 @@ template <u32 LOGC> struct Slot {
             et = square(c, lo, Tl);
             __syncthreads();
             if (et != 0) {  // T = T' + et R^2: only T' < 0 with et = 1 stands for a number below R^2
-                const u32 neg = t_negative(Tl);
+                const u32 neg = t_negative(Tl, k);
                 bad |= et != neg;
                 et = neg;
             }
@@ -652,10 +693,10 @@ template <u32 LOGC> struct Slot {
         load(v, 0);
         settle(v);
         __syncthreads();
-        forward<LOGC, LOGC>(v, A.w, lds, true);
+        forward<LOGC, LOGC>(v, A.w, lds, true, A.w.t0);
         Spectrum<T>(np, tid()).apply(v);
         settle(v);
-        inverse<LOGC, LOGC>(v, A.w, lds, true);
+        inverse<LOGC, LOGC>(v, A.w, lds, true, A.w.t0);
         __syncthreads();
         {
             const u32 x = G::at(tid());
@@ -675,10 +716,10 @@ template <u32 LOGC> struct Slot {
         load_half(v, on);
         settle(v);
         __syncthreads();
-        forward<LOGC, LOGC - 1>(v, A.w, lds, on);
+        forward<LOGC, LOGC - 1>(v, A.w, lds, on, A.w.t0);
         if (on) Spectrum<T / 2>(nh, tid()).apply(v);
         settle(v);
-        inverse<LOGC, LOGC - 1>(v, A.w, lds, on);
+        inverse<LOGC, LOGC - 1>(v, A.w, lds, on, A.w.t0);
         __syncthreads();
         if (on) {
             const u32 x = G::at(tid());
@@ -704,32 +745,7 @@ template <u32 LOGC> struct Slot {
         }
         put(l);
         __syncthreads();
-        const u32 t = tid();
-        if (t < 64) {
-            u32* w = words();
-            if (t == 0) add_small(w, k, -(i64)(int)top);
-            wsync();
-            // X'' = words - bias is x, or x - (R + 1) where x > R / 2. A top word of zero leaves that open
-            // only if T / R is in the upper half itself (its top word is read then: x below R / 2
-            // is short of its bucket and has zeros there in every step).
-            u32 neg = w[k - 1] < SGN;
-            if (w[k - 1] == SGN && (et || Tl[2 * k - 1] - SGN >= 0x40000000u)) neg = sign_of(w, k) & 1;
-            ex = neg;
-            if (neg) {
-                if (t == 0) add_small(w, k, 1);
-                wsync();
-                if (sign_of(w, k) == 2) bad = 1;  // x = R stands as digits 0 and ex = 1
-            }
-            if (t == 0) flag[1] = neg;
-        }
-        __syncthreads();
-        // x is T / R + m N / R (within 1) with m N / R < N, or that less R + 1 if it passed R: the
-        // top limbs tell.
-        if (t == T - 1) {
-            const i64 d = (i64)words()[k - 1] - (i64)Tl[2 * k - 1] + ((i64)flag[1] << 32) - ((i64)et << 32);
-            bad |= d < -4;
-        }
-        return bad;
+        return bad | fix_x(k, top, et, Tl);
     }
 
     // k limbs as digits into the words (barriers on both sides); returns the flag e (value =
@@ -816,7 +832,7 @@ __device__ __forceinline__ void constants(const Args& A, const u32* npl, const u
     s.load(v, 0);
     fence();
     __syncthreads();
-    forward<LOGC, LOGC>(v, A.w, lds, true);
+    forward<LOGC, LOGC>(v, A.w, lds, true, A.w.t0);
     const u32 t = tid();
 #pragma unroll
     for (u32 e = 0; e < 16; e++) np[T * e + t] = make_double2(v[e].r, v[e].i);
@@ -828,19 +844,312 @@ __device__ __forceinline__ void constants(const Args& A, const u32* npl, const u
     s.load_half(v, on);
     fence();
     __syncthreads();
-    forward<LOGC, LOGC - 1>(v, A.w, lds, on);
+    forward<LOGC, LOGC - 1>(v, A.w, lds, on, A.w.t0);
     if (on)
 #pragma unroll
         for (u32 e = 0; e < 16; e++) nh[T / 2 * e + t] = make_double2(v[e].r, v[e].i);
 }
 
+// ---- k = 16,384 (L = 32,768): the product in two parts --------------------------------------------
+// 32,768 complex elements would take every register of a CU. But X^C - i (C = 32,768) is (X^H - z)
+// (X^H + z), H = C / 2, z = exp(i pi / 4): the product modulo each factor is a weighted transform of
+// length H of a_j + z a_(j+H), or a_j - z a_(j+H) (weights exp(i pi j / 4H) and exp(5 i pi j / 4H)), and from
+// the two results A and B the coefficients are (A + B) / 2 and (A - B) / 2z. The parts run one
+// after the other on the length-16,384 machinery; the digits are kept packed and A as it is in the
+// slot's HBM scratch, each thread reading back only what it wrote. The last product has length H itself.
+// Coefficients are carried a quarter (8,192 limbs) at a time, what the staging buffer holds.
+//
+// The bound on the error is closest here, so counted in full (u = 2^-53; a complex product by a table
+// element or constant 3 u, with fused multiply-adds): a radix-16 pass 4 u and one inner rotation
+// 3 u, the four twiddle factors 12 u, radix 4 across lanes 2 u, weights 3 u; 38 u a transform, 3 u more
+// for the split, 4 u for the combination: 41 + 41 + 3 + 42 = 127 u, and C 2^30 127 2^-53 = 0.496.
+struct SplitSlot : Slot<14> {
+    typedef Slot<14> B;
+    static constexpr u32 H = C, K = 2 * k;  // limbs: K; `k` is half of them
+
+    __device__ __forceinline__ SplitSlot(const Args& a, unsigned char* l) : B(a, l) {}
+
+    // The element weights of a part (wave-uniform loads).
+    __device__ __forceinline__ const double2* weights(u32 p) const {
+        u64 w = (u64)(A.w.ts + 8 * T + 16 * p);
+        asm volatile("" : "+s"(w));
+        return (const double2*)w;
+    }
+    // Part p of the words' number, weighted; its digits go to dig in part 0 and come from it in part 1.
+    __device__ __forceinline__ void load_part(Z* v, u32 p, u32 top, u32* dig) {
+        const double2* w = weights(p);
+        const double s = p ? -RH : RH;
+        const u32 t = tid();
+#pragma unroll
+        for (u32 e = 0; e < 16; e++) {
+            u32 d;
+            if (p == 0) {
+                const u16* W = (const u16*)X;
+                d = (u32)W[t + T * e] | (u32)W[t + T * e + H] << 16;
+                d ^= SGN;
+                dig[T * e + t] = d;
+            } else
+                d = dig[T * e + t];
+            const double lo = (double)(int)(int16_t)d, hi = (double)((int)d >> 16);
+            double zr = __builtin_fma(hi, s, lo);
+            double zi = hi * s;
+            if (e == 0 && t == 0) zi += (double)top;
+            const double2 we = w[e];
+            v[e] = mulw<false>(Z{zr, zi}, we.x, we.y);
+            if (e % 4 == 3) fence();
+        }
+    }
+    // A product by both parts, from the words (barrier before): the square, or times the spectrum np.
+    // A is left in `part`, B in v.
+    __device__ __forceinline__ void parts(Z* v, u32 top, const double2* np, double2* part, u32* dig) {
+        u32 p = 0;
+#pragma clang loop unroll(disable)
+        do {
+            load_part(v, p, top, dig);
+            settle(v);
+            __syncthreads();
+            forward<14, 14>(v, A.w, lds, true, A.w.ts + 4 * T * p);
+            if (np) {
+                Spectrum<T>(np + H * p, tid()).apply(v);
+            } else {
+#pragma unroll
+                for (u32 e = 0; e < 16; e++) v[e] = Z{(v[e].r + v[e].i) * (v[e].r - v[e].i), 2.0 * v[e].r * v[e].i};
+            }
+            settle(v);
+            inverse<14, 14>(v, A.w, lds, true, A.w.ts + 4 * T * p);
+            const double2* w = weights(p);
+            const u32 t = tid();
+#pragma unroll
+            for (u32 e = 0; e < 16; e++) {
+                const double2 we = w[e];
+                v[e] = mulw<true>(v[e], we.x, we.y);
+                if (p == 0) part[T * e + t] = make_double2(v[e].r, v[e].i);
+                if (e % 4 == 3) fence();
+            }
+            settle(v);
+        } while (++p < 2);
+    }
+    // Quarter q of the coefficients of parts() into staging (barriers around it are the caller's).
+    __device__ __forceinline__ void stage_quarter(const Z* v, u32 q, const double2* part) {
+        const u32 t = tid(), x = G::at(t);
+#pragma unroll
+        for (u32 e = 0; e < 16; e++) {
+            const double2 a = part[T * e + t];
+            const double dr = a.x - v[e].r, di = a.y - v[e].i;
+            const double f = q == 0 ? a.x + v[e].r : q == 1 ? RH * (dr + di) : q == 2 ? a.y + v[e].i : RH * (di - dr);
+            stage<2 * H>(x + XT * e, f);
+            if (e % 4 == 3) fence();
+        }
+    }
+
+    // T = c x^2: biased limbs to Tl (2K; each thread rereads only its own). Returns what stands above T.
+    __device__ __forceinline__ u32 square(u32 c, u32* Tl, double2* part, u32* dig) {
+        Z v[16];
+        if (tid() == 0) flag[0] = ex;
+        parts(v, ex, nullptr, part, dig);
+        const u32 up = c * flag[0];  // as in Slot::square
+        u32 in = (u32)BETA + up, q = 0;
+#pragma clang loop unroll(disable)
+        do {
+            __syncthreads();
+            stage_quarter(v, q, part);
+            fence();
+            __syncthreads();
+            u32 l[8];
+            in = carry_staged(c, in, l, sc);
+            put_at(Tl + k * q, l);
+        } while (++q < 4);
+        return in - (u32)BETA + up;
+    }
+    // The low half of T into the words.
+    __device__ __forceinline__ void put_low(const u32* Tl) {
+#pragma unroll
+        for (u32 h = 0; h < 2; h++) {
+            u32 l[8];
+            const u32* p = Tl + k * h + 8 * tid();
+#pragma unroll
+            for (u32 i = 0; i < 8; i++) l[i] = p[i];
+            put_at(words() + k * h, l);
+        }
+    }
+
+    __device__ __forceinline__ u32 step(u32 c, const double2* np, const double2* nh, u32* Tl, double2* part, u32* dig) {
+        u32 bad = 0, et = square(c, Tl, part, dig);
+        __syncthreads();
+        if (et != 0) {  // as in Slot::step
+            const u32 neg = t_negative(Tl, K);
+            bad |= et != neg;
+            et = neg;
+        }
+        put_low(Tl);
+        __syncthreads();
+        Z v[16];
+        parts(v, 0, np, part, dig);
+        u32 l0[8], l1[8];
+        __syncthreads();
+        stage_quarter(v, 0, part);
+        fence();
+        __syncthreads();
+        const u32 mid = carry_staged(1, (u32)BETA, l0, sc + 64);
+        __syncthreads();
+        stage_quarter(v, 1, part);
+        fence();
+        __syncthreads();
+        carry_staged(1, mid, l1, sc + 32);
+        __syncthreads();
+        put_at(words(), l0);
+        put_at(words() + k, l1);
+        __syncthreads();
+        if (tid() < 64 && sign_of(words(), K) == 1 && tid() == 0) add_small(words(), K, -1);
+        __syncthreads();
+        // V = m N mod (R + 1).
+        {
+            const u32 t = tid();
+#pragma unroll
+            for (u32 e = 0; e < 16; e++) v[e] = mulw<false>(Z{digit(t + T * e), digit(t + T * e + H)}, wre(e), wim(e));
+        }
+        settle(v);
+        __syncthreads();
+        forward<14, 14>(v, A.w, lds, true, A.w.t0);
+        Spectrum<T>(nh, tid()).apply(v);
+        settle(v);
+        inverse<14, 14>(v, A.w, lds, true, A.w.t0);
+#pragma unroll
+        for (u32 e = 0; e < 16; e++) v[e] = mulw<true>(v[e], wre(e), wim(e));
+        settle(v);
+        u32 in = (u32)BETA - et;
+#pragma unroll
+        for (u32 h = 0; h < 2; h++) {
+            __syncthreads();
+            const u32 x = G::at(tid());
+#pragma unroll
+            for (u32 e = 0; e < 16; e++) stage<H>(x + XT * e, h ? v[e].i : v[e].r);
+            fence();
+            __syncthreads();
+            u64 s[8];
+            const u32 t = tid();
+            const u32* p = Tl + k * h + 8 * t;
+#pragma unroll
+            for (u32 i = 0; i < 8; i++) s[i] = (u64)((i64)p[K + i] - (i64)p[i] - sum(t, i)) + BIAS + SGN;
+            if (t == 0) s[0] += in;
+            in = bcarry<G::waves>(s, h ? l1 : l0, sc + 32 * h, t);
+        }
+        __syncthreads();
+        put_at(words(), l0);
+        put_at(words() + k, l1);
+        __syncthreads();
+        return bad | fix_x(K, in - (u32)BETA, et, Tl);
+    }
+
+    __device__ __forceinline__ u32 digits_in(const u32* src) {
+        u64 s[8];
+        u32 l0[8], l1[8];
+        const u32 t = tid();
+#pragma unroll
+        for (u32 i = 0; i < 8; i++) s[i] = (u64)src[8 * t + i] + SGN;
+        const u32 mid = bcarry<G::waves>(s, l0, sc + 64, t);
+#pragma unroll
+        for (u32 i = 0; i < 8; i++) s[i] = (u64)src[k + 8 * t + i] + SGN;
+        if (t == 0) s[0] += mid;
+        const u32 e = bcarry<G::waves>(s, l1, sc + 32, t);
+        __syncthreads();
+        put_at(words(), l0);
+        put_at(words() + k, l1);
+        __syncthreads();
+        return e;
+    }
+    // The number of `quarters` times 8,192 biased limbs at src, without its bias, to dst; returns the carry.
+    __device__ __forceinline__ u32 unbias_all(const u32* src, u32* dst, u32 quarters) {
+        u32 in = 1;
+#pragma clang loop unroll(disable)
+        for (u32 q = 0; q < quarters; q++) {
+            u32 l[8];
+            const u32* p = src + k * q + 8 * tid();
+#pragma unroll
+            for (u32 i = 0; i < 8; i++) l[i] = p[i];
+            __syncthreads();
+            in = unbias(l, in, sc + 64);
+            put_at(dst + k * q, l);
+        }
+        return in;
+    }
+};
+
+template <bool BARE> __device__ __forceinline__ void steps_split(const Args& A, u32 slot, u32 bits, unsigned char* lds) {
+    typedef SplitSlot S;
+    constexpr u32 K = S::K;
+    S s(A, lds);
+    u32* x = A.x + (size_t)slot * K;
+    const u32* ex = A.exp + (size_t)slot * A.ew;
+    const double2* np = A.np + (size_t)slot * 2 * S::H;
+    const double2* nh = A.n + (size_t)slot * S::H;
+    double2* part = A.part + (size_t)slot * S::H;
+    u32* dig = A.dig + (size_t)slot * S::H;
+    u32* Tl = A.lim + (size_t)slot * 3 * K;
+    const u32 nb = A.nbits[slot];
+    u32 pos = A.pos[slot], bad = 0;
+    const u32 first = pos;
+    if (!BARE) s.ex = s.digits_in(x);
+    for (u32 it = 0; it < bits && pos < nb; it++, pos++) {
+        const u32 c = (ex[pos >> 5] >> (31 - (pos & 31))) & 1 ? A.base : 1;
+        if constexpr (BARE) {
+            s.ex = s.digits_in(x);
+            const u32 e = s.square(c, Tl, part, dig);
+            const u32 top = s.unbias_all(Tl, Tl, 4);
+            bad |= top + e != 1;  // T = limbs + (top - 1 + e) R^2
+            __syncthreads();
+        } else {
+            bad |= s.step(c, np, nh, Tl, part, dig);
+        }
+    }
+    if (!BARE && pos != first) s.unbias_all(s.words(), x, 2);
+    if (tid() == 0) A.pos[slot] = pos;
+    if (bad) A.err[slot] = 1;
+}
+
+// The spectra of N' (both parts) and N of one slot from their limbs.
+__device__ __forceinline__ void constants_split(const Args& A, const u32* npl, const u32* nl, double2* np, double2* nh, u32* dig,
+                                                unsigned char* lds) {
+    typedef SplitSlot S;
+    constexpr u32 T = S::T, K = S::K, H = S::H;
+    S s(A, lds);
+    Z v[16];
+    s.digits_in(npl);
+    u32 p = 0;
+#pragma clang loop unroll(disable)
+    do {
+        s.load_part(v, p, 0, dig);
+        settle(v);
+        __syncthreads();
+        forward<14, 14>(v, A.w, lds, true, A.w.ts + 4 * T * p);
+        const u32 t = tid();
+#pragma unroll
+        for (u32 e = 0; e < 16; e++) np[H * p + T * e + t] = make_double2(v[e].r, v[e].i);
+        __syncthreads();
+    } while (++p < 2);
+    const u32 en = s.digits_in(nl);
+    if (tid() == 0 && en) add_small(s.words(), K, -1);
+    __syncthreads();
+    const u32 t = tid();
+#pragma unroll
+    for (u32 e = 0; e < 16; e++) v[e] = mulw<false>(Z{s.digit(t + T * e), s.digit(t + T * e + H)}, wre(e), wim(e));
+    settle(v);
+    __syncthreads();
+    forward<14, 14>(v, A.w, lds, true, A.w.t0);
+#pragma unroll
+    for (u32 e = 0; e < 16; e++) nh[T * e + t] = make_double2(v[e].r, v[e].i);
+}
+
 // Host side (mm_fd.hip).
 // Whether a batch of k limbs and base c can run on this path.
 bool fits(u32 k, u32 base);
-// The tables of complex length C, back to back: 7 C/16, C/16 and C/256 elements.
+// The tables of complex length C, back to back: 7 C/16, C/16, C/256, and for the split length 2C
+// C/2 and 32 elements.
 void make_tables(u32 C, double2* out);
-inline size_t table_elems(u32 C) { return C / 2 + C / 256; }
-inline Tables tables_at(const double2* p, u32 C) { return Tables{p, p + 7 * (C / 16), p + C / 2}; }
+inline size_t table_elems(u32 C) { return C + C / 256 + 32; }
+inline Tables tables_at(const double2* p, u32 C) { return Tables{p, p + 7 * (C / 16), p + C / 2, p + C / 2 + C / 256}; }
+// Transform length of a batch of k limbs: 2k, or k for the one that runs in two parts.
+inline u32 length(u32 k) { return k == 16384 ? k : 2 * k; }
 hipError_t set_lds_limit();
 hipError_t launch(const Args& A, u32 k, u32 slots, u32 bits, bool bare, hipStream_t sm);
 // The spectra of `count` slots from their limbs (npl, nl: k words per slot).

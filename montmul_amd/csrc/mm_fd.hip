@@ -1,4 +1,4 @@
-// mm_fd.hip - the double-precision step kernels of every length they run (L = 4,096 .. 16,384), in an
+// mm_fd.hip - the double-precision step kernels of every length they run (L = 4,096 .. 32,768), in an
 // object of their own, and their tables.
 
 #include "mm_fd.h"
@@ -25,8 +25,20 @@ __global__ __launch_bounds__(Geo<LOGC>::T) __attribute__((amdgpu_waves_per_eu(4)
     constants<LOGC>(A, npl + v * S::k, nl + v * S::k, np + v * S::C, nh + v * S::H, lds);
 }
 
-// k = 2,048 .. 8,192 limbs; c C <= 2^16 keeps the limb sums of T below BETA (2^32 - 1).
-bool fits(u32 k, u32 base) { return (k == 2048 || k == 4096 || k == 8192) && (u64)base * 2 * k <= 65536; }
+template <bool BARE> __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void k_steps_fd_split(Args A, u32 bits) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    steps_split<BARE>(A, blockIdx.x, bits, lds);
+}
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void k_constants_fd_split(Args A, const u32* npl, const u32* nl, double2* np,
+                                                                                                double2* nh, u32* dig) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    typedef SplitSlot S;
+    const size_t v = blockIdx.x;
+    constants_split(A, npl + v * S::K, nl + v * S::K, np + v * 2 * S::H, nh + v * S::H, dig + v * S::H, lds);
+}
+
+// k = 2,048 .. 16,384 limbs; c C < 2^17 keeps the limb sums of T below BETA (2^32 - 1).
+bool fits(u32 k, u32 base) { return k >= 2048 && k <= 16384 && (k & (k - 1)) == 0 && (u64)base * 2 * k < 131072; }
 
 void make_tables(u32 C, double2* out) {
     auto unit = [](u64 num, u64 den) {  // exp(2 pi i num / den), den a power of two >= 8
@@ -55,6 +67,12 @@ void make_tables(u32 C, double2* out) {
     out += C / 16;
     for (u32 m = 0; m < 16; m++)
         for (u32 j = 0; j < S2; j++) out[m * S2 + j] = unit((u64)j * m, S1);
+    out += C / 256;
+    for (u32 p = 0; p < 2; p++)
+        for (u32 a = 0; a < 4; a++)
+            for (u32 t = 0; t < T; t++) out[(4 * p + a) * T + t] = unit((u64)t * (32 * a + 4 * p + 1), 8ull * C);
+    for (u32 p = 0; p < 2; p++)
+        for (u32 e = 0; e < 16; e++) out[8 * T + 16 * p + e] = unit((4ull * p + 1) * e, 128);
 }
 
 template <u32 LOGC> static hipError_t limit() {
@@ -68,6 +86,8 @@ hipError_t set_lds_limit() {
     hipError_t e = limit<12>();
     if (e == hipSuccess) e = limit<13>();
     if (e == hipSuccess) e = limit<14>();
+    for (const void* k : {(const void*)k_steps_fd_split<false>, (const void*)k_steps_fd_split<true>, (const void*)k_constants_fd_split})
+        if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Geo<14>::lds);
     return e;
 }
 
@@ -84,6 +104,12 @@ hipError_t launch(const Args& A, u32 k, u32 slots, u32 bits, bool bare, hipStrea
         case 2048: return go<12>(A, slots, bits, bare, sm);
         case 4096: return go<13>(A, slots, bits, bare, sm);
         case 8192: return go<14>(A, slots, bits, bare, sm);
+        case 16384:
+            if (bare)
+                hipLaunchKernelGGL((k_steps_fd_split<true>), dim3(slots), dim3(1024), Geo<14>::lds, sm, A, bits);
+            else
+                hipLaunchKernelGGL((k_steps_fd_split<false>), dim3(slots), dim3(1024), Geo<14>::lds, sm, A, bits);
+            return hipGetLastError();
         default: return hipErrorInvalidValue;
     }
 }
@@ -99,6 +125,9 @@ hipError_t launch_constants(const Args& A, u32 k, u32 count, const u32* npl, con
         case 2048: return consts<12>(A, count, npl, nl, np, nh, sm);
         case 4096: return consts<13>(A, count, npl, nl, np, nh, sm);
         case 8192: return consts<14>(A, count, npl, nl, np, nh, sm);
+        case 16384:
+            hipLaunchKernelGGL(k_constants_fd_split, dim3(count), dim3(1024), Geo<14>::lds, sm, A, npl, nl, np, nh, A.dig);
+            return hipGetLastError();
         default: return hipErrorInvalidValue;
     }
 }

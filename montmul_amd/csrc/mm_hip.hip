@@ -717,7 +717,11 @@ struct State {
     }
     fd::Args fd_args() const {
         fd::Args A{};
-        A.w = fd::tables_at(fd_tab->p, len);
+        A.w = fd::tables_at(fd_tab->p, fd::length(k));
+        if (k == 16384) {  // the global mode's work vectors, which the register kernel's steps use
+            A.part = (double2*)d_work2;
+            A.dig = (uint32_t*)d_work1;
+        }
         A.x = d_x;
         A.np = d_fnp;
         A.n = d_fn;
@@ -1605,7 +1609,7 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
     if ((S->global || tune) && (dalloc(&S->d_work1, sl * n) || dalloc(&S->d_work2, sl * n) || dalloc(&S->d_lim, sl * 3 * k)))
         return 1;
     if (S->mx && dalloc(&S->d_nl, sl * 2 * k)) return 1;
-    if (S->fd && (get_fd_tables(C, st->len, &S->fd_tab) || dalloc(&S->d_fnp, sl * st->len) || dalloc(&S->d_fn, sl * (st->len / 2))))
+    if (S->fd && (get_fd_tables(C, fd::length(k), &S->fd_tab) || dalloc(&S->d_fnp, sl * st->len) || dalloc(&S->d_fn, sl * (st->len / 2))))
         return 1;
     if (v2ok) {
         if (dalloc(&S->d_iwc1, n) || dalloc(&S->d_iwc2, n)) return 1;
