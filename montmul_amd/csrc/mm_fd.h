@@ -12,8 +12,9 @@
 // 3.3 u (tables within u / 2), the last radix-2 or 4 stage 2 u: 49 u a transform. The two transforms
 // of a product, its pointwise step and the inverse make at most 150 u, and a coefficient of a b is
 // off by at most |a| |b| 150 u <= C 2^30 150 2^-53: 0.07, 0.15 and 0.29 at L = 4,096, 8,192 and
-// 16,384, below the 0.5 that rounding needs, for any digits (SplitSlot counts L = 32,768). (Random
-// digits err by 1e-4 or less.)
+// 16,384, below the 0.5 that rounding needs, for any digits (SplitSlot counts L = 32,768). Measured,
+// the farthest from an integer at L = 4,096 / 8,192 / 16,384 / 32,768: 6e-5 / 9e-5 / 1.2e-4 / 2.7e-4 on random
+// moduli, 0.003 / 0.006 / 0.012 / 0.024 on digits of the largest size with equal or alternating signs.
 //
 // A step, R = 2^(32k) = 2^(16 C):
 //     T = c x^2                  transform of length C, square, inverse
@@ -598,18 +599,22 @@ template <u32 LOGC> struct Slot {
         return neg;
     }
 
-    // T = c x^2 from the words (barrier before): biased limbs of its halves to Tl (k each; each
-    // thread rereads only its own), the low half in lo too. Returns what stands above T (in units
-    // of R^2, workgroup-uniform).
-    __device__ __forceinline__ u32 square(u32 c, u32* lo, u32* Tl) {
+    // T = c x^2, or c x times the number of spectrum `by` (digit C of that number: ea), from the words
+    // (barrier before): biased limbs of its halves to Tl (k each; each thread rereads only its
+    // own), the low half in lo too. Returns what stands above T (in units of R^2, workgroup-uniform).
+    __device__ __forceinline__ u32 square(u32 c, u32* lo, u32* Tl, const double2* by = nullptr, u32 ea = 1) {
         Z v[16];
-        if (tid() == 0) flag[0] = ex;
+        if (tid() == 0) flag[0] = ex & ea;
         load(v, ex);
         settle(v);
         __syncthreads();
         forward<LOGC, LOGC>(v, A.w, lds, true, A.w.t0);
+        if (by) {
+            Spectrum<T>(by, tid()).apply(v);
+        } else {
 #pragma unroll
-        for (u32 e = 0; e < 16; e++) v[e] = Z{(v[e].r + v[e].i) * (v[e].r - v[e].i), 2.0 * v[e].r * v[e].i};
+            for (u32 e = 0; e < 16; e++) v[e] = Z{(v[e].r + v[e].i) * (v[e].r - v[e].i), 2.0 * v[e].r * v[e].i};
+        }
         settle(v);
         inverse<LOGC, LOGC>(v, A.w, lds, true, A.w.t0);
         __syncthreads();
@@ -624,7 +629,7 @@ template <u32 LOGC> struct Slot {
         }
         fence();
         __syncthreads();
-        // Digit C of x, squared, stands at 2 C, where X^2C = -1: c more at the bottom and the top.
+        // The product of the digits C stands at 2 C, where X^2C = -1: c more at the bottom and the top.
         const u32 up = c * flag[0];
         const u32 mid = carry_staged(c, (u32)BETA + up, lo, sc);
         put_at(Tl, lo);
@@ -674,11 +679,11 @@ template <u32 LOGC> struct Slot {
     }
 
     // One step on the words; returns nonzero (in some thread) on a carry that must vanish but does not.
-    __device__ __forceinline__ u32 step(u32 c, const double2* np, const double2* nh, u32* Tl) {
+    __device__ __forceinline__ u32 step(u32 c, const double2* np, const double2* nh, u32* Tl, const double2* by = nullptr, u32 ea = 1) {
         u32 bad = 0, et;
         {
             u32 lo[8];
-            et = square(c, lo, Tl);
+            et = square(c, lo, Tl, by, ea);
             __syncthreads();
             if (et != 0) {  // T = T' + et R^2: only T' < 0 with et = 1 stands for a number below R^2
                 const u32 neg = t_negative(Tl, k);
@@ -821,6 +826,35 @@ template <u32 LOGC, bool BARE> __device__ __forceinline__ void steps(const Args&
     if (bad) A.err[slot] = 1;
 }
 
+// x[out] <- x[a] x[b] R^-1 with out's modulus (reference: `mul_slots`, lib.rs:963-988); `spec`: scratch
+// for the spectrum of x[a] (2k elements, each thread reads back its own) and T (2k limbs).
+template <u32 LOGC> __device__ __forceinline__ void product(const Args& A, u32 out, u32 a, u32 b, double2* spec, unsigned char* lds) {
+    typedef Slot<LOGC> S;
+    constexpr u32 k = S::k, T = S::T;
+    S s(A, lds);
+    const u32 ea = s.digits_in(A.x + (size_t)a * k);
+    {
+        Z v[16];
+        s.load(v, ea);
+        settle(v);
+        __syncthreads();
+        forward<LOGC, LOGC>(v, A.w, lds, true, A.w.t0);
+        const u32 t = tid();
+#pragma unroll
+        for (u32 e = 0; e < 16; e++) spec[T * e + t] = make_double2(v[e].r, v[e].i);
+        __syncthreads();
+    }
+    s.ex = s.digits_in(A.x + (size_t)b * k);
+    const u32 bad = s.step(1, A.np + (size_t)out * S::C, A.n + (size_t)out * S::H, (u32*)(spec + 2 * k), spec, ea);
+    u32 l[8];
+    const u32* w = s.words() + 8 * tid();
+#pragma unroll
+    for (u32 i = 0; i < 8; i++) l[i] = w[i];
+    s.unbias(l, 1, s.sc + 64);
+    s.put_at(A.x + (size_t)out * k, l);
+    if (bad) A.err[out] = 1;
+}
+
 // The spectra of N' and N of one slot from their limbs (k each).
 template <u32 LOGC>
 __device__ __forceinline__ void constants(const Args& A, const u32* npl, const u32* nl, double2* np, double2* nh, unsigned char* lds) {
@@ -942,11 +976,12 @@ struct SplitSlot : Slot<14> {
         }
     }
 
-    // T = c x^2: biased limbs to Tl (2K; each thread rereads only its own). Returns what stands above T.
-    __device__ __forceinline__ u32 square(u32 c, u32* Tl, double2* part, u32* dig) {
+    // T = c x^2, or by the spectrum `by`, as Slot::square: biased limbs to Tl (2K; each thread rereads
+    // only its own). Returns what stands above T.
+    __device__ __forceinline__ u32 square(u32 c, u32* Tl, double2* part, u32* dig, const double2* by = nullptr, u32 ea = 1) {
         Z v[16];
-        if (tid() == 0) flag[0] = ex;
-        parts(v, ex, nullptr, part, dig);
+        if (tid() == 0) flag[0] = ex & ea;
+        parts(v, ex, by, part, dig);
         const u32 up = c * flag[0];  // as in Slot::square
         u32 in = (u32)BETA + up, q = 0;
 #pragma clang loop unroll(disable)
@@ -973,8 +1008,9 @@ struct SplitSlot : Slot<14> {
         }
     }
 
-    __device__ __forceinline__ u32 step(u32 c, const double2* np, const double2* nh, u32* Tl, double2* part, u32* dig) {
-        u32 bad = 0, et = square(c, Tl, part, dig);
+    __device__ __forceinline__ u32 step(u32 c, const double2* np, const double2* nh, u32* Tl, double2* part, u32* dig,
+                                        const double2* by = nullptr, u32 ea = 1) {
+        u32 bad = 0, et = square(c, Tl, part, dig, by, ea);
         __syncthreads();
         if (et != 0) {  // as in Slot::step
             const u32 neg = t_negative(Tl, K);
@@ -1107,6 +1143,31 @@ template <bool BARE> __device__ __forceinline__ void steps_split(const Args& A, 
     if (bad) A.err[slot] = 1;
 }
 
+__device__ __forceinline__ void product_split(const Args& A, u32 out, u32 a, u32 b, double2* spec, unsigned char* lds) {
+    typedef SplitSlot S;
+    constexpr u32 K = S::K, H = S::H, T = S::T;
+    S s(A, lds);
+    u32* dig = A.dig + (size_t)out * H;
+    const u32 ea = s.digits_in(A.x + (size_t)a * K);
+    u32 p = 0;
+#pragma clang loop unroll(disable)
+    do {
+        Z v[16];
+        s.load_part(v, p, ea, dig);
+        settle(v);
+        __syncthreads();
+        forward<14, 14>(v, A.w, lds, true, A.w.ts + 4 * T * p);
+        const u32 t = tid();
+#pragma unroll
+        for (u32 e = 0; e < 16; e++) spec[H * p + T * e + t] = make_double2(v[e].r, v[e].i);
+        __syncthreads();
+    } while (++p < 2);
+    s.ex = s.digits_in(A.x + (size_t)b * K);
+    const u32 bad = s.step(1, A.np + (size_t)out * 2 * H, A.n + (size_t)out * H, (u32*)(spec + 2 * K), A.part + (size_t)out * H, dig, spec, ea);
+    s.unbias_all(s.words(), A.x + (size_t)out * K, 2);
+    if (bad) A.err[out] = 1;
+}
+
 // The spectra of N' (both parts) and N of one slot from their limbs.
 __device__ __forceinline__ void constants_split(const Args& A, const u32* npl, const u32* nl, double2* np, double2* nh, u32* dig,
                                                 unsigned char* lds) {
@@ -1152,6 +1213,9 @@ inline Tables tables_at(const double2* p, u32 C) { return Tables{p, p + 7 * (C /
 inline u32 length(u32 k) { return k == 16384 ? k : 2 * k; }
 hipError_t set_lds_limit();
 hipError_t launch(const Args& A, u32 k, u32 slots, u32 bits, bool bare, hipStream_t sm);
+// x[out] <- x[a] x[b] R^-1; spec: mul_elems(k) elements of scratch.
+inline size_t mul_elems(u32 k) { return 2 * k + k / 2; }
+hipError_t launch_mul(const Args& A, u32 k, u32 out, u32 a, u32 b, double2* spec, hipStream_t sm);
 // The spectra of `count` slots from their limbs (npl, nl: k words per slot).
 hipError_t launch_constants(const Args& A, u32 k, u32 count, const u32* npl, const u32* nl, double2* np, double2* nh, hipStream_t sm);
 

@@ -37,6 +37,17 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) void 
     constants_split(A, npl + v * S::K, nl + v * S::K, np + v * 2 * S::H, nh + v * S::H, dig + v * S::H, lds);
 }
 
+// One product; four waves per SIMD as the steps, whose code it shares.
+template <u32 LOGC>
+__global__ __launch_bounds__(LOGC == 15 ? 1024 : Geo<LOGC == 15 ? 14 : LOGC>::T) __attribute__((amdgpu_waves_per_eu(4))) void k_mul_fd(
+    Args A, u32 out, u32 a, u32 b, double2* spec) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    if constexpr (LOGC == 15)
+        product_split(A, out, a, b, spec, lds);
+    else
+        product<LOGC>(A, out, a, b, spec, lds);
+}
+
 // k = 2,048 .. 16,384 limbs; c C < 2^17 keeps the limb sums of T below BETA (2^32 - 1).
 bool fits(u32 k, u32 base) { return k >= 2048 && k <= 16384 && (k & (k - 1)) == 0 && (u64)base * 2 * k < 131072; }
 
@@ -76,7 +87,8 @@ void make_tables(u32 C, double2* out) {
 }
 
 template <u32 LOGC> static hipError_t limit() {
-    for (const void* k : {(const void*)k_steps_fd<LOGC, false>, (const void*)k_steps_fd<LOGC, true>, (const void*)k_constants_fd<LOGC>}) {
+    for (const void* k : {(const void*)k_steps_fd<LOGC, false>, (const void*)k_steps_fd<LOGC, true>, (const void*)k_constants_fd<LOGC>,
+                          (const void*)k_mul_fd<LOGC>}) {
         const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Geo<LOGC>::lds);
         if (e != hipSuccess) return e;
     }
@@ -86,7 +98,7 @@ hipError_t set_lds_limit() {
     hipError_t e = limit<12>();
     if (e == hipSuccess) e = limit<13>();
     if (e == hipSuccess) e = limit<14>();
-    for (const void* k : {(const void*)k_steps_fd_split<false>, (const void*)k_steps_fd_split<true>, (const void*)k_constants_fd_split})
+    for (const void* k : {(const void*)k_steps_fd_split<false>, (const void*)k_steps_fd_split<true>, (const void*)k_constants_fd_split, (const void*)k_mul_fd<15>})
         if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Geo<14>::lds);
     return e;
 }
@@ -130,6 +142,17 @@ hipError_t launch_constants(const Args& A, u32 k, u32 count, const u32* npl, con
             return hipGetLastError();
         default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_mul(const Args& A, u32 k, u32 out, u32 a, u32 b, double2* spec, hipStream_t sm) {
+    switch (k) {
+        case 2048: hipLaunchKernelGGL(k_mul_fd<12>, dim3(1), dim3(Geo<12>::T), Geo<12>::lds, sm, A, out, a, b, spec); break;
+        case 4096: hipLaunchKernelGGL(k_mul_fd<13>, dim3(1), dim3(Geo<13>::T), Geo<13>::lds, sm, A, out, a, b, spec); break;
+        case 8192: hipLaunchKernelGGL(k_mul_fd<14>, dim3(1), dim3(Geo<14>::T), Geo<14>::lds, sm, A, out, a, b, spec); break;
+        case 16384: hipLaunchKernelGGL(k_mul_fd<15>, dim3(1), dim3(1024), Geo<14>::lds, sm, A, out, a, b, spec); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
 }
 
 }  // namespace fd

@@ -649,6 +649,8 @@ struct State {
     bool fd = false;
     std::shared_ptr<FdTables> fd_tab;
     double2 *d_fnp = nullptr, *d_fn = nullptr;
+    double2* d_spec = nullptr;  // mul: its scratch (the spectrum of one factor, and T)
+    unsigned char* d_mul = nullptr;  // mul by the radix-4 kernel: its scratch, from the first one on
     uint32_t* d_coef = nullptr;  // n = 2^14 register step: coefficient staging, 6 n words per slot
     v2::S2* d_iwc2 = nullptr;
     // set_modulus staging (N' and N limbs, the half factors' work vectors), allocated on the
@@ -690,7 +692,7 @@ struct State {
                         (void*)d_nphat1, (void*)d_nhat1, (void*)d_work1, (void*)d_nphat2, (void*)d_nhat2, (void*)d_work2,
                         (void*)d_iwc1, (void*)d_iwc2, (void*)d_stage_lim, (void*)d_stage1, (void*)d_stage2, (void*)d_coef,
                         (void*)d_ones, (void*)d_ones_list, (void*)d_ones_out, (void*)d_nl,
-                        (void*)d_fnp, (void*)d_fn})
+                        (void*)d_fnp, (void*)d_fn, (void*)d_spec, (void*)d_mul})
             if (p) hipFree(p);
     }
     v2::VArgs vargs() const {
@@ -1609,7 +1611,7 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
     if ((S->global || tune) && (dalloc(&S->d_work1, sl * n) || dalloc(&S->d_work2, sl * n) || dalloc(&S->d_lim, sl * 3 * k)))
         return 1;
     if (S->mx && dalloc(&S->d_nl, sl * 2 * k)) return 1;
-    if (S->fd && (get_fd_tables(C, fd::length(k), &S->fd_tab) || dalloc(&S->d_fnp, sl * st->len) || dalloc(&S->d_fn, sl * (st->len / 2))))
+    if (S->fd && (get_fd_tables(C, fd::length(k), &S->fd_tab) || dalloc(&S->d_fnp, sl * st->len) || dalloc(&S->d_fn, sl * (st->len / 2)) || dalloc(&S->d_spec, fd::mul_elems(k))))
         return 1;
     if (v2ok) {
         if (dalloc(&S->d_iwc1, n) || dalloc(&S->d_iwc2, n)) return 1;
@@ -1762,30 +1764,61 @@ int64_t mm_run_group(void* const* states, size_t count, uint64_t bits, size_t* w
     return group_steps(G.data(), count, bits, which);
 }
 
+}  // extern "C"
+
+namespace {
+
+// Scratch of the radix-4 kernel's product: the spectrum of x_b and the working vector in both
+// fields, and 3k limbs.
+struct MulScratch {
+    size_t mb2, w1, w2, lim, bytes;
+    MulScratch(uint32_t n, uint32_t k) {
+        auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
+        mb2 = up(n * sizeof(F1));
+        w1 = mb2 + up(n * sizeof(F2));
+        w2 = w1 + up(n * sizeof(F1));
+        lim = w2 + up(n * sizeof(F2));
+        bytes = lim + up(12ull * k);
+    }
+};
+
+// x[out] <- x[a] x[b] R^-1 on the context's stream, by the kernel that steps the batch where that is
+// the matrix-core or the double-precision one, else by the radix-4 kernel in `scratch`, or in the
+// batch's own (allocated once) when that is null.
+hipError_t launch_mul(State* S, uint32_t out, uint32_t a, uint32_t b, unsigned char* scratch) {
+    hipStream_t sm = S->C->stream;
+    if (S->mx) return mx::launch_mul(S->mx_args(false), S->k, out, a, b, sm);
+    if (S->fd) return fd::launch_mul(S->fd_args(), S->k, out, a, b, S->d_spec, sm);
+    const MulScratch M(S->n, S->k);
+    if (!scratch) {
+        if (!S->d_mul) {
+            const hipError_t e = hipMalloc((void**)&S->d_mul, M.bytes);
+            if (e != hipSuccess) return e;
+        }
+        scratch = S->d_mul;
+    }
+    auto kern = S->wrap ? k_mul<true> : k_mul<false>;
+    hipLaunchKernelGGL(kern, dim3(1), dim3(S->threads), lds_scratch_bytes(S->threads), sm, S->args(), out, a, b, (F1*)scratch,
+                       (F2*)(scratch + M.mb2), (F1*)(scratch + M.w1), (F2*)(scratch + M.w2), (uint32_t*)(scratch + M.lim));
+    return hipGetLastError();
+}
+
+}  // namespace
+
+extern "C" {
+
 int64_t mm_mul(void* st, size_t out, size_t a, size_t b) {  // gpu/mod.rs:386-391
     State* S = (State*)st;
     Ctx* C = S->C;
     if (out >= S->slots || a >= S->slots || b >= S->slots) { fail("slot out of range"); return MM_EFAULT; }
     if (hipSetDevice(C->device) != hipSuccess || push(S)) return MM_EFAULT;
     S->failed.clear();
-    const uint32_t n = S->n, k = S->k;
-    F1 *mb1 = nullptr, *w1 = nullptr;
-    F2 *mb2 = nullptr, *w2 = nullptr;
-    uint32_t* lim = nullptr;
-    int64_t r = MM_EFAULT;
-    if (!dalloc(&mb1, n) && !dalloc(&mb2, n) && !dalloc(&w1, n) && !dalloc(&w2, n) && !dalloc(&lim, 3ull * k)) {
-        auto kern = S->wrap ? k_mul<true> : k_mul<false>;
-        hipLaunchKernelGGL(kern, dim3(1), dim3(S->threads), lds_scratch_bytes(S->threads), C->stream, S->args(), (uint32_t)out,
-                           (uint32_t)a, (uint32_t)b, mb1, mb2, w1, w2, lim);
-        hipError_t le = hipGetLastError();
-        hipError_t se = hipStreamSynchronize(C->stream);
-        if (le != hipSuccess) hip_fail("mul launch", le);
-        else if (se != hipSuccess) hip_fail("mul", se);
-        else r = check_err(S, "mul");
+    if (hipError_t e = launch_mul(S, (uint32_t)out, (uint32_t)a, (uint32_t)b, nullptr); e != hipSuccess) {
+        hip_fail("mul launch", e);
+        return MM_EFAULT;
     }
-    for (void* p : {(void*)mb1, (void*)mb2, (void*)w1, (void*)w2, (void*)lim}) if (p) hipFree(p);
     S->x_fresh[out] = 0;
-    return r;
+    return check_err(S, "mul");
 }
 
 // mm_mul with its scratch (the spectrum of x_b, the working vector, 3k limbs) carved from this
@@ -1799,9 +1832,7 @@ int64_t mm_mul_noalloc(void* st, size_t out, size_t a, size_t b) {
     if (out >= S->slots || a >= S->slots || b >= S->slots) { fail("slot out of range"); return MM_EFAULT; }
     if (!C->scratch) { fail("mul_noalloc: no fixed scratch on this device: " + C->scratch_err); return MM_EFAULT; }
     const uint32_t n = S->n, k = S->k;
-    auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
-    const size_t o_mb2 = up(n * sizeof(F1)), o_w1 = o_mb2 + up(n * sizeof(F2)), o_w2 = o_w1 + up(n * sizeof(F1));
-    const size_t o_lim = o_w2 + up(n * sizeof(F2)), need = o_lim + up(12ull * k);
+    const size_t need = MulScratch(n, k).bytes;
     if (need > MUL_SCRATCH_BYTES) {
         fail("mul_noalloc: length " + std::to_string(S->len) + " needs " + std::to_string(need) +
              " bytes of scratch, the fixed scratch holds " + std::to_string(MUL_SCRATCH_BYTES) + " (lengths up to 131072)");
@@ -1810,12 +1841,7 @@ int64_t mm_mul_noalloc(void* st, size_t out, size_t a, size_t b) {
     if (hipSetDevice(C->device) != hipSuccess) { fail("hipSetDevice failed"); return MM_EFAULT; }
     if (push_x(S)) return MM_EFAULT;
     S->failed.clear();
-    unsigned char* base = C->scratch;
-    auto kern = S->wrap ? k_mul<true> : k_mul<false>;
-    hipLaunchKernelGGL(kern, dim3(1), dim3(S->threads), lds_scratch_bytes(S->threads), C->stream, S->args(), (uint32_t)out,
-                       (uint32_t)a, (uint32_t)b, (F1*)base, (F2*)(base + o_mb2), (F1*)(base + o_w1), (F2*)(base + o_w2),
-                       (uint32_t*)(base + o_lim));
-    hipError_t le = hipGetLastError();
+    const hipError_t le = launch_mul(S, (uint32_t)out, (uint32_t)a, (uint32_t)b, C->scratch);
     if (le != hipSuccess) { hip_fail("mul_noalloc launch", le); return MM_EFAULT; }
     S->x_fresh[out] = 0;
     uint32_t err = 0;

@@ -325,7 +325,9 @@ template <u32 NB> struct Slot {
     static constexpr u32 EK = k >= 64 ? k / 64 : 1, AK = k / EK;  // limbs per lane of a residue, and lanes
     const Lane L;
     unsigned char* const lds;
-    u32 ex = 0, en = 0;  // x = x' + ex R, N = N'' + en R over the signed digits
+    // x = x' + ex R, N = N'' + en R over the signed digits; xb: the planes' factor of T, x itself
+    // between steps.
+    u32 ex = 0, exb = 0, en = 0;
 
     __device__ __forceinline__ Slot(u32 lane, unsigned char* base) : L(lane), lds(base) {}
 
@@ -354,7 +356,8 @@ template <u32 NB> struct Slot {
         for (u32 i = 0; i < EK; i++) v[i] = L.id < AK ? (u64)src[EK * L.id + i] + SGN : 0;
         return carry<EK, AK>(v, l, L.id);
     }
-    __device__ void init(const u32* x, const u32* np, const u32* n) {
+    // Factors x and xb (the same for steps), N' and N.
+    __device__ void init(const u32* x, const u32* xb, const u32* np, const u32* n) {
         for (u32 o = 16 * L.id; o < Y::st; o += 1024) *(v4i*)(lds + o) = v4i{0, 0, 0, 0};
         wsync();
         u32 l[EK];
@@ -364,6 +367,7 @@ template <u32 NB> struct Slot {
         put_planes(Y::nn, l);
         ex = digits_in(x, l);
         put(l);
+        exb = digits_in(xb, l);
         put_planes(Y::xb, l);
         wsync();
     }
@@ -403,7 +407,7 @@ template <u32 NB> struct Slot {
         return carry<EK, AK>(v, l, L.id);
     }
 
-    // T = c x^2 as biased limbs, low and high half; returns what stands above them (in units of
+    // T = c x xb as biased limbs, low and high half; returns what stands above them (in units of
     // R^2). The halves are carried one after the other, so that the sums of one half are staged.
     __device__ __forceinline__ u32 square(u32 c, u32* lo, u32* hi) {
         const unsigned char *X = lds + Y::op, *XB = lds + Y::xb;
@@ -428,14 +432,15 @@ template <u32 NB> struct Slot {
         }
         wsync();
         u32 top;
-        if (ex) {  // + c (2 x' R + R^2)
+        if (ex | exb) {  // + c (ex xb' R + exb x' R + ex exb R^2)
             u64 v[EK];
 #pragma unroll
             for (u32 i = 0; i < EK; i++) {
                 const u32 q = EK * L.id + i;
-                v[i] = L.id < AK ? (u64)((i64)c * (staged(i) + 2 * value(word(Y::op)[q]))) + BIAS + SGN + (q == 0 ? mid : 0) : 0;
+                const i64 more = (ex ? value(*word(Y::at(Y::xb, q))) : 0) + (exb ? value(word(Y::op)[q]) : 0);
+                v[i] = L.id < AK ? (u64)((i64)c * (staged(i) + more)) + BIAS + SGN + (q == 0 ? mid : 0) : 0;
             }
-            top = carry<EK, AK>(v, hi, L.id) + c;
+            top = carry<EK, AK>(v, hi, L.id) + c * (ex & exb);
         } else {
             top = carry_staged(c, mid, hi);  // mid holds the low half's BETA
         }
@@ -506,6 +511,7 @@ template <u32 NB> struct Slot {
             ex = sign_of<EK, AK>(l, L.id) & 1;
             bad |= f != ex;
         }
+        exb = ex;
         wsync();
         put(l);
         put_planes(Y::xb, l);
@@ -542,7 +548,8 @@ __device__ __forceinline__ void steps(const Args& A, u32 slot, u32 bits, u32 lan
     typedef Slot<NB> S;
     constexpr u32 k = S::k;
     S s(lane, lds);
-    s.init(A.x + (size_t)slot * k, A.np + (size_t)slot * k, A.n + (size_t)slot * k);
+    const u32* x0 = A.x + (size_t)slot * k;
+    s.init(x0, x0, A.np + (size_t)slot * k, A.n + (size_t)slot * k);
     const u32* ex = A.exp + (size_t)slot * A.ew;
     const u32 nb = A.nbits[slot];
     u32 pos = A.pos[slot], bad = 0;
@@ -569,10 +576,22 @@ __device__ __forceinline__ void steps(const Args& A, u32 slot, u32 bits, u32 lan
     }
 }
 
+// x[out] <- x[a] x[b] R^-1 with out's modulus, by one wave (reference: `mul_slots`, lib.rs:963-988).
+template <u32 NB> __device__ __forceinline__ void product_of(const Args& A, u32 out, u32 a, u32 b, u32 lane, unsigned char* lds) {
+    typedef Slot<NB> S;
+    constexpr size_t k = S::k;
+    S s(lane, lds);
+    s.init(A.x + a * k, A.x + b * k, A.np + out * k, A.n + out * k);
+    const u32 bad = s.step(1);
+    s.store_x(A.x + out * k);
+    if (lane == 0 && bad) A.err[out] = 1;
+}
+
 // Host side (mm_mx.hip): whether a batch can run on this path (log2 of the length L = 2k, the
 // base c), and the launch of its steps, one wave per slot.
 bool fits(u32 k, u32 base);
 hipError_t launch(const Args& A, u32 k, u32 slots, u32 bits, bool bare, hipStream_t sm);
+hipError_t launch_mul(const Args& A, u32 k, u32 out, u32 a, u32 b, hipStream_t sm);
 
 }  // namespace mx
 }  // namespace mm

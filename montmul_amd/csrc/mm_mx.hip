@@ -3,6 +3,8 @@
 
 #include "mm_mx.h"
 
+#include <type_traits>
+
 namespace mm {
 namespace mx {
 
@@ -10,6 +12,11 @@ template <u32 NB, bool BARE>
 __global__ __launch_bounds__(64) void k_steps_mx(Args A, u32 bits) {
     extern __shared__ __align__(16) unsigned char lds[];
     steps<NB, BARE>(A, blockIdx.x, bits, threadIdx.x, lds);
+}
+
+template <u32 NB> __global__ __launch_bounds__(64) void k_mul_mx(Args A, u32 out, u32 a, u32 b) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    product_of<NB>(A, out, a, b, threadIdx.x, lds);
 }
 
 // k = 8 .. 1,024 limbs. The limb sums stay below BETA (2^32 - 1) while c n <= 2^20.
@@ -32,18 +39,28 @@ template <u32 NB> static hipError_t go(const Args& A, u32 slots, u32 bits, bool 
     return hipGetLastError();
 }
 
-hipError_t launch(const Args& A, u32 k, u32 slots, u32 bits, bool bare, hipStream_t sm) {
+template <class Go> static hipError_t by_length(u32 k, Go&& g) {
     switch (k / 8) {
-        case 1: return go<1>(A, slots, bits, bare, sm);
-        case 2: return go<2>(A, slots, bits, bare, sm);
-        case 4: return go<4>(A, slots, bits, bare, sm);
-        case 8: return go<8>(A, slots, bits, bare, sm);
-        case 16: return go<16>(A, slots, bits, bare, sm);
-        case 32: return go<32>(A, slots, bits, bare, sm);
-        case 64: return go<64>(A, slots, bits, bare, sm);
-        case 128: return go<128>(A, slots, bits, bare, sm);
+        case 1: return g(std::integral_constant<u32, 1>());
+        case 2: return g(std::integral_constant<u32, 2>());
+        case 4: return g(std::integral_constant<u32, 4>());
+        case 8: return g(std::integral_constant<u32, 8>());
+        case 16: return g(std::integral_constant<u32, 16>());
+        case 32: return g(std::integral_constant<u32, 32>());
+        case 64: return g(std::integral_constant<u32, 64>());
+        case 128: return g(std::integral_constant<u32, 128>());
         default: return hipErrorInvalidValue;
     }
+}
+hipError_t launch(const Args& A, u32 k, u32 slots, u32 bits, bool bare, hipStream_t sm) {
+    return by_length(k, [&](auto nb) { return go<decltype(nb)::value>(A, slots, bits, bare, sm); });
+}
+hipError_t launch_mul(const Args& A, u32 k, u32 out, u32 a, u32 b, hipStream_t sm) {
+    return by_length(k, [&](auto nb) {
+        constexpr u32 NB = decltype(nb)::value;
+        hipLaunchKernelGGL(k_mul_mx<NB>, dim3(1), dim3(64), Lay<NB>::bytes, sm, A, out, a, b);
+        return hipGetLastError();
+    });
 }
 
 }  // namespace mx

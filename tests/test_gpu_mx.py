@@ -100,3 +100,35 @@ def test_matrix_step_carry_out_and_bare(default, length):
     if Hip.plan_of(b)["global"]:
         assert Hip.read_product(b, 0) == 4 * x * x
     b.free()
+
+
+@pytest.mark.parametrize("bits", [200, 1000, 2044, 8000, 20000, 32764, 40000, 100000, 200000, 300000])
+def test_mul_by_the_step_kernels(default, bits):
+    """mul on the matrix-core and double-precision kernels: random factors, values at the ends of the
+    range, factors in the upper half of [0, R) (each, and both), the output a factor, and a carry out."""
+    rng = random.Random(bits)
+    n = common.rand_odd(rng, bits)
+    b = ModBatch(default, [n] * 3, 2)
+    assert Hip.step_kernel(b) in (32, 64)
+    k = b.params().k
+    r = 1 << (32 * k)
+    nprime = -pow(n, -1, r) % r
+
+    def load(i, x):
+        assert default.table.load(ctypes.c_void_p(b.state), i, mm.to_limbs(x, k)) == 0
+
+    big = [rng.randrange(r // 2, r // 4 * 3) for _ in range(2)]
+    small = rng.randrange(2 * n)
+    for x, y in ((small, rng.randrange(2 * n)), (0, small), (2 * n - 1, 2 * n - 1), (1, n), (big[0], small), (small, big[1]), big):
+        for out in (0, 1, 2):
+            load(0, x)
+            load(1, y)
+            b.mul(out, 0, 1)
+            t = x * y
+            assert b.read_raw(out) == (t + (t % r * nprime) % r * n) >> (32 * k), (bits, out)
+    load(0, r - 1)
+    load(1, r - 1)
+    with pytest.raises(CarryError) as ei:
+        b.mul(2, 0, 1)
+    assert ei.value.slot == 2
+    b.free()
