@@ -72,7 +72,7 @@ template <u32 NB> struct Lay {
     static constexpr u32 plane = 4 * pad + 3 * (n / 2);
     static constexpr u32 xb = pl + pad, np = xb + n / 2 + pad, nn = np + n / 2 + pad;
     static constexpr u32 st = pl + 2 * plane;                // limb sums, 9 words of 8 bytes per 8 limbs
-    static constexpr u32 bytes = st + 9 * k;
+    static constexpr u32 bytes = st + 9 * k + (NB < 32 ? 8 : 0);  // and the limb below (high_product)
     // Limb q of the planes' operand at `area` (q = -1: zeros).
     static __device__ __forceinline__ u32 at(u32 area, int q) { return area + plane * ((u32)q >> 2 & 1) + 16 * (u32)(q >> 3) + 4 * ((u32)q & 3); }
 };
@@ -241,17 +241,20 @@ __device__ __forceinline__ v16i product1(const Lane& L, const unsigned char* A, 
     return acc[0];
 }
 
+// Rows 4 g .. 4 g + 3 of the lane's column as a limb: three multiply-adds (the multipliers are hidden
+// from the compiler, which would make shifts and adds of them).
+__device__ __forceinline__ i64 limb_sum(const v16i& acc, u32 g) {
+    int b8 = 1 << 8, b16 = 1 << 16, b24 = 1 << 24;
+    asm("" : "+s"(b8), "+s"(b16), "+s"(b24));
+    return acc[4 * g] + (i64)acc[4 * g + 1] * b8 + (i64)acc[4 * g + 2] * b16 + (i64)acc[4 * g + 3] * b24;
+}
 // Columns of a tile into limb sums: lane (j, h) holds rows 8 g + 4 h + (0 .. 3) of column j, the
 // four digits of limb 8 j + 2 g + h of the tile. Columns from `first`, `cols` of them.
 __device__ __forceinline__ void stage(i64* st, u32 tile, const v16i& acc, const Lane& L, u32 first, u32 cols) {
     const u32 j = L.j - first;
-    i64 b8 = 1 << 8, b16 = 1 << 16, b24 = 1 << 24;
-    asm("" : "+s"(b8), "+s"(b16), "+s"(b24));  // products: three multiply-adds, not shifts and adds
     if (j < cols) {
 #pragma unroll
-        for (u32 g = 0; g < 4; g++)
-            st[288 * tile + 9 * j + 2 * g + L.h] =
-                acc[4 * g] + (i64)acc[4 * g + 1] * (int)b8 + (i64)acc[4 * g + 2] * (int)b16 + (i64)acc[4 * g + 3] * (int)b24;
+        for (u32 g = 0; g < 4; g++) st[288 * tile + 9 * j + 2 * g + L.h] = limb_sum(acc, g);
     }
 }
 template <u32 E> __device__ __forceinline__ u32 stage_pos(u32 lane, u32 i) {
@@ -474,24 +477,11 @@ template <u32 NB> struct Slot {
         const u32 em = sign_of<EK, AK>(l, L.id) & 1;
         put(l);
         wsync();
-        // The last four low columns of m N, and with T's digits there q = (L + T mod R) / R.
-        int g0 = 0, g1 = 0, g2 = 0, g3 = 0;
-#pragma unroll
-        for (u32 r = 0; r < (k + 63) / 64; r++) {
-            const u32 w = 64 * r + L.id;
-            const int md = w < k ? (int)word(Y::op)[w] : 0;
-            const int W = w < k ? (int)(k - 1 - w) : 0;
-            const u32 hi = *word(Y::at(Y::nn, W)), lo = *word(Y::at(Y::nn, W - 1));
-            g0 = __builtin_amdgcn_sdot4(md, (int)__builtin_amdgcn_perm(hi, lo, 0x01020304u), g0, false);
-            g1 = __builtin_amdgcn_sdot4(md, (int)__builtin_amdgcn_perm(hi, lo, 0x02030405u), g1, false);
-            g2 = __builtin_amdgcn_sdot4(md, (int)__builtin_amdgcn_perm(hi, lo, 0x03040506u), g2, false);
-            g3 = __builtin_amdgcn_sdot4(md, (int)__builtin_amdgcn_perm(hi, lo, 0x04050607u), g3, false);
-        }
-        const i64 cols = (i64)wave_sum(g0) + ((i64)wave_sum(g1) << 8) + ((i64)wave_sum(g2) << 16) + ((i64)wave_sum(g3) << 24);
+        // The last four low columns of m N, and with T's digits there q = (L + T mod R) / R; then the
+        // high columns.
+        const i64 cols = high_product();
         const i64 q = (cols + tlow + (1ll << 31)) >> 32;
         // x = floor(T / R) + the high columns of m N + q + e_m N + e_N m.
-        high_product();
-        wsync();
         u64 v[EK];
 #pragma unroll
         for (u32 i = 0; i < EK; i++) {
@@ -529,14 +519,37 @@ template <u32 NB> struct Slot {
             stage(sums(), 0, product1<NB>(L, lds + Y::op, lds + Y::np, 0), L, 0, NB);
         }
     }
-    __device__ __forceinline__ void high_product() {
+    // The high columns' limb sums of m N into staging; returns the sum of the limb below them. Below
+    // n = 1,024 the tile has columns to spare and starts one of them lower (the dot products and their
+    // reduction were 4 % of a step at L = 64, 2 % at 256); above, that limb's four columns come by dot
+    // products.
+    __device__ __forceinline__ i64 high_product() {
         if constexpr (NB >= 32) {
+            int g0 = 0, g1 = 0, g2 = 0, g3 = 0;
+#pragma unroll
+            for (u32 r = 0; r < k / 64; r++) {
+                const u32 w = 64 * r + L.id, W = k - 1 - w;
+                const int md = (int)word(Y::op)[w];
+                const u32 hi = *word(Y::at(Y::nn, (int)W)), lo = *word(Y::at(Y::nn, (int)W - 1));
+                g0 = __builtin_amdgcn_sdot4(md, (int)__builtin_amdgcn_perm(hi, lo, 0x01020304u), g0, false);
+                g1 = __builtin_amdgcn_sdot4(md, (int)__builtin_amdgcn_perm(hi, lo, 0x02030405u), g1, false);
+                g2 = __builtin_amdgcn_sdot4(md, (int)__builtin_amdgcn_perm(hi, lo, 0x03040506u), g2, false);
+                g3 = __builtin_amdgcn_sdot4(md, (int)__builtin_amdgcn_perm(hi, lo, 0x04050607u), g3, false);
+            }
+            const i64 cols = (i64)wave_sum(g0) + ((i64)wave_sum(g1) << 8) + ((i64)wave_sum(g2) << 16) + ((i64)wave_sum(g3) << 24);
             v16i acc[Q];
             product<NB, Q, 2 * Q>(L, lds + Y::op, lds + Y::nn, acc);
 #pragma unroll
             for (u32 t = 0; t < Q; t++) stage(sums(), t, acc[t], L, 0, 32);
+            wsync();
+            return cols;
         } else {
-            stage(sums(), 0, product1<NB>(L, lds + Y::op, lds + Y::nn, (int)NB), L, 0, NB);
+            // Column 0 is the last below R: its limb 7 stands past the sums of the others.
+            const v16i acc = product1<NB>(L, lds + Y::op, lds + Y::nn, (int)NB - 1);
+            stage(sums(), 0, acc, L, 1, NB);
+            if (L.id == 32) sums()[9 * NB] = limb_sum(acc, 3);
+            wsync();
+            return sums()[9 * NB];
         }
     }
 };
