@@ -1,4 +1,4 @@
-// mm_fd.h - the Montgomery step on double-precision transforms (wraparound path, L = 4,096 ..
+// mm_fd.h - the Montgomery step on double-precision transforms (wraparound path, L = 2,048 ..
 // 32,768, k = L / 2 limbs).
 //
 // A residue is C = L signed digits of 16 bits (-2^15 .. 2^15), in double precision, which issues one
@@ -11,8 +11,8 @@
 // 2 x 3 u (its inner rotations), each of the four twiddle factors between passes and the weights
 // 3.3 u (tables within u / 2), the last radix-2 or 4 stage 2 u: 49 u a transform. The two transforms
 // of a product, its pointwise step and the inverse make at most 150 u, and a coefficient of a b is
-// off by at most |a| |b| 150 u <= C 2^30 150 2^-53: 0.07, 0.15 and 0.29 at L = 4,096, 8,192 and
-// 16,384, below the 0.5 that rounding needs, for any digits (SplitSlot counts L = 32,768). Measured,
+// off by at most |a| |b| 150 u <= C 2^30 150 2^-53: 0.04, 0.07, 0.15 and 0.29 at L = 2,048, 4,096,
+// 8,192 and 16,384, below the 0.5 that rounding needs, for any digits (SplitSlot counts L = 32,768). Measured,
 // the farthest from an integer at L = 4,096 / 8,192 / 16,384 / 32,768: 6e-5 / 9e-5 / 1.2e-4 / 2.7e-4 on random
 // moduli, 0.003 / 0.006 / 0.012 / 0.024 on digits of the largest size with equal or alternating signs.
 //
@@ -30,9 +30,11 @@
 // component at a time (8 bytes per element), so that two workgroups share a CU at L = 8,192 beside
 // the later passes' twiddles, which stay in LDS.
 //
-// Measured against the modular transforms (mm_v2.h) that it replaces by default: L = 4,096 (1,024
-// slots) 7.0 -> 15.7 M squarings/s, 8,192 (4,096 slots) 3.6 -> 9.1 M, 16,384 (1,024 slots) 1.31 -> 3.7 M,
-// 32,768 (1,024 slots) 0.42 -> 1.18 M; one slot alone at 8,192 92 -> 34 us a step, at 32,768 560 -> 147 us.
+// Measured against the modular transforms (mm_v2.h) that it replaces by default: L = 2,048 (2,048
+// slots) 14.4 -> 36 M squarings/s (30 M on the matrix cores, whose work grows as n^2; at 1,024 they
+// do 91 M, and this step, by its work, 75 M), 4,096 (1,024 slots) 7.0 -> 15.7 M, 8,192 (4,096
+// slots) 3.6 -> 9.1 M, 16,384 (1,024 slots) 1.31 -> 3.7 M, 32,768 (1,024 slots) 0.42 -> 1.18 M;
+// one slot alone at 8,192 92 -> 34 us a step, at 32,768 560 -> 147 us.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -87,7 +89,7 @@ template <u32 LOGC> struct Geo {
     // LDS: the exchange buffer (doubles), passes 1 and 2's twiddles, carry scratch, flags.
     static constexpr u32 xwords = C + C / 16;
     static constexpr u32 o1 = xwords * 8, o2 = o1 + 256 * S1, osc = o2 + 256 * R2, lds = osc + 3 * 32 * 4 + 16;
-    static_assert(LOGC >= 11 && LOGC <= 14, "2,048 <= C <= 16,384");
+    static_assert(LOGC >= 10 && LOGC <= 14, "1,024 <= C <= 16,384");
     // Exchange position: 16 R elements and R of padding, which spreads the strides of the second
     // exchange over the banks.
     static __device__ __forceinline__ u32 at(u32 p) { return p + R * (p / (16 * R)); }
@@ -308,7 +310,7 @@ template <u32 T> struct Spectrum {
 };
 
 // Buffer positions of a thread's elements S apart, relative to the first: with the padding (16 R
-// divides S, or S = 8 and R = 1), or within one block.
+// divides S, or S divides 16, R = 1 and the first is below S in its block), or within one block.
 constexpr u32 WITHIN = 1u << 31;
 __device__ __forceinline__ constexpr u32 spaced(u32 S, u32 e) { return S & WITHIN ? (S & ~WITHIN) * e : S * e + S * e / 16; }
 // Exchange of one component at a time: element e written at w + spaced(WS, e), read at
@@ -340,8 +342,8 @@ template <bool BLOCK, u32 WS, u32 RS> __device__ __forceinline__ void exchange(Z
 }
 
 // Positions of thread t's elements: pass 0 at t + T e, pass 1 at p1 + S1 e, pass 2 at p2 + R e. At
-// C = 2,048 pass 2 is two 8-point transforms of neighbours. x0, x1, x2: the first one's position in
-// the buffer.
+// C = 2,048 and 1,024 pass 2 is two 8-point or four 4-point transforms of neighbours. x0, x1, x2: the
+// first one's position in the buffer.
 template <u32 LOGC> struct Pos {
     typedef Geo<LOGC> G;
     static constexpr u32 X0 = G::T, X1 = G::S1, X2 = G::R | WITHIN;  // spacings of the passes' elements
@@ -357,11 +359,14 @@ template <u32 LOGC> struct Pos {
     }
 };
 
-// Pass 2's butterflies: one of 16 points, or two of 8 where only 8 are left.
+// Pass 2's butterflies: one of 16 points, or two of 8 or four of 4 where no more are left.
 template <u32 LOGC, bool INV> __device__ __forceinline__ void last16(Z* v) {
     if constexpr (LOGC >= 12)
         dft16<INV>(v);
-    else {
+    else if constexpr (LOGC == 10) {
+#pragma unroll
+        for (u32 g = 0; g < 16; g += 4) dft4<INV>(v[g], v[g + 1], v[g + 2], v[g + 3]);
+    } else {
         dft8<INV>(v);
         dft8<INV>(v + 8);
     }

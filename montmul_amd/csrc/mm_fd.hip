@@ -1,4 +1,4 @@
-// mm_fd.hip - the double-precision step kernels of every length they run (L = 4,096 .. 32,768), in an
+// mm_fd.hip - the double-precision step kernels of every length they run (L = 2,048 .. 32,768), in an
 // object of their own, and their tables.
 
 #include "mm_fd.h"
@@ -48,8 +48,8 @@ __global__ __launch_bounds__(LOGC == 15 ? 1024 : Geo<LOGC == 15 ? 14 : LOGC>::T)
         product<LOGC>(A, out, a, b, spec, lds);
 }
 
-// k = 2,048 .. 16,384 limbs; c C < 2^17 keeps the limb sums of T below BETA (2^32 - 1).
-bool fits(u32 k, u32 base) { return k >= 2048 && k <= 16384 && (k & (k - 1)) == 0 && (u64)base * 2 * k < 131072; }
+// k = 1,024 .. 16,384 limbs; c C < 2^17 keeps the limb sums of T below BETA (2^32 - 1).
+bool fits(u32 k, u32 base) { return k >= 1024 && k <= 16384 && (k & (k - 1)) == 0 && (u64)base * 2 * k < 131072; }
 
 void make_tables(u32 C, double2* out) {
     auto unit = [](u64 num, u64 den) {  // exp(2 pi i num / den), den a power of two >= 8
@@ -95,7 +95,8 @@ template <u32 LOGC> static hipError_t limit() {
     return hipSuccess;
 }
 hipError_t set_lds_limit() {
-    hipError_t e = limit<12>();
+    hipError_t e = limit<11>();
+    if (e == hipSuccess) e = limit<12>();
     if (e == hipSuccess) e = limit<13>();
     if (e == hipSuccess) e = limit<14>();
     for (const void* k : {(const void*)k_steps_fd_split<false>, (const void*)k_steps_fd_split<true>, (const void*)k_constants_fd_split, (const void*)k_mul_fd<15>})
@@ -113,6 +114,7 @@ template <u32 LOGC> static hipError_t go(const Args& A, u32 slots, u32 bits, boo
 }
 hipError_t launch(const Args& A, u32 k, u32 slots, u32 bits, bool bare, hipStream_t sm) {
     switch (k) {
+        case 1024: return go<11>(A, slots, bits, bare, sm);
         case 2048: return go<12>(A, slots, bits, bare, sm);
         case 4096: return go<13>(A, slots, bits, bare, sm);
         case 8192: return go<14>(A, slots, bits, bare, sm);
@@ -134,6 +136,7 @@ static hipError_t consts(const Args& A, u32 count, const u32* npl, const u32* nl
 }
 hipError_t launch_constants(const Args& A, u32 k, u32 count, const u32* npl, const u32* nl, double2* np, double2* nh, hipStream_t sm) {
     switch (k) {
+        case 1024: return consts<11>(A, count, npl, nl, np, nh, sm);
         case 2048: return consts<12>(A, count, npl, nl, np, nh, sm);
         case 4096: return consts<13>(A, count, npl, nl, np, nh, sm);
         case 8192: return consts<14>(A, count, npl, nl, np, nh, sm);
@@ -146,6 +149,7 @@ hipError_t launch_constants(const Args& A, u32 k, u32 count, const u32* npl, con
 
 hipError_t launch_mul(const Args& A, u32 k, u32 out, u32 a, u32 b, double2* spec, hipStream_t sm) {
     switch (k) {
+        case 1024: hipLaunchKernelGGL(k_mul_fd<11>, dim3(1), dim3(Geo<11>::T), Geo<11>::lds, sm, A, out, a, b, spec); break;
         case 2048: hipLaunchKernelGGL(k_mul_fd<12>, dim3(1), dim3(Geo<12>::T), Geo<12>::lds, sm, A, out, a, b, spec); break;
         case 4096: hipLaunchKernelGGL(k_mul_fd<13>, dim3(1), dim3(Geo<13>::T), Geo<13>::lds, sm, A, out, a, b, spec); break;
         case 8192: hipLaunchKernelGGL(k_mul_fd<14>, dim3(1), dim3(Geo<14>::T), Geo<14>::lds, sm, A, out, a, b, spec); break;

@@ -1581,9 +1581,8 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
     }
     // The matrix-core step and the double-precision step run every plan that names no transform
     // kernel, mode or tile of its own
-    // (force_global at n >= 512 is the default plan). Its work grows as n^2: at L = 2,048 it does
-    // 25 M squarings/s against the transforms' 14.4 M; L = 4,096 would take 4.6 K matrix
-    // instructions a step, 37 K cycles of a CU at best, where the double-precision step takes 39 K.
+    // (force_global at n >= 512 is the default plan). The first one's work grows as n^2: at L = 1,024 it
+    // does 91 M squarings/s, where the second would do 75 M by its work; at 2,048 30 M against 36 M.
     const bool unnamed = wrap && !tune && !C->opts.prefer_lds && C->opts.tile == 0 && C->opts.slots_per_cu == 0 &&
                          (v2ok || (!C->opts.force_global && !(kenv && strcmp(kenv, "v1") == 0)));
     S->mx = unnamed && mx::fits(k, st->base);

@@ -26,7 +26,7 @@
 // them nonnegative through the carry.
 //
 // Measured against the transform kernels it replaces by default (4,096 slots unless said):
-// L = 1,024 30.6 -> 91 M squarings/s, 2,048 (2,048 slots) 14.4 -> 30 M; one step of a slot among 64
+// L = 1,024 30.6 -> 91 M squarings/s; one step of a slot among 64
 // at L = 512 59 -> 5.6 us, of one among 16 at L = 256 53 -> 2.8 us (the radix-4 kernel's barriers).
 // At L = 1,024 power binds as much as issue: a loop of these instructions alone on random digits
 // runs at 1.64 of 2.4 GHz, this kernel with its matrix cores 60 % busy at 1.75. Before the planes, the

@@ -1,4 +1,4 @@
-// mm_mx.hip - the matrix-core step kernels of every length they run (L = 16 .. 2,048), in an
+// mm_mx.hip - the matrix-core step kernels of every length they run (L = 16 .. 1,024), in an
 // object of their own.
 
 #include "mm_mx.h"
@@ -19,8 +19,8 @@ template <u32 NB> __global__ __launch_bounds__(64) void k_mul_mx(Args A, u32 out
     product_of<NB>(A, out, a, b, threadIdx.x, lds);
 }
 
-// k = 8 .. 1,024 limbs. The limb sums stay below BETA (2^32 - 1) while c n <= 2^20.
-bool fits(u32 k, u32 base) { return k >= 8 && k <= 1024 && (k & (k - 1)) == 0 && (u64)base * 4 * k <= (1u << 20); }
+// k = 8 .. 512 limbs. The limb sums stay below BETA (2^32 - 1) while c n <= 2^20.
+bool fits(u32 k, u32 base) { return k >= 8 && k <= 512 && (k & (k - 1)) == 0 && (u64)base * 4 * k <= (1u << 20); }
 
 // Dynamic LDS of a workgroup (one wave): padded so that a whole number of waves per SIMD fits a CU's
 // 160 KiB. At L = 1,024 nine waves would fit, one SIMD has three of them and the others wait for it:
@@ -48,7 +48,6 @@ template <class Go> static hipError_t by_length(u32 k, Go&& g) {
         case 16: return g(std::integral_constant<u32, 16>());
         case 32: return g(std::integral_constant<u32, 32>());
         case 64: return g(std::integral_constant<u32, 64>());
-        case 128: return g(std::integral_constant<u32, 128>());
         default: return hipErrorInvalidValue;
     }
 }

@@ -1,4 +1,4 @@
-"""The double-precision step (L = 4,096 .. 32,768) against the closed form and the oracle, bit for
+"""The double-precision step (L = 2,048 .. 32,768) against the closed form and the oracle, bit for
 bit, with digits at the ends of their range, where rounding has the least room."""
 
 import ctypes
@@ -13,8 +13,9 @@ from oracle_backends import Gmp
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [(32765, 4096), (50001, 4096), (65532, 4096), (65533, 8192), (100000, 8192), (131068, 8192), (131069, 16384),
-         (200003, 16384), (262140, 16384), (262141, 32768), (400000, 32768), (524284, 32768)]
+SIZES = [(16381, 2048), (20000, 2048), (32764, 2048), (32765, 4096), (50001, 4096), (65532, 4096), (65533, 8192), (100000, 8192), (131068, 8192), (131069, 16384),
+         (200003, 16384), (262140, 16384), (262141, 32768),
+         (400000, 32768), (524284, 32768)]
 
 
 @pytest.fixture(scope="module")
@@ -45,7 +46,7 @@ def pattern(words, k):
     return int.from_bytes((b * (4 * k // len(b) + 1))[: 4 * k], "little")
 
 
-@pytest.mark.parametrize("length", [4096, 8192, 16384, 32768])
+@pytest.mark.parametrize("length", [2048, 4096, 8192, 16384, 32768])
 def test_double_step_edges(default, length):
     """One step at the ends of the range and on digits of the largest size (0x7fff, 0x8000 and
     alternating signs), and for raw values in the upper half of [0, R) (x = x' + R)."""
@@ -78,7 +79,7 @@ def test_double_step_edges(default, length):
             b.free()
 
 
-@pytest.mark.parametrize("length", [4096, 8192, 16384, 32768])
+@pytest.mark.parametrize("length", [2048, 4096, 8192, 16384, 32768])
 def test_double_step_carry_out_bare_and_readmission(default, length):
     """A carry out names its slots; run_bare leaves x and T = c x^2; a replaced modulus is used."""
     k = length // 2
