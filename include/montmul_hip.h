@@ -166,6 +166,11 @@ int mm_set_exponent(void *state, size_t slot, const uint32_t *words, size_t nwor
 int64_t mm_run(void *state, uint64_t bits);                            /* gpu/mod.rs:383-385 */
 int64_t mm_mul(void *state, size_t out, size_t a, size_t b);           /* gpu/mod.rs:386-391 */
 int mm_read(void *state, size_t slot, uint32_t *out);                  /* gpu/mod.rs:392-394 */
+/* mm_read after the conversion out of Montgomery form on the device: x R^-1 mod N, k limbs, or N itself
+ * for 0. Returns 0; 1 on an error; -1 when the value is on the host already (loaded, or read with
+ * mm_read) or the caller's own conversion is the faster one: it uses mm_read then. No reference
+ * counterpart: the reference converts on the host (batch.rs:173-176). */
+int mm_read_plain(void *state, size_t slot, uint32_t *out);
 uint64_t mm_remaining(void *state, size_t slot);                       /* gpu/mod.rs:395-397 */
 const char *mm_last_error(void);
 

@@ -128,6 +128,7 @@ def _load_lib():
         "mm_push": (C.c_int, [vp]),
         "mm_plan": (C.c_int, [vp, C.POINTER(PlanInfo)]),
         "mm_step_kernel": (C.c_int, [vp]),
+        "mm_read_plain": (C.c_int, [vp, C.c_size_t, u32p]),
         "mm_free_memory": (C.c_uint64, [vp]),
         "mm_cu_count": (C.c_int, [vp]),
         "mm_max_lds": (C.c_uint64, [vp]),

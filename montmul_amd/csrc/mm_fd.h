@@ -697,6 +697,11 @@ template <u32 LOGC> struct Slot {
             }
             put(lo);
         }
+        return bad | reduce(np, nh, Tl, et);
+    }
+    // x = (T + m N) / R from T: its biased halves at Tl, the low one in the words too, and what stands
+    // above them: 1 for T' < 0, else 0.
+    __device__ __forceinline__ u32 reduce(const double2* np, const double2* nh, const u32* Tl, u32 et) {
         // m = (T mod R) N' mod R.
         __syncthreads();
         Z v[16];
@@ -755,7 +760,7 @@ template <u32 LOGC> struct Slot {
         }
         put(l);
         __syncthreads();
-        return bad | fix_x(k, top, et, Tl);
+        return fix_x(k, top, et, Tl);
     }
 
     // k limbs as digits into the words (barriers on both sides); returns the flag e (value =
@@ -858,6 +863,30 @@ template <u32 LOGC> __device__ __forceinline__ void product(const Args& A, u32 o
     s.unbias(l, 1, s.sc + 64);
     s.put_at(A.x + (size_t)out * k, l);
     if (bad) A.err[out] = 1;
+}
+
+// x[slot] R^-1 mod N to `out` (k limbs; N itself may stand for 0): the reduction of T = x, kept at Tl (2k
+// limbs). For any x below R: (x + m N) / R < N + 1.
+template <u32 LOGC> __device__ __forceinline__ void plain(const Args& A, u32 slot, u32* out, u32* Tl, unsigned char* lds) {
+    typedef Slot<LOGC> S;
+    constexpr u32 k = S::k;
+    S s(A, lds);
+    const u32 e = s.digits_in(A.x + (size_t)slot * k), t = tid();
+    u32 l[8], hi[8];
+    const u32* w = s.words() + 8 * t;
+#pragma unroll
+    for (u32 i = 0; i < 8; i++) {
+        l[i] = w[i];
+        hi[i] = SGN + (t == 0 && i == 0 ? e : 0);
+    }
+    s.put_at(Tl, l);
+    s.put_at(Tl + k, hi);
+    s.reduce(A.np + (size_t)slot * S::C, A.n + (size_t)slot * S::H, Tl, 0);
+    w = s.words() + 8 * tid();
+#pragma unroll
+    for (u32 i = 0; i < 8; i++) l[i] = w[i];
+    s.unbias(l, 1, s.sc + 64);
+    s.put_at(out, l);
 }
 
 // The spectra of N' and N of one slot from their limbs (k each).
@@ -1023,6 +1052,9 @@ struct SplitSlot : Slot<14> {
             et = neg;
         }
         put_low(Tl);
+        return bad | reduce(np, nh, Tl, et, part, dig);
+    }
+    __device__ __forceinline__ u32 reduce(const double2* np, const double2* nh, const u32* Tl, u32 et, double2* part, u32* dig) {
         __syncthreads();
         Z v[16];
         parts(v, 0, np, part, dig);
@@ -1079,7 +1111,7 @@ struct SplitSlot : Slot<14> {
         put_at(words(), l0);
         put_at(words() + k, l1);
         __syncthreads();
-        return bad | fix_x(K, in - (u32)BETA, et, Tl);
+        return fix_x(K, in - (u32)BETA, et, Tl);
     }
 
     __device__ __forceinline__ u32 digits_in(const u32* src) {
@@ -1173,6 +1205,27 @@ __device__ __forceinline__ void product_split(const Args& A, u32 out, u32 a, u32
     if (bad) A.err[out] = 1;
 }
 
+__device__ __forceinline__ void plain_split(const Args& A, u32 slot, u32* out, u32* Tl, unsigned char* lds) {
+    typedef SplitSlot S;
+    constexpr u32 k = S::k, K = S::K;
+    S s(A, lds);
+    const u32 e = s.digits_in(A.x + (size_t)slot * K), t = tid();
+#pragma unroll
+    for (u32 h = 0; h < 2; h++) {
+        u32 l[8], hi[8];
+        const u32* w = s.words() + k * h + 8 * t;
+#pragma unroll
+        for (u32 i = 0; i < 8; i++) {
+            l[i] = w[i];
+            hi[i] = SGN + (h == 0 && t == 0 && i == 0 ? e : 0);
+        }
+        s.put_at(Tl + k * h, l);
+        s.put_at(Tl + K + k * h, hi);
+    }
+    s.reduce(A.np + (size_t)slot * 2 * S::H, A.n + (size_t)slot * S::H, Tl, 0, A.part + (size_t)slot * S::H, A.dig + (size_t)slot * S::H);
+    s.unbias_all(s.words(), out, 2);
+}
+
 // The spectra of N' (both parts) and N of one slot from their limbs.
 __device__ __forceinline__ void constants_split(const Args& A, const u32* npl, const u32* nl, double2* np, double2* nh, u32* dig,
                                                 unsigned char* lds) {
@@ -1221,6 +1274,8 @@ hipError_t launch(const Args& A, u32 k, u32 slots, u32 bits, bool bare, hipStrea
 // x[out] <- x[a] x[b] R^-1; spec: mul_elems(k) elements of scratch.
 inline size_t mul_elems(u32 k) { return 2 * k + k / 2; }
 hipError_t launch_mul(const Args& A, u32 k, u32 out, u32 a, u32 b, double2* spec, hipStream_t sm);
+// x R^-1 mod N (or N for 0) of `count` slots from `first`: k limbs each to out; T: 2k limbs each.
+hipError_t launch_plain(const Args& A, u32 k, u32 first, u32 count, u32* out, u32* T, hipStream_t sm);
 // The spectra of `count` slots from their limbs (npl, nl: k words per slot).
 hipError_t launch_constants(const Args& A, u32 k, u32 count, const u32* npl, const u32* nl, double2* np, double2* nh, hipStream_t sm);
 

@@ -48,6 +48,18 @@ __global__ __launch_bounds__(LOGC == 15 ? 1024 : Geo<LOGC == 15 ? 14 : LOGC>::T)
         product<LOGC>(A, out, a, b, spec, lds);
 }
 
+template <u32 LOGC>
+__global__ __launch_bounds__(LOGC == 15 ? 1024 : Geo<LOGC == 15 ? 14 : LOGC>::T) __attribute__((amdgpu_waves_per_eu(4))) void k_plain_fd(
+    Args A, u32 first, u32* out, u32* T) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    constexpr size_t k = 1u << (LOGC - 1);
+    const size_t row = blockIdx.x;
+    if constexpr (LOGC == 15)
+        plain_split(A, first + blockIdx.x, out + row * k, T + row * 2 * k, lds);
+    else
+        plain<LOGC>(A, first + blockIdx.x, out + row * k, T + row * 2 * k, lds);
+}
+
 // k = 1,024 .. 16,384 limbs; c C < 2^17 keeps the limb sums of T below BETA (2^32 - 1).
 bool fits(u32 k, u32 base) { return k >= 1024 && k <= 16384 && (k & (k - 1)) == 0 && (u64)base * 2 * k < 131072; }
 
@@ -88,7 +100,7 @@ void make_tables(u32 C, double2* out) {
 
 template <u32 LOGC> static hipError_t limit() {
     for (const void* k : {(const void*)k_steps_fd<LOGC, false>, (const void*)k_steps_fd<LOGC, true>, (const void*)k_constants_fd<LOGC>,
-                          (const void*)k_mul_fd<LOGC>}) {
+                          (const void*)k_mul_fd<LOGC>, (const void*)k_plain_fd<LOGC>}) {
         const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Geo<LOGC>::lds);
         if (e != hipSuccess) return e;
     }
@@ -99,7 +111,8 @@ hipError_t set_lds_limit() {
     if (e == hipSuccess) e = limit<12>();
     if (e == hipSuccess) e = limit<13>();
     if (e == hipSuccess) e = limit<14>();
-    for (const void* k : {(const void*)k_steps_fd_split<false>, (const void*)k_steps_fd_split<true>, (const void*)k_constants_fd_split, (const void*)k_mul_fd<15>})
+    for (const void* k : {(const void*)k_steps_fd_split<false>, (const void*)k_steps_fd_split<true>, (const void*)k_constants_fd_split, (const void*)k_mul_fd<15>,
+                          (const void*)k_plain_fd<15>})
         if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Geo<14>::lds);
     return e;
 }
@@ -154,6 +167,19 @@ hipError_t launch_mul(const Args& A, u32 k, u32 out, u32 a, u32 b, double2* spec
         case 4096: hipLaunchKernelGGL(k_mul_fd<13>, dim3(1), dim3(Geo<13>::T), Geo<13>::lds, sm, A, out, a, b, spec); break;
         case 8192: hipLaunchKernelGGL(k_mul_fd<14>, dim3(1), dim3(Geo<14>::T), Geo<14>::lds, sm, A, out, a, b, spec); break;
         case 16384: hipLaunchKernelGGL(k_mul_fd<15>, dim3(1), dim3(1024), Geo<14>::lds, sm, A, out, a, b, spec); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_plain(const Args& A, u32 k, u32 first, u32 count, u32* out, u32* T, hipStream_t sm) {
+    const dim3 g(count);
+    switch (k) {
+        case 1024: hipLaunchKernelGGL(k_plain_fd<11>, g, dim3(Geo<11>::T), Geo<11>::lds, sm, A, first, out, T); break;
+        case 2048: hipLaunchKernelGGL(k_plain_fd<12>, g, dim3(Geo<12>::T), Geo<12>::lds, sm, A, first, out, T); break;
+        case 4096: hipLaunchKernelGGL(k_plain_fd<13>, g, dim3(Geo<13>::T), Geo<13>::lds, sm, A, first, out, T); break;
+        case 8192: hipLaunchKernelGGL(k_plain_fd<14>, g, dim3(Geo<14>::T), Geo<14>::lds, sm, A, first, out, T); break;
+        case 16384: hipLaunchKernelGGL(k_plain_fd<15>, g, dim3(1024), Geo<14>::lds, sm, A, first, out, T); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -673,6 +673,11 @@ struct State {
     // Reads of consecutive slots: the slot that would continue them, and the rows that the latest
     // copy brought (mm_read doubles it).
     size_t read_next = 0, read_rows = 1;
+    // mm_read_plain: the rows of the latest copies as numbers below N (or N for 0), which of them stand
+    // for the device's x, and the device's side of a copy; allocated by the first one.
+    std::unique_ptr<uint32_t[]> h_plain;
+    std::vector<uint8_t> plain_fresh;
+    uint32_t* d_plain = nullptr;
     std::vector<uint8_t> x_dirty;     // rows written on the host since the last upload
     std::vector<uint32_t> x_dirty_list;
     std::vector<std::vector<uint32_t>> exps;
@@ -692,8 +697,17 @@ struct State {
                         (void*)d_nphat1, (void*)d_nhat1, (void*)d_work1, (void*)d_nphat2, (void*)d_nhat2, (void*)d_work2,
                         (void*)d_iwc1, (void*)d_iwc2, (void*)d_stage_lim, (void*)d_stage1, (void*)d_stage2, (void*)d_coef,
                         (void*)d_ones, (void*)d_ones_list, (void*)d_ones_out, (void*)d_nl,
-                        (void*)d_fnp, (void*)d_fn, (void*)d_spec, (void*)d_mul})
+                        (void*)d_fnp, (void*)d_fn, (void*)d_spec, (void*)d_mul, (void*)d_plain})
             if (p) hipFree(p);
+    }
+    // The device's x of a slot, or of all, is another than the host's copies.
+    void x_changed(size_t i) {
+        x_fresh[i] = 0;
+        if (!plain_fresh.empty()) plain_fresh[i] = 0;
+    }
+    void x_changed() {
+        std::fill(x_fresh.begin(), x_fresh.end(), 0);
+        std::fill(plain_fresh.begin(), plain_fresh.end(), 0);
     }
     v2::VArgs vargs() const {
         v2::VArgs A{};
@@ -1066,7 +1080,7 @@ int64_t steps(State* S, uint64_t bits, bool bare) {
         S->ms_per_slot_step[bare] = std::max(1e-6, (double)ms) / ((double)(s * reps) * std::max<uint32_t>(1, S->slots));
         int64_t r = check_err(S, bare ? "run_bare" : "run");
         for (uint32_t i = 0; i < S->slots; i++) S->pos[i] += (uint32_t)std::min<uint64_t>(s * reps, S->nbits[i] - S->pos[i]);
-        if (!bare) std::fill(S->x_fresh.begin(), S->x_fresh.end(), 0);
+        if (!bare) S->x_changed();
         if (r != MM_OK) return r;
         left -= s * reps;
     }
@@ -1449,7 +1463,7 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
                 if (which) *which = g;
             }
             for (uint32_t i = 0; i < S->slots; i++) S->pos[i] += (uint32_t)std::min<uint64_t>(s * reps, S->nbits[i] - S->pos[i]);
-            std::fill(S->x_fresh.begin(), S->x_fresh.end(), 0);
+            S->x_changed();
         }
         if (first != MM_OK) return first;
         left -= s * reps;
@@ -1678,6 +1692,7 @@ int mm_load(void* st, size_t i, const uint32_t* limbs) {  // gpu/mod.rs:371-375
     State* S = (State*)st;
     if (i >= S->slots) return fail("slot out of range");
     std::copy(limbs, limbs + S->k, S->h_x.begin() + i * S->k);
+    if (!S->plain_fresh.empty()) S->plain_fresh[i] = 0;
     if (!S->x_dirty[i]) {
         S->x_dirty[i] = 1;
         S->x_dirty_list.push_back((uint32_t)i);
@@ -1707,6 +1722,7 @@ int mm_set_modulus(void* st, size_t i, const uint32_t* nl, const uint32_t* npl, 
     (void)two_n;  // the device path has no use for 2N
     if (i >= S->slots) return fail("slot out of range");
     if (hipSetDevice(C->device) != hipSuccess) return fail("hipSetDevice failed");
+    if (!S->plain_fresh.empty()) S->plain_fresh[i] = 0;
     S->ones_set[i] = 0;  // the values of 1 belong to the old modulus until set_ones
     const uint32_t k = S->k, n = S->n;
     hipStream_t sm = C->stream;
@@ -1781,6 +1797,20 @@ struct MulScratch {
     }
 };
 
+// Rows that a read of slot i, absent on the host, brings with it: the device row alone (the reference
+// downloads every slot here, gpu/mod.rs:247-269); a read that continues the one before brings up to
+// twice the rows of that one, at most 4 MiB: a batch read slot after slot waited 24 us for each
+// row's copy. *rows: the count for the next one to double.
+size_t read_rows_max(const State* S) { return std::max<size_t>(1, (1u << 20) / S->k); }
+size_t read_window(const State* S, size_t i, bool plain, size_t* rows) {
+    *rows = i == S->read_next ? std::min(2 * S->read_rows, read_rows_max(S)) : 1;
+    plain = plain && !S->plain_fresh.empty();
+    auto absent = [&](size_t j) { return !S->x_dirty[j] && !S->x_fresh[j] && !(plain && S->plain_fresh[j]); };
+    size_t c = 1;
+    while (c < *rows && i + c < S->slots && absent(i + c)) c++;
+    return c;
+}
+
 // x[out] <- x[a] x[b] R^-1 on the context's stream, by the kernel that steps the batch where that is
 // the matrix-core or the double-precision one, else by the radix-4 kernel in `scratch`, or in the
 // batch's own (allocated once) when that is null.
@@ -1816,7 +1846,7 @@ int64_t mm_mul(void* st, size_t out, size_t a, size_t b) {  // gpu/mod.rs:386-39
         hip_fail("mul launch", e);
         return MM_EFAULT;
     }
-    S->x_fresh[out] = 0;
+    S->x_changed(out);
     return check_err(S, "mul");
 }
 
@@ -1842,7 +1872,7 @@ int64_t mm_mul_noalloc(void* st, size_t out, size_t a, size_t b) {
     S->failed.clear();
     const hipError_t le = launch_mul(S, (uint32_t)out, (uint32_t)a, (uint32_t)b, C->scratch);
     if (le != hipSuccess) { hip_fail("mul_noalloc launch", le); return MM_EFAULT; }
-    S->x_fresh[out] = 0;
+    S->x_changed(out);
     uint32_t err = 0;
     hipError_t e = hipMemcpyAsync(&err, S->d_err + out, 4, hipMemcpyDeviceToHost, C->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(C->stream);
@@ -1902,13 +1932,8 @@ int mm_read(void* st, size_t i, uint32_t* out) {  // gpu/mod.rs:392-394
     State* S = (State*)st;
     if (i >= S->slots) return fail("slot out of range");
     if (!S->x_dirty[i] && !S->x_fresh[i]) {
-        // The device row alone (the reference downloads every slot here, gpu/mod.rs:247-269); a
-        // read that continues the one before brings twice the rows of that one, up to 4 MiB: a
-        // batch read slot after slot waited 24 us for each row's copy.
-        const size_t most = std::max<size_t>(1, (1u << 20) / S->k);
-        const size_t rows = i == S->read_next ? std::min(2 * S->read_rows, most) : 1;
-        size_t c = 1;
-        while (c < rows && i + c < S->slots && !S->x_dirty[i + c] && !S->x_fresh[i + c]) c++;
+        size_t rows;
+        const size_t c = read_window(S, i, false, &rows);
         if (hipSetDevice(S->C->device) != hipSuccess) return fail("hipSetDevice failed");
         HIPCHK(hipMemcpyAsync(S->h_x.data() + i * S->k, S->d_x + i * S->k, c * S->k * 4, hipMemcpyDeviceToHost, S->C->stream));
         HIPCHK(hipStreamSynchronize(S->C->stream));
@@ -1917,6 +1942,44 @@ int mm_read(void* st, size_t i, uint32_t* out) {  // gpu/mod.rs:392-394
         S->read_rows = rows;
     }
     std::copy(S->h_x.begin() + i * S->k, S->h_x.begin() + (i + 1) * S->k, out);
+    return 0;
+}
+
+int mm_read_plain(void* st, size_t i, uint32_t* out) {
+    State* S = (State*)st;
+    if (i >= S->slots) return fail("slot out of range");
+    if ((!S->mx && !S->fd) || S->x_dirty[i] || S->x_fresh[i]) return -1;
+    const size_t k = S->k;
+    if (S->plain_fresh.empty() || !S->plain_fresh[i]) {
+        // One launch converts the rows of a window: 2.5 us a row at 9,001 bits, copy and call included,
+        // where the host's product and division took 13 us (1.5 against 1.6 at 400 bits, 12 against 510
+        // at 120,000). The double-precision lengths gain with a single row too (39 us against 62 at
+        // 20,000 bits); below them the launch costs what the division does (34 us with either).
+        size_t rows;
+        const size_t c = read_window(S, i, true, &rows);
+        if (S->mx && c < 8) return -1;
+        if (hipSetDevice(S->C->device) != hipSuccess) return fail("hipSetDevice failed");
+        const size_t cap = std::min<size_t>(S->slots, read_rows_max(S));
+        if (!S->h_plain) S->h_plain.reset(new (std::nothrow) uint32_t[S->slots * k]);
+        if (!S->h_plain) return -1;
+        if (!S->d_plain && hipMalloc((void**)&S->d_plain, cap * k * (S->fd ? 12 : 4)) != hipSuccess) {
+            S->d_plain = nullptr;
+            (void)hipGetLastError();
+            return -1;
+        }
+        hipStream_t sm = S->C->stream;
+        if (S->mx)
+            HIPCHK(mx::launch_plain(S->mx_args(false), S->k, (uint32_t)i, (uint32_t)c, S->d_plain, sm));
+        else
+            HIPCHK(fd::launch_plain(S->fd_args(), S->k, (uint32_t)i, (uint32_t)c, S->d_plain, S->d_plain + cap * k, sm));
+        HIPCHK(hipMemcpyAsync(S->h_plain.get() + i * k, S->d_plain, c * k * 4, hipMemcpyDeviceToHost, sm));
+        HIPCHK(hipStreamSynchronize(sm));
+        if (S->plain_fresh.empty()) S->plain_fresh.assign(S->slots, 0);
+        std::fill(S->plain_fresh.begin() + i, S->plain_fresh.begin() + i + c, 1);
+        S->read_next = i + c;
+        S->read_rows = rows;
+    }
+    std::copy(S->h_plain.get() + i * k, S->h_plain.get() + (i + 1) * k, out);
     return 0;
 }
 

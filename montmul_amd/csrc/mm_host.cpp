@@ -377,8 +377,19 @@ int mm_modbatch_read_raw(mm_modbatch* b, size_t i, uint32_t* out) {  // batch.rs
 }
 
 int mm_modbatch_read(mm_modbatch* b, size_t i, uint32_t* out) {  // batch.rs:173-176
-    if (mm_modbatch_read_raw(b, i, out)) return 1;
+    if (check_slot(b, i)) return 1;
     const MmModulus& m = b->moduli[i];
+    if (b->be.read == mm_read) {  // the Hip backend converts many rows at once
+        const int r = mm_read_plain(b->state, i, out);
+        if (r > 0) return fail(b->be.last_error());
+        if (r == 0) {
+            Mpz x;
+            from_signed_limbs(x.v, 1, out, b->k);
+            if (mpz_cmp(x.v, m.n.v) == 0) memset(out, 0, b->k * 4);
+            return 0;
+        }
+    }
+    if (mm_modbatch_read_raw(b, i, out)) return 1;
     Mpz x;
     from_signed_limbs(x.v, 1, out, b->k);
     mpz_mul(x.v, x.v, m.rinv.v);

@@ -466,6 +466,11 @@ template <u32 NB> struct Slot {
             bad |= et != neg;
             et = neg;
         }
+        return bad | reduce(l, hi, et);
+    }
+    // x = (T + m N) / R from T's biased halves (l, hi) and what stands above them: 1 for T' < 0, else 0.
+    __device__ __forceinline__ u32 reduce(u32* l, const u32* hi, u32 et) {
+        u32 bad = 0;
         // T's top limb below R, for q.
         const i64 tlow = (i64)rdlane(l[EK - 1], AK - 1) - (i64)SGN;
         put(l);
@@ -600,11 +605,29 @@ template <u32 NB> __device__ __forceinline__ void product_of(const Args& A, u32 
     if (lane == 0 && bad) A.err[out] = 1;
 }
 
+// x[slot] R^-1 mod N to `out` (k limbs; N itself may stand for 0), by one wave: the reduction of T = x. For
+// any x below R: (x + m N) / R < N + 1.
+template <u32 NB> __device__ __forceinline__ void plain(const Args& A, u32 slot, u32* out, u32 lane, unsigned char* lds) {
+    typedef Slot<NB> S;
+    constexpr u32 k = S::k;
+    S s(lane, lds);
+    const u32* x = A.x + (size_t)slot * k;
+    s.init(x, x, A.np + (size_t)slot * k, A.n + (size_t)slot * k);
+    u32 l[S::EK], hi[S::EK];
+    const u32 e = s.digits_in(x, l);
+#pragma unroll
+    for (u32 i = 0; i < S::EK; i++) hi[i] = SGN + (S::EK * lane + i == 0 ? e : 0);
+    s.reduce(l, hi, 0);
+    s.store_x(out);
+}
+
 // Host side (mm_mx.hip): whether a batch can run on this path (log2 of the length L = 2k, the
 // base c), and the launch of its steps, one wave per slot.
 bool fits(u32 k, u32 base);
 hipError_t launch(const Args& A, u32 k, u32 slots, u32 bits, bool bare, hipStream_t sm);
 hipError_t launch_mul(const Args& A, u32 k, u32 out, u32 a, u32 b, hipStream_t sm);
+// x R^-1 mod N (or N for 0) of `count` slots from `first`: k limbs each to out.
+hipError_t launch_plain(const Args& A, u32 k, u32 first, u32 count, u32* out, hipStream_t sm);
 
 }  // namespace mx
 }  // namespace mm

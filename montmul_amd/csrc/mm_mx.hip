@@ -19,6 +19,11 @@ template <u32 NB> __global__ __launch_bounds__(64) void k_mul_mx(Args A, u32 out
     product_of<NB>(A, out, a, b, threadIdx.x, lds);
 }
 
+template <u32 NB> __global__ __launch_bounds__(64) void k_plain_mx(Args A, u32 first, u32* out) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    plain<NB>(A, first + blockIdx.x, out + (size_t)blockIdx.x * Slot<NB>::k, threadIdx.x, lds);
+}
+
 // k = 8 .. 512 limbs. The limb sums stay below BETA (2^32 - 1) while c n <= 2^20.
 bool fits(u32 k, u32 base) { return k >= 8 && k <= 512 && (k & (k - 1)) == 0 && (u64)base * 4 * k <= (1u << 20); }
 
@@ -58,6 +63,13 @@ hipError_t launch_mul(const Args& A, u32 k, u32 out, u32 a, u32 b, hipStream_t s
     return by_length(k, [&](auto nb) {
         constexpr u32 NB = decltype(nb)::value;
         hipLaunchKernelGGL(k_mul_mx<NB>, dim3(1), dim3(64), Lay<NB>::bytes, sm, A, out, a, b);
+        return hipGetLastError();
+    });
+}
+hipError_t launch_plain(const Args& A, u32 k, u32 first, u32 count, u32* out, hipStream_t sm) {
+    return by_length(k, [&](auto nb) {
+        constexpr u32 NB = decltype(nb)::value;
+        hipLaunchKernelGGL(k_plain_mx<NB>, dim3(count), dim3(64), lds_bytes<NB>(), sm, A, first, out);
         return hipGetLastError();
     });
 }

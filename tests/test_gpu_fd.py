@@ -13,9 +13,8 @@ from oracle_backends import Gmp
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [(16381, 2048), (20000, 2048), (32764, 2048), (32765, 4096), (50001, 4096), (65532, 4096), (65533, 8192), (100000, 8192), (131068, 8192), (131069, 16384),
-         (200003, 16384), (262140, 16384), (262141, 32768),
-         (400000, 32768), (524284, 32768)]
+SIZES = [(16381, 2048), (20000, 2048), (32764, 2048), (32765, 4096), (50001, 4096), (65532, 4096), (65533, 8192),
+         (100000, 8192), (131068, 8192), (131069, 16384), (200003, 16384), (262140, 16384), (262141, 32768), (400000, 32768), (524284, 32768)]
 
 
 @pytest.fixture(scope="module")
