@@ -61,6 +61,7 @@ def build(verbose=False, out=LIB, extra=()):
     hip_obj = os.path.join(OUT_DIR, "mm_hip.o")
     mx_obj = os.path.join(OUT_DIR, "mm_mx.o")
     fd_obj = os.path.join(OUT_DIR, "mm_fd.o")
+    fdw_obj = os.path.join(OUT_DIR, "mm_fdw.o")
     probe_obj = os.path.join(OUT_DIR, "mm_probe.o")
     host_obj = os.path.join(OUT_DIR, "mm_host.o")
     serve_obj = os.path.join(OUT_DIR, "mm_serve.o")
@@ -71,6 +72,7 @@ def build(verbose=False, out=LIB, extra=()):
     _run_all([[HIPCC, *HIP_FLAGS, *extra, "-c", os.path.join(CSRC, "mm_hip.hip"), "-o", hip_obj],
               [HIPCC, *HIP_FLAGS, *extra, "-c", os.path.join(CSRC, "mm_mx.hip"), "-o", mx_obj],
               [HIPCC, *HIP_FLAGS, *extra, "-c", os.path.join(CSRC, "mm_fd.hip"), "-o", fd_obj],
+              [HIPCC, *HIP_FLAGS, *extra, "-c", os.path.join(CSRC, "mm_fdw.hip"), "-o", fdw_obj],
               [HIPCC, *HIP_FLAGS, *extra, "-c", os.path.join(CSRC, "mm_probe.hip"), "-o", probe_obj]] +
              [[HIPCC, *HIP_FLAGS, *extra, f"-DMM_MIX_NT={nt}", "-c", os.path.join(CSRC, "mm_mix.hip"), "-o", o]
               for nt, o in zip((512, 1024), mix_objs)] +
@@ -81,7 +83,7 @@ def build(verbose=False, out=LIB, extra=()):
               ["g++", "-O2", "-std=c++17", "-fPIC", "-Wall", "-pthread", f"-I{GMP_INCLUDE}", "-c",
                os.path.join(CSRC, "mm_multi.cpp"), "-o", multi_obj]], verbose)
     tmp = out + ".tmp"
-    _run([HIPCC, "-shared", f"--offload-arch={ARCH}", "-o", tmp, hip_obj, mx_obj, fd_obj, probe_obj, *mix_objs, host_obj, serve_obj, multi_obj,
+    _run([HIPCC, "-shared", f"--offload-arch={ARCH}", "-o", tmp, hip_obj, mx_obj, fd_obj, fdw_obj, probe_obj, *mix_objs, host_obj, serve_obj, multi_obj,
           GMP_LIB, "-pthread"], verbose)
     os.replace(tmp, out)
     return out

@@ -517,14 +517,46 @@ __device__ inline void add_small(u32* w, u32 k, i64 v) {
 }
 // Sign of the biased number of k words (multiples of 64): 1 below 0x8000..8000, 0 above, 2 there. One
 // whole wave; its first 64 words from the top almost always tell.
-__device__ inline u32 sign_of(const u32* w, u32 k) {
+template <u32 BIASED = SGN> __device__ inline u32 sign_of(const u32* w, u32 k) {
     const u32 lane = threadIdx.x & 63;
     for (u32 q = k; q != 0; q -= 64) {
         const u32 v = w[q - 64 + lane];
-        const u64 lt = __ballot(v < SGN), gt = __ballot(v > SGN);
+        const u64 lt = __ballot(v < BIASED), gt = __ballot(v > BIASED);
         if (lt | gt) return lt > gt;
     }
     return 2;
+}
+
+// x from the K words w (biased, carried; `top` stands above them), its flag in the first wave's ex, and the
+// overflow check: nonzero in some thread of the NT. Tl: T's biased halves, et what stands above them.
+template <u32 BIASED, u32 NT>
+__device__ __forceinline__ u32 fix_number(u32* w, u32 K, u32 top, u32 et, const u32* Tl, u32* flag, u32& ex) {
+    u32 bad = 0;
+    const u32 t = tid();
+    if (t < 64) {
+        if (t == 0) add_small(w, K, -(i64)(int)top);
+        wsync();
+        // X'' = words - bias is x, or x - (R + 1) where x > R / 2. A top word of zero leaves that open
+        // only if T / R is in the upper half itself (its top word is read then: x below R / 2
+        // is short of its bucket and has zeros there in every step).
+        u32 neg = w[K - 1] < BIASED;
+        if (w[K - 1] == BIASED && (et || Tl[2 * K - 1] - BIASED >= 0x40000000u)) neg = sign_of<BIASED>(w, K) & 1;
+        ex = neg;
+        if (neg) {
+            if (t == 0) add_small(w, K, 1);
+            wsync();
+            if (sign_of<BIASED>(w, K) == 2) bad = 1;  // x = R stands as digits 0 and ex = 1
+        }
+        if (t == 0) flag[1] = neg;
+    }
+    __syncthreads();
+    // x is T / R + m N / R (within 1) with m N / R < N, or that less R + 1 if it passed R: the
+    // top limbs tell.
+    if (t == NT - 1) {
+        const i64 d = (i64)w[K - 1] - (i64)Tl[2 * K - 1] + ((i64)flag[1] << 32) - ((i64)et << 32);
+        bad |= d < -4;
+    }
+    return bad;
 }
 
 // ---- The step -----------------------------------------------------------------------------------
@@ -652,35 +684,8 @@ template <u32 LOGC> struct Slot {
         return top - (u32)BETA + up;
     }
 
-    // x from the words (biased, carried; `top` stands above them) and the overflow check, for K limbs.
     __device__ __forceinline__ u32 fix_x(u32 K, u32 top, u32 et, const u32* Tl) {
-        u32 bad = 0;
-        const u32 t = tid();
-        if (t < 64) {
-            u32* w = words();
-            if (t == 0) add_small(w, K, -(i64)(int)top);
-            wsync();
-            // X'' = words - bias is x, or x - (R + 1) where x > R / 2. A top word of zero leaves that open
-            // only if T / R is in the upper half itself (its top word is read then: x below R / 2
-            // is short of its bucket and has zeros there in every step).
-            u32 neg = w[K - 1] < SGN;
-            if (w[K - 1] == SGN && (et || Tl[2 * K - 1] - SGN >= 0x40000000u)) neg = sign_of(w, K) & 1;
-            ex = neg;
-            if (neg) {
-                if (t == 0) add_small(w, K, 1);
-                wsync();
-                if (sign_of(w, K) == 2) bad = 1;  // x = R stands as digits 0 and ex = 1
-            }
-            if (t == 0) flag[1] = neg;
-        }
-        __syncthreads();
-        // x is T / R + m N / R (within 1) with m N / R < N, or that less R + 1 if it passed R: the
-        // top limbs tell.
-        if (t == T - 1) {
-            const i64 d = (i64)words()[K - 1] - (i64)Tl[2 * K - 1] + ((i64)flag[1] << 32) - ((i64)et << 32);
-            bad |= d < -4;
-        }
-        return bad;
+        return fix_number<SGN, T>(words(), K, top, et, Tl, flag, ex);
     }
 
     // One step on the words; returns nonzero (in some thread) on a carry that must vanish but does not.
@@ -1262,6 +1267,8 @@ __device__ __forceinline__ void constants_split(const Args& A, const u32* npl, c
 // Host side (mm_fd.hip).
 // Whether a batch of k limbs and base c can run on this path.
 bool fits(u32 k, u32 base);
+// exp(2 pi i num / den), den a power of two >= 8.
+double2 unit(u64 num, u64 den);
 // The tables of complex length C, back to back: 7 C/16, C/16, C/256, and for the split length 2C
 // C/2 and 32 elements.
 void make_tables(u32 C, double2* out);

@@ -63,22 +63,23 @@ __global__ __launch_bounds__(LOGC == 15 ? 1024 : Geo<LOGC == 15 ? 14 : LOGC>::T)
 // k = 1,024 .. 16,384 limbs; c C < 2^17 keeps the limb sums of T below BETA (2^32 - 1).
 bool fits(u32 k, u32 base) { return k >= 1024 && k <= 16384 && (k & (k - 1)) == 0 && (u64)base * 2 * k < 131072; }
 
+double2 unit(u64 num, u64 den) {
+    // The octant's sine and cosine, so that both are rounded from small angles.
+    num %= den;
+    const u64 q = num / (den / 4), r = num % (den / 4);
+    const bool flip = r > den / 8;
+    const long double a = 2 * 3.14159265358979323846264338327950288L * (long double)(flip ? den / 4 - r : r) / (long double)den;
+    double c = (double)cosl(a), s = (double)sinl(a);
+    if (flip) std::swap(c, s);
+    switch (q) {
+        case 0: return make_double2(c, s);
+        case 1: return make_double2(-s, c);
+        case 2: return make_double2(-c, -s);
+        default: return make_double2(s, -c);
+    }
+}
+
 void make_tables(u32 C, double2* out) {
-    auto unit = [](u64 num, u64 den) {  // exp(2 pi i num / den), den a power of two >= 8
-        // The octant's sine and cosine, so that both are rounded from small angles.
-        num %= den;
-        const u64 q = num / (den / 4), r = num % (den / 4);
-        const bool flip = r > den / 8;
-        const long double a = 2 * 3.14159265358979323846264338327950288L * (long double)(flip ? den / 4 - r : r) / (long double)den;
-        double c = (double)cosl(a), s = (double)sinl(a);
-        if (flip) std::swap(c, s);
-        switch (q) {
-            case 0: return make_double2(c, s);
-            case 1: return make_double2(-s, c);
-            case 2: return make_double2(-c, -s);
-            default: return make_double2(s, -c);
-        }
-    };
     const u32 T = C / 16, S1 = C / 256, S2 = C / 4096;
     for (u32 a = 0; a < 4; a++)
         for (u32 t = 0; t < T; t++) out[a * T + t] = unit((u64)t * (16 * a + 1), 4ull * C);

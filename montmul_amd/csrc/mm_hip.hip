@@ -23,6 +23,7 @@
 
 #include "../../include/montmul_hip.h"
 #include "mm_fd.h"
+#include "mm_fdw.h"
 #include "mm_mx.h"
 #include "mm_slot_steps.h"
 
@@ -618,8 +619,9 @@ int get_fd_tables(Ctx* C, uint32_t len, std::shared_ptr<FdTables>* out) {
     if (it != C->fd_tabs.end()) { *out = it->second; return 0; }
     auto D = std::make_shared<FdTables>();
     D->device = C->device;
-    std::vector<double2> h(fd::table_elems(len));
-    fd::make_tables(len, h.data());
+    const bool wide = len == 4 * fdw::K;  // the length in several workgroups: its parts' tables
+    std::vector<double2> h(wide ? fdw::TABLE : fd::table_elems(len));
+    wide ? fdw::make_tables(h.data()) : fd::make_tables(len, h.data());
     HIPCHK(hipMalloc((void**)&D->p, h.size() * sizeof(double2)));
     HIPCHK(hipMemcpy(D->p, h.data(), h.size() * sizeof(double2), hipMemcpyHostToDevice));
     C->fd_tabs[len] = D;
@@ -647,6 +649,9 @@ struct State {
     uint32_t* d_nl = nullptr;
     // The double-precision step (mm_fd.h) runs them; the spectra of N' and N.
     bool fd = false;
+    // Or the one that spreads a slot over several workgroups (mm_fdw.h), with its scratch.
+    bool wide = false;
+    unsigned char* d_wide = nullptr;
     std::shared_ptr<FdTables> fd_tab;
     double2 *d_fnp = nullptr, *d_fn = nullptr;
     double2* d_spec = nullptr;  // mul: its scratch (the spectrum of one factor, and T)
@@ -697,7 +702,7 @@ struct State {
                         (void*)d_nphat1, (void*)d_nhat1, (void*)d_work1, (void*)d_nphat2, (void*)d_nhat2, (void*)d_work2,
                         (void*)d_iwc1, (void*)d_iwc2, (void*)d_stage_lim, (void*)d_stage1, (void*)d_stage2, (void*)d_coef,
                         (void*)d_ones, (void*)d_ones_list, (void*)d_ones_out, (void*)d_nl,
-                        (void*)d_fnp, (void*)d_fn, (void*)d_spec, (void*)d_mul, (void*)d_plain})
+                        (void*)d_fnp, (void*)d_fn, (void*)d_spec, (void*)d_mul, (void*)d_plain, (void*)d_wide})
             if (p) hipFree(p);
     }
     // The device's x of a slot, or of all, is another than the host's copies.
@@ -747,6 +752,26 @@ struct State {
         A.base = base;
         return A;
     }
+    fdw::Args fdw_args() const {
+        fdw::Args A{};
+        A.w = fd::tables_at(fd_tab->p, fdw::H);
+        A.tw = fd_tab->p + fdw::TABLE - fdw::WEIGHTS;
+        A.x = d_x;
+        A.np = d_fnp;
+        A.n = d_fn;
+        A.exp = d_exp; A.nbits = d_nbits; A.pos = d_pos; A.err = d_err;
+        A.lim = d_lim;
+        const size_t group = std::min(slots, fdw::GROUP);
+        A.part = (double2*)d_wide;
+        A.sum = (int64_t*)(A.part + group * 8 * fdw::H);
+        A.dig = (uint32_t*)(A.sum + group * 2 * fdw::K);
+        A.fl = A.dig + group * fdw::K;
+        A.ew = ew ? ew : 1;
+        A.base = base;
+        return A;
+    }
+    // A kernel of its own steps this batch, not a transform kernel.
+    bool direct(bool bare) const { return mx || fd || (wide && !bare); }
     // The step kernel's arguments: args() plus the radix-4 kernel's LDS tile in global mode.
     KArgs step_args() const {
         KArgs A = args();
@@ -867,6 +892,7 @@ int set_lds_limit(Ctx* C) {
         C->max_dyn_lds_v2 = std::min(C->max_dyn_lds_v2 ? C->max_dyn_lds_v2 : dyn, dyn);
     }
     HIPCHK(fd::set_lds_limit());
+    HIPCHK(fdw::set_lds_limit());
     HIPCHK(mix_lds_limit<512>(C->max_lds, &C->max_dyn_lds_mix[0]));
     HIPCHK(mix_lds_limit<1024>(C->max_lds, &C->max_dyn_lds_mix[1]));
     C->max_dyn_lds = dyn_max;
@@ -1025,7 +1051,9 @@ template <class Launch> int run_chunks(Ctx* C, uint64_t reps, Launch&& launch, f
 
 // Up to `s` steps of one batch by the kernel that steps it alone (matrix-core or double-precision).
 hipError_t launch_direct(State* S, uint32_t s, bool bare, hipStream_t sm) {
-    return S->mx ? mx::launch(S->mx_args(bare), S->k, S->slots, s, bare, sm) : fd::launch(S->fd_args(), S->k, S->slots, s, bare, sm);
+    if (S->mx) return mx::launch(S->mx_args(bare), S->k, S->slots, s, bare, sm);
+    if (S->wide) return fdw::launch(S->fdw_args(), S->slots, s, sm);
+    return fd::launch(S->fd_args(), S->k, S->slots, s, bare, sm);
 }
 
 // Runs up to `bits` steps on every slot with bits left (reference: Gpu::steps, gpu/mod.rs:113-158).
@@ -1066,7 +1094,7 @@ int64_t steps(State* S, uint64_t bits, bool bare) {
         float ms = 0;
         if (run_chunks(C, reps,
                        [&]() {
-                           if (S->mx || S->fd) return launch_direct(S, (uint32_t)s, bare, C->stream);
+                           if (S->direct(bare)) return launch_direct(S, (uint32_t)s, bare, C->stream);
                            if (kern2)
                                hipLaunchKernelGGL(kern2, dim3(S->slots), dim3(S->threads), S->lds, C->stream, A2, 0u, (uint32_t)s);
                            else
@@ -1312,9 +1340,9 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
     std::vector<size_t> queued, direct;  // through the mixed-length kernel, by their own kernels
     for (size_t g = 0; g < count; g++) {
         const State* S = G[g];
-        (S->mx || S->fd ? direct : queued).push_back(g);
+        (S->direct(false) ? direct : queued).push_back(g);
         for (uint32_t i = 0; i < S->slots; i++) most = std::max<uint64_t>(most, S->nbits[i] - S->pos[i]);
-        if (!S->mx && !S->fd && S->v2 && S->n <= 8192 && S->n / 8 > nt) nt = S->n / 8;
+        if (!S->direct(false) && S->v2 && S->n <= 8192 && S->n / 8 > nt) nt = S->n / 8;
         G[g]->last_ms = 0;
         G[g]->last_launches = 0;
         G[g]->failed.clear();
@@ -1378,7 +1406,7 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
             const State* S = G[g];
             uint64_t r = 0;
             for (uint32_t i = 0; i < S->slots; i++) r = std::max<uint64_t>(r, S->nbits[i] - S->pos[i]);
-            const double per_cu = S->mx ? std::min(32.0, 4096.0 / S->k) : std::max(1.0, 8192.0 / S->k);
+            const double per_cu = S->mx ? std::min(32.0, 4096.0 / S->k) : S->wide ? 0.125 : std::max(1.0, 8192.0 / S->k);
             by_time.push_back({(double)std::min<uint64_t>(r, s) * S->k * std::max(1.0, S->slots / (per_cu * C->cus)), g});
         }
         std::stable_sort(by_time.begin(), by_time.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
@@ -1597,19 +1625,27 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
     // kernel, mode or tile of its own
     // (force_global at n >= 512 is the default plan). The first one's work grows as n^2: at L = 1,024 it
     // does 91 M squarings/s, where the second would do 75 M by its work; at 2,048 30 M against 36 M.
+    // At L = 65,536 a slot takes several workgroups: 148 K squarings/s at 64 slots against the radix-4
+    // kernel's 32 K, at 256 148 K against 86 K.
     const bool unnamed = wrap && !tune && !C->opts.prefer_lds && C->opts.tile == 0 && C->opts.slots_per_cu == 0 &&
                          (v2ok || (!C->opts.force_global && !(kenv && strcmp(kenv, "v1") == 0)));
     S->mx = unnamed && mx::fits(k, st->base);
     S->fd = unnamed && !S->mx && S->global && fd::fits(k, st->base);  // T goes through HBM
+    S->wide = unnamed && !S->mx && !S->fd && S->global && fdw::fits(k, st->base);
     // Device memory: x, N'-hat, N-hat or A|B, work vectors and limbs in global mode, exponents
     // of up to k words, per-slot words, the two raw values of 1 with a list word and a flag,
     // tables (about 6n elements per field, twice), a margin.
     const uint64_t per_slot = 4ull * k + 48ull * n + (S->global || tune ? 24ull * n + 12ull * k : 0) + 16 + 4ull * k +
-                              (v2ok && n > 8192 ? 24ull * n : 0) + 8ull * k + 8 + (S->mx ? 8ull * k : 0) + (S->fd ? 48ull * n : 0);
+                              (v2ok && n > 8192 ? 24ull * n : 0) + 8ull * k + 8;
     const uint64_t need = (uint64_t)st->slots * per_slot + 300ull * n + 48ull * n * 2 + (64ull << 20);
+    // What the step kernels' own constants and scratch take; a batch that fits only without them
+    // is stepped by its transform plan.
+    const uint64_t own = st->slots * (S->mx ? 8ull * k : S->fd ? 48ull * n + 4ull * k : S->wide ? 100ull * n : 0) +
+                         (S->wide ? std::min(st->slots, fdw::GROUP) * fdw::SCRATCH : 0);
     size_t freeb = 0, total = 0;
     if (hipMemGetInfo(&freeb, &total) != hipSuccess) return fail("hipMemGetInfo failed");
     if (need > freeb) return fail("batch needs " + std::to_string(need) + " bytes, " + std::to_string(freeb) + " free");
+    if (need + own > freeb) S->mx = S->fd = S->wide = false;
     if (get_tables(C, n, &S->tab)) return 1;
     if (wrap && get_tables(C, n / 2, &S->half)) return 1;
     const size_t sl = st->slots;
@@ -1625,6 +1661,9 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
         return 1;
     if (S->mx && dalloc(&S->d_nl, sl * 2 * k)) return 1;
     if (S->fd && (get_fd_tables(C, fd::length(k), &S->fd_tab) || dalloc(&S->d_fnp, sl * st->len) || dalloc(&S->d_fn, sl * (st->len / 2)) || dalloc(&S->d_spec, fd::mul_elems(k))))
+        return 1;
+    if (S->wide && (get_fd_tables(C, 4 * k, &S->fd_tab) || dalloc(&S->d_fnp, sl * 8 * fdw::H) || dalloc(&S->d_fn, sl * 4 * fdw::H) ||
+                    dalloc(&S->d_wide, std::min<size_t>(sl, fdw::GROUP) * fdw::SCRATCH)))
         return 1;
     if (v2ok) {
         if (dalloc(&S->d_iwc1, n) || dalloc(&S->d_iwc2, n)) return 1;
@@ -1642,15 +1681,16 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
     // Constants: N'-hat by a weighted forward transform; A|B (or N-hat) from N.
     {
         uint32_t* limbs = S->d_nl;
-        if (!S->mx && dalloc(&limbs, sl * k * (S->fd ? 2 : 1))) return 1;
+        if (!S->mx && dalloc(&limbs, sl * k * (S->fd || S->wide ? 2 : 1))) return 1;
         std::unique_ptr<uint32_t, void (*)(uint32_t*)> guard(S->mx ? nullptr : limbs, [](uint32_t* p) { hipFree(p); });
         const uint32_t tt = plan_threads(n);
         HIPCHK(hipMemcpyAsync(limbs, st->nprime, sl * k * 4, hipMemcpyHostToDevice, sm));
         hipLaunchKernelGGL(k_load_forward, dim3(st->slots), dim3(tt), 0, sm, S->tab->t, limbs, k, S->d_nphat1, S->d_nphat2);
         HIPCHK(hipGetLastError());
-        if (S->mx || S->fd) limbs += sl * k;  // N' stays
+        if (S->direct(false)) limbs += sl * k;  // N' stays
         HIPCHK(hipMemcpyAsync(limbs, st->n, sl * k * 4, hipMemcpyHostToDevice, sm));
         if (S->fd) HIPCHK(fd::launch_constants(S->fd_args(), k, st->slots, limbs - sl * k, limbs, S->d_fnp, S->d_fn, sm));
+        if (S->wide) HIPCHK(fdw::launch_constants(S->fdw_args(), st->slots, limbs - sl * k, limbs, sm));
         if (wrap) {
             const uint32_t h = n / 2;
             F1 c1 = cinv(F1{mod1(8 * h), 0});
@@ -1738,6 +1778,11 @@ int mm_set_modulus(void* st, size_t i, const uint32_t* nl, const uint32_t* npl, 
         HIPCHK(hipMemcpyAsync(S->d_nl + ((size_t)S->slots + i) * k, lim + k, 4ull * k, hipMemcpyDeviceToDevice, sm));
     }
     if (S->fd) HIPCHK(fd::launch_constants(S->fd_args(), k, 1, lim, lim + k, S->d_fnp + i * S->len, S->d_fn + i * (S->len / 2), sm));
+    if (S->wide) {
+        fdw::Args A = S->fdw_args();
+        A.first = (uint32_t)i;
+        HIPCHK(fdw::launch_constants(A, 1, lim, lim + k, sm));
+    }
     const uint32_t tt = plan_threads(n);
     hipLaunchKernelGGL(k_load_forward, dim3(1), dim3(tt), 0, sm, S->tab->t, lim, k, S->d_nphat1 + i * n, S->d_nphat2 + i * n);
     HIPCHK(hipGetLastError());
@@ -2014,7 +2059,7 @@ int mm_plan(void* st, mm_plan_info* out) {
 
 int mm_step_kernel(void* st) {
     const State* S = (const State*)st;
-    return S->mx ? 32 : S->fd ? 64 : S->v2 ? 8 : 4;
+    return S->mx ? 32 : S->fd || S->wide ? 64 : S->v2 ? 8 : 4;
 }
 
 uint64_t mm_free_memory(void* self) {
