@@ -181,10 +181,10 @@ int64_t mm_run_bare(void *state, uint64_t bits);
 int mm_push(void *state);
 /* Gpu::plan_of (gpu/mod.rs:102-104). */
 int mm_plan(void *state, mm_plan_info *out);
-/* The kernel that mm_run and mm_run_bare step this batch with: 32 = matrix cores, 64 =
- * double-precision transforms (mm_options names no transform plan, and the length and base fit
- * them); else mm_plan's kernel, 4 or 8. mm_plan describes the modular transform kernels, which run
- * the mixed launch in every case. No reference counterpart. */
+/* The kernel that mm_run steps this batch with: 32 = matrix cores, 64 = double-precision transforms
+ * (mm_options names no transform plan, the length and base fit them, and their constants the
+ * memory); else mm_plan's kernel, 4 or 8. mm_run_bare uses it too, but at L = 65,536 mm_plan's.
+ * No reference counterpart. */
 int mm_step_kernel(void* state);
 /* Gpu::free_memory, sm_count, max_dyn_smem, device_name (gpu/mod.rs:83-99). */
 uint64_t mm_free_memory(void *self);
@@ -436,8 +436,9 @@ typedef struct mm_server_stats {
 
 /* Device memory of one pool slot at transform length L in the server's accounting: on the HIP
  * backend in global mode, x and the exponent (k words each), N'-hat and A|B (24 L bytes), the
- * work vectors (12 L) and the limb staging (6 L), with k = L/2: 46 L + 16 bytes, plus 12 L at
- * L = 32,768 for the coefficient staging of its register-transform step. */
+ * work vectors (12 L), the limb staging (6 L) and the two values of 1 (4 L), with k = L/2: 50 L + 24
+ * bytes, plus 12 L at L = 32,768 for the coefficient staging of its register-transform step, plus the
+ * step kernels' constants: 4 L at L = 16 .. 1,024, 24 L at 2,048 .. 32,768, 94 L + 8 at 65,536. */
 uint64_t mm_server_slot_bytes(uint32_t len);
 
 int mm_server_new(const mm_server_options *opts, mm_open_fn open, mm_close_fn close, void *user, mm_server **out);

@@ -365,8 +365,13 @@ void hip_close(void* user, mm_backend* be) {
 
 extern "C" {
 
-// At L = 32,768 the register-transform step also stages its coefficients in HBM (24 n = 12 L).
-uint64_t mm_server_slot_bytes(uint32_t len) { return 50ull * len + 24 + (len == 32768 ? 12ull * len : 0); }
+// At L = 32,768 the register-transform step also stages its coefficients in HBM (24 n = 12 L). The step
+// kernels' own constants: the limbs of N' and N (4 L) on the matrix cores, their spectra (24 L) in double
+// precision, at L = 65,536 50 L and the scratch of a slot that runs (44 L and 8).
+uint64_t mm_server_slot_bytes(uint32_t len) {
+    const uint64_t own = len < 16 ? 0 : len <= 1024 ? 4ull * len : len <= 32768 ? 24ull * len : len == 65536 ? 94ull * len + 8 : 0;
+    return 50ull * len + 24 + (len == 32768 ? 12ull * len : 0) + own;
+}
 
 int mm_server_new(const mm_server_options* o, mm_open_fn open, mm_close_fn close, void* user, mm_server** out) {
     *out = nullptr;
