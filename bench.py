@@ -10,8 +10,9 @@ run(2,000), so every step-kernel launch of a run with a fixed slot count does th
 
 The slot count is the best of 256 x {1, 2, 4, 8, 16} (CUs x {1, 2, 4, 8, 16}, as the
 reference's candidates, main.rs:199-216) at 200-bit exponents, unless --slots is given. The
-headline is global mode (transform vectors in HBM, as the workload specifies); LDS mode
-(vectors resident in LDS) is measured and reported beside it. Slot 0, the last slot and two
+headline is global mode (T and the constants in HBM, as the workload specifies; the default, the
+double-precision step); LDS mode (the modular transforms' vectors resident in LDS) is measured and
+reported beside it. Slot 0, the last slot and two
 seeded random slots must equal 3^e mod N (GMP powm) or no number is reported
 (score.rs:105-115); after the timed passes every headline slot is checked the same way, on
 the host's threads (--no-check-all skips it).
@@ -32,20 +33,18 @@ sys.path.insert(0, ROOT)
 
 METRIC = "squarings/s at 100k-bit, 1 MI355X"
 HBM_PEAK = 8.0e12          # MI355X HBM3E, bytes/s
-# Attainable VALU issue of the step kernel's own instruction mix, in wave instructions per CU
-# per cycle: the issue rates measured by mm_probe_issue (32-bit operations 1.37, 64-bit 0.95)
-# weighted by the kernel's INT32 / INT64 / other counts (profiles/valu_issue_probe.md), over
-# 256 CUs at 2.4 GHz.
-VALU_MIX_PER_CU_CYCLE = {8192: 1.22}
-VALU_PROBE = "profiles/valu_issue_probe.md"
-# Per slot-step of the global-mode step kernel, by transform length L, from the rocprofv3 summary
+# VALU issue bound of the double-precision step, in wave instructions per CU per cycle: each of the
+# four SIMDs takes four cycles for a wave's double-precision instruction. Over 256 CUs at 2.4 GHz.
+VALU_PER_CU_CYCLE = 1.0
+# Per slot-step of the double-precision step kernel, by transform length L, from the rocprofv3 summary
 # named in PROFILE: HBM bytes moved (FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000, scales from a
 # 1 GiB device copy in the same run) and VALU wave instructions (SQ_INSTS_VALU). Counters cannot
 # be read from inside this process; the summaries are re-measured whenever the kernel changes.
-PROFILE = {8192: "profiles/k_steps_v2_global_100kbit_4096slots.md",
-           32768: "profiles/k_steps_v2_split_300kbit_1024slots.md"}
-TRAFFIC_PER_SLOT_STEP = {8192: 324_955, 32768: 9_757_633}
-VALU_PER_SLOT_STEP = {8192: 170_223, 32768: 832_892}
+PROFILE = {8192: "profiles/k_steps_fd_100kbit_4096slots.md",
+           32768: "profiles/k_steps_fd_100kbit_4096slots.md"}
+TRAFFIC_PER_SLOT_STEP = {8192: 261_363, 32768: 3_550_055}
+VALU_PER_SLOT_STEP = {8192: 43_132, 32768: 233_944}
+KERNELS = {4: "k_steps (radix-4)", 8: "k_steps_v2", 32: "k_steps_mx (matrix cores)", 64: "k_steps_fd (double precision)"}
 REF_5090 = 1_536_441.0     # reference, RTX 5090, 170 slots (README.md:14)
 
 
@@ -155,15 +154,13 @@ def cpu_baseline(bits, threads, gmp_steps=8_000, ntt_steps=1_000, single_steps=2
 
 def valu_roof(L, slot_steps_per_s):
     """The kernel's VALU issue rate (instructions per slot-step from the profile, rate from this
-    run's kernel time) against the rate its instruction mix can issue, where measured."""
+    run's kernel time) against the rate the SIMDs can issue."""
     achieved = VALU_PER_SLOT_STEP[L] * slot_steps_per_s
-    out = {"bound": "valu", "achieved": round(achieved / 1e9, 2), "unit": "G wave-instr/s",
-           "instr_per_slot_step": VALU_PER_SLOT_STEP[L], "source": PROFILE[L],
-           "per_cu_per_cycle_at_2.4GHz": round(achieved / (256 * 2.4e9), 4)}
-    if L in VALU_MIX_PER_CU_CYCLE:
-        peak = VALU_MIX_PER_CU_CYCLE[L] * 256 * 2.4e9
-        out.update(peak=round(peak / 1e9, 1), frac=round(achieved / peak, 4), peak_source=VALU_PROBE)
-    return out
+    peak = VALU_PER_CU_CYCLE * 256 * 2.4e9
+    return {"bound": "valu", "achieved": round(achieved / 1e9, 2), "unit": "G wave-instr/s",
+            "instr_per_slot_step": VALU_PER_SLOT_STEP[L], "source": PROFILE[L],
+            "per_cu_per_cycle_at_2.4GHz": round(achieved / (256 * 2.4e9), 4),
+            "peak": round(peak / 1e9, 1), "frac": round(achieved / peak, 4)}
 
 
 def host_threads():
@@ -259,7 +256,7 @@ def main():
         overhead = statistics.mean(kms) / (bare_ms / max(1, bare_launches))
         results[mode] = dict(slots=best, rates=rates, secs=secs, kernel_ms=kms, plan=plan, L=L, k=k, ups=ups,
                              sweep={str(s): round(r) for s, r in sw.items()}, checked=picked, overhead=overhead,
-                             all_slots=all_slots)
+                             all_slots=all_slots, kernel=mm.Hip.step_kernel(b))
         log(f"mode {mode}: median {median(rates):.4g} sq/s, kernel {statistics.mean(kms):.1f} ms/launch")
         b.free()
         hip.close()
@@ -269,9 +266,13 @@ def main():
     total = slots * ebits * len(head["secs"])
     value = total / sum(head["secs"])
     kms = statistics.mean(head["kernel_ms"])
-    # Algorithmic HBM bytes per slot-step in global mode: the per-slot constant spectra N'-hat
-    # and A|B (12 L bytes each, read once per step) plus x read and written (2 L each): 28 L.
-    alg_bytes = 28 * L * slots * ebits
+    # Algorithmic HBM bytes per slot-step of the double-precision step: the per-slot constant spectra
+    # of N' and N (16 L and 8 L bytes, read once per step); x stays in LDS through a launch. The
+    # matrix-core step keeps its constants there too. The transform kernels: their spectra N'-hat and
+    # A|B (12 L bytes each) plus x read and written (2 L each), 28 L.
+    profiled = head["kernel"] == 64 and L in VALU_PER_SLOT_STEP
+    alg_per_step = {64: 24 * L, 32: 0}.get(head["kernel"], 28 * L)
+    alg_bytes = alg_per_step * slots * ebits
     achieved = alg_bytes / (kms * 1e-3)
     line = {
         "metric": METRIC,
@@ -288,12 +289,12 @@ def main():
         "dtype": "u32",
         "data": "synthetic (GMP generator seeded 2026, as the reference's score workload)",
         "config": {"workload": f"{args.bits:,}-bit moduli, L={L}, k={head['k']}, base 3, top {ebits:,} bits of N-1, " +
-                               ("global mode (T, x and constants in HBM; transform exchanges through LDS tiles)"
+                               ("global mode (T and constants in HBM; transform exchanges through LDS)"
                                 if "global" in results else f"{modes[0]} mode"),
                    "bits": args.bits, "L": L, "k": head["k"], "slots": slots, "ebits": ebits,
                    "mode": "global" if "global" in results else modes[0],
-                   "threads_per_wg": head["plan"]["threads"], "lds_bytes": head["plan"]["lds_bytes"],
-                   "tile": head["plan"]["tile"]},
+                   "step_kernel": KERNELS[head["kernel"]],
+                   "transform_plan": {k: head["plan"][k] for k in ("threads", "lds_bytes", "tile")}},
         # The same passes with the upload of x and the exponents (host to device) inside the
         # clock, as the reference's score times run() (score.rs:98-102).
         "value_incl_upload": round(total / (sum(head["secs"]) + sum(head["ups"])), 1),
@@ -305,15 +306,16 @@ def main():
         "fermat_tests_per_hour": round(value * 3600 / args.bits, 1),
         "roofline": {"bound": "hbm", "achieved": round(achieved / 1e9, 2), "peak": HBM_PEAK / 1e9,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK, 5),
-                     "traffic": (TRAFFIC_PER_SLOT_STEP[L] * slots * ebits) if L in TRAFFIC_PER_SLOT_STEP else None,
-                     "traffic_per_slot_step": TRAFFIC_PER_SLOT_STEP.get(L), "traffic_source": PROFILE.get(L),
-                     "kernel": "k_steps_v2 (global mode)", "kernel_ms_per_launch": round(kms, 3),
-                     "alg_bytes_per_slot_step": 28 * L},
+                     "traffic": (TRAFFIC_PER_SLOT_STEP[L] * slots * ebits) if profiled else None,
+                     "traffic_per_slot_step": TRAFFIC_PER_SLOT_STEP[L] if profiled else None,
+                     "traffic_source": PROFILE[L] if profiled else None,
+                     "kernel": KERNELS[head["kernel"]], "kernel_ms_per_launch": round(kms, 3),
+                     "alg_bytes_per_slot_step": alg_per_step},
         "checked_slots": head["checked"],
         "checked_all_slots": head.get("all_slots"),
-        # The bound that binds: VALU issue (integer work, no MFMA). Instructions per slot-step
-        # from the profile, rate from this run's kernel time.
-        "valu": (valu_roof(L, slots * ebits / (kms * 1e-3)) if L in VALU_PER_SLOT_STEP else None),
+        # The bound that binds: VALU issue (double-precision transforms, no MFMA). Instructions per
+        # slot-step from the profile, rate from this run's kernel time.
+        "valu": (valu_roof(L, slots * ebits / (kms * 1e-3)) if profiled else None),
         "sweep": head["sweep"],
     }
     if "lds" in results and "global" in results:

@@ -118,10 +118,12 @@ typedef struct mm_options {
     int32_t force_global;    /* keep transform vectors in HBM even when LDS would hold them */
     int32_t wraparound;      /* reduction through the half-length cyclic product; k = L/2 */
     uint32_t max_launch_ms;  /* target duration of one kernel launch; 0 = no splitting */
-    int32_t prefer_lds;      /* keep vectors in LDS whenever they fit (the reference planner's
-                              * rule, plan.rs:26-42); by default the register-transform kernel
-                              * (wraparound, L = 1,024 .. 8,192) runs in global mode, whose smaller
-                              * LDS footprint fits more workgroups per CU and is faster there */
+    int32_t prefer_lds;      /* step by the modular transforms, their vectors in LDS whenever they
+                              * fit (the reference planner's rule, plan.rs:26-42); by default batches
+                              * of L = 16 .. 65,536 are stepped on the matrix cores or in double
+                              * precision (mm_step_kernel), and mm_plan has the register-transform
+                              * kernel (L = 1,024 .. 8,192) in global mode, whose smaller LDS
+                              * footprint fits more workgroups per CU and is faster there */
     int32_t autotune;        /* time every plan that can run a new batch's length (radix-8
                               * register kernel or radix-4 kernel, global mode with LDS tiles or
                               * LDS-resident, the register kernel's exchange tile, one or as many
