@@ -1459,15 +1459,20 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
                                if ((fe = hipEventRecord(C->fork, sm)) != hipSuccess) break;
                                fe = hipStreamWaitEvent(C->side[l - 1], C->fork, 0);
                            }
-                           for (int l = 3; l >= 0 && fe == hipSuccess; l--)
-                               for (size_t i = 0; i < lane[l].size() && fe == hipSuccess; i++)
-                                   fe = launch_direct(G[lane[l][i]], (uint32_t)s, false, l ? C->side[l - 1] : sm);
+                           // The batches of many launches a step come last: the others run meanwhile.
+                           auto enqueue = [&](bool wide) {
+                               for (int l = 3; l >= 0 && fe == hipSuccess; l--)
+                                   for (size_t i = 0; i < lane[l].size() && fe == hipSuccess; i++)
+                                       if (G[lane[l][i]]->wide == wide) fe = launch_direct(G[lane[l][i]], (uint32_t)s, false, l ? C->side[l - 1] : sm);
+                           };
+                           enqueue(false);
                            if (fe == hipSuccess && !queue.empty()) {
                                hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, sm, head, 1u, 0u);
                                if ((fe = hipGetLastError()) == hipSuccess)
                                    fe = nt == 1024 ? mix_launch<1024>(grid, lds, sm, dcls, ditems, dlist, (uint32_t)queue.size(), head)
                                                    : mix_launch<512>(grid, lds, sm, dcls, ditems, dlist, (uint32_t)queue.size(), head);
                            }
+                           enqueue(true);
                            for (int l = 1; l < 4; l++) {  // join, also after an error: nothing runs on
                                if (lane[l].empty()) continue;
                                hipError_t je = hipEventRecord(C->join[l - 1], C->side[l - 1]);
