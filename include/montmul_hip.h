@@ -158,6 +158,13 @@ int mm_device_count(void);
 int mm_hip_open(const mm_options *opts, mm_backend *out);
 /* Releases what mm_hip_open allocated; every state created from it must be destroyed first. */
 void mm_hip_close(mm_backend *be);
+/* The most device memory that a batch created from now on may take beyond what its transform plan
+ * holds, for a step kernel of its own: at L = 65,536 its constants and scratch are 50 L bytes a slot and
+ * 42 L + 8 for each of up to 64 slots. A batch that would take more is stepped by its transform plan, as
+ * one is that the device's free memory would not hold otherwise. By default there is no limit; a
+ * server with a memory budget sets 0. Returns 1 when `be` is no Hip table. No reference
+ * counterpart. */
+int mm_hip_step_memory(mm_backend *be, uint64_t bytes);
 
 /* The table's functions, also callable directly with the `self`/state of a Hip table. */
 int mm_create(void *self, const mm_batch_setup *setup, void **state);    /* gpu/mod.rs:325-370 */
@@ -439,8 +446,9 @@ typedef struct mm_server_stats {
 /* Device memory of one pool slot at transform length L in the server's accounting: on the HIP
  * backend in global mode, x and the exponent (k words each), N'-hat and A|B (24 L bytes), the
  * work vectors (12 L), the limb staging (6 L) and the two values of 1 (4 L), with k = L/2: 50 L + 24
- * bytes, plus 12 L at L = 32,768 for the coefficient staging of its register-transform step, plus the
- * step kernels' constants: 4 L at L = 16 .. 1,024, 24 L at 2,048 .. 32,768, 94 L + 8 at 65,536. */
+ * bytes, plus 12 L at L = 32,768 for the coefficient staging of its register-transform step. The
+ * step kernels of L = 16 .. 32,768 hold less; the one of L = 65,536 would hold more, so that a server
+ * with a budget (hbm_bytes) leaves it out (mm_hip_step_memory). */
 uint64_t mm_server_slot_bytes(uint32_t len);
 
 int mm_server_new(const mm_server_options *opts, mm_open_fn open, mm_close_fn close, void *user, mm_server **out);

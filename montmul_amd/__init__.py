@@ -128,6 +128,7 @@ def _load_lib():
         "mm_push": (C.c_int, [vp]),
         "mm_plan": (C.c_int, [vp, C.POINTER(PlanInfo)]),
         "mm_step_kernel": (C.c_int, [vp]),
+        "mm_hip_step_memory": (C.c_int, [C.POINTER(BackendTable), C.c_uint64]),
         "mm_read_plain": (C.c_int, [vp, C.c_size_t, u32p]),
         "mm_free_memory": (C.c_uint64, [vp]),
         "mm_cu_count": (C.c_int, [vp]),
@@ -326,6 +327,12 @@ class Hip(Backend):
 
     def free_memory(self):
         return lib.mm_free_memory(self.table.self)
+
+    def limit_step_memory(self, nbytes):
+        """The most device memory that a batch created from now on may take beyond its transform
+        plan's, for a step kernel of its own (at L = 65,536; mm_hip_step_memory)."""
+        if lib.mm_hip_step_memory(C.byref(self.table), nbytes) != 0:
+            raise MontmulError((lib.mm_last_error() or b"").decode())
 
     def cu_count(self):
         return lib.mm_cu_count(self.table.self)

@@ -523,6 +523,7 @@ struct Ctx {
     std::mutex mu;
     std::map<uint32_t, std::shared_ptr<DevTables>> tabs;
     std::map<uint32_t, std::shared_ptr<FdTables>> fd_tabs;
+    uint64_t step_memory = UINT64_MAX;  // mm_hip_step_memory
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // This device's copy of the fixed product scratch (null, with scratch_err, if its address
     // could not be taken).
@@ -654,8 +655,9 @@ struct State {
     unsigned char* d_wide = nullptr;
     std::shared_ptr<FdTables> fd_tab;
     double2 *d_fnp = nullptr, *d_fn = nullptr;
-    double2* d_spec = nullptr;  // mul: its scratch (the spectrum of one factor, and T)
-    unsigned char* d_mul = nullptr;  // mul by the radix-4 kernel: its scratch, from the first one on
+    double2* d_part = nullptr;       // L = 32,768: the first part's result and the digits of the second
+    uint32_t* d_dig = nullptr;
+    unsigned char* d_mul = nullptr;  // mul's scratch, from the first one on
     uint32_t* d_coef = nullptr;  // n = 2^14 register step: coefficient staging, 6 n words per slot
     v2::S2* d_iwc2 = nullptr;
     // set_modulus staging (N' and N limbs, the half factors' work vectors), allocated on the
@@ -702,7 +704,7 @@ struct State {
                         (void*)d_nphat1, (void*)d_nhat1, (void*)d_work1, (void*)d_nphat2, (void*)d_nhat2, (void*)d_work2,
                         (void*)d_iwc1, (void*)d_iwc2, (void*)d_stage_lim, (void*)d_stage1, (void*)d_stage2, (void*)d_coef,
                         (void*)d_ones, (void*)d_ones_list, (void*)d_ones_out, (void*)d_nl,
-                        (void*)d_fnp, (void*)d_fn, (void*)d_spec, (void*)d_mul, (void*)d_plain, (void*)d_wide})
+                        (void*)d_fnp, (void*)d_fn, (void*)d_part, (void*)d_dig, (void*)d_mul, (void*)d_plain, (void*)d_wide})
             if (p) hipFree(p);
     }
     // The device's x of a slot, or of all, is another than the host's copies.
@@ -739,10 +741,8 @@ struct State {
     fd::Args fd_args() const {
         fd::Args A{};
         A.w = fd::tables_at(fd_tab->p, fd::length(k));
-        if (k == 16384) {  // the global mode's work vectors, which the register kernel's steps use
-            A.part = (double2*)d_work2;
-            A.dig = (uint32_t*)d_work1;
-        }
+        A.part = d_part;
+        A.dig = d_dig;
         A.x = d_x;
         A.np = d_fnp;
         A.n = d_fn;
@@ -772,6 +772,9 @@ struct State {
     }
     // A kernel of its own steps this batch, not a transform kernel.
     bool direct(bool bare) const { return mx || fd || (wide && !bare); }
+    // The transform kernels run on this batch too, and their constants and work vectors are held (the
+    // wide step leaves mul and run_bare to them).
+    bool transforms() const { return !mx && !fd; }
     // The step kernel's arguments: args() plus the radix-4 kernel's LDS tile in global mode.
     KArgs step_args() const {
         KArgs A = args();
@@ -1071,11 +1074,16 @@ int64_t steps(State* S, uint64_t bits, bool bare) {
     // Only run_bare leaves each step's product in HBM: a full step of the register kernel keeps
     // it on chip where it can.
     S->product_in_hbm = bare;
-    KArgs A = S->step_args();
-    StepKernel kern = pick_step(S->global, S->wrap, bare);
+    const bool direct = S->direct(bare);
+    KArgs A{};
+    StepKernel kern = nullptr;
     v2::VArgs A2{};
     StepKernelV2 kern2 = nullptr;
-    if (S->v2) {
+    if (!direct) {
+        A = S->step_args();
+        kern = pick_step(S->global, S->wrap, bare);
+    }
+    if (!direct && S->v2) {
         A2 = S->vargs();
         kern2 = pick_step_v2(ilog2(S->n), S->global, bare, S->tile);
     }
@@ -1094,7 +1102,7 @@ int64_t steps(State* S, uint64_t bits, bool bare) {
         float ms = 0;
         if (run_chunks(C, reps,
                        [&]() {
-                           if (S->direct(bare)) return launch_direct(S, (uint32_t)s, bare, C->stream);
+                           if (direct) return launch_direct(S, (uint32_t)s, bare, C->stream);
                            if (kern2)
                                hipLaunchKernelGGL(kern2, dim3(S->slots), dim3(S->threads), S->lds, C->stream, A2, 0u, (uint32_t)s);
                            else
@@ -1587,6 +1595,12 @@ void mm_hip_close(mm_backend* be) {
     be->self = nullptr;
 }
 
+int mm_hip_step_memory(mm_backend* be, uint64_t bytes) {
+    if (be->create != mm_create) return fail("not a HIP backend");
+    ((Ctx*)be->self)->step_memory = bytes;
+    return 0;
+}
+
 // Backend::create (reference: Gpu::create, gpu/mod.rs:325-370).
 int mm_create(void* self, const mm_batch_setup* st, void** out) {
     Ctx* C = (Ctx*)self;
@@ -1637,45 +1651,57 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
     S->mx = unnamed && mx::fits(k, st->base);
     S->fd = unnamed && !S->mx && S->global && fd::fits(k, st->base);  // T goes through HBM
     S->wide = unnamed && !S->mx && !S->fd && S->global && fdw::fits(k, st->base);
-    // Device memory: x, N'-hat, N-hat or A|B, work vectors and limbs in global mode, exponents
-    // of up to k words, per-slot words, the two raw values of 1 with a list word and a flag,
-    // tables (about 6n elements per field, twice), a margin.
-    const uint64_t per_slot = 4ull * k + 48ull * n + (S->global || tune ? 24ull * n + 12ull * k : 0) + 16 + 4ull * k +
-                              (v2ok && n > 8192 ? 24ull * n : 0) + 8ull * k + 8;
+    // Device memory. Of every slot: x, the exponent of up to k words, the words of its state, the two raw
+    // values of 1 with a list word and a flag. By the transform kernels: N'-hat, N-hat or A|B, work
+    // vectors and limbs in global mode. By the matrix-core step: the limbs of N' and N (and of T, for
+    // run_bare in global mode); by the double-precision step: their spectra, T, the constants' limbs
+    // while they are made, and at L = 32,768 its parts. These two take no more than the transform
+    // kernels, and hold nothing of theirs: those state 100 k bytes a slot here in global mode, where
+    // the matrix-core step holds 24 k or 36 k and the double-precision one 76 k (96 k at L = 32,768).
+    uint64_t per_slot = 16ull * k + 24;
+    if (S->mx)
+        per_slot += 8ull * k + (S->global ? 12ull * k : 0);
+    else if (S->fd)
+        per_slot += (12ull + 48 + 8) * k + (k == 16384 ? 20ull * k : 0);
+    else
+        per_slot += 48ull * n + (S->global || tune ? 24ull * n + 12ull * k : 0) + (v2ok && n > 8192 ? 24ull * n : 0);
+    // Tables (about 6n elements per field, twice) and a margin.
     const uint64_t need = (uint64_t)st->slots * per_slot + 300ull * n + 48ull * n * 2 + (64ull << 20);
-    // What the step kernels' own constants and scratch take; a batch that fits only without them
-    // is stepped by its transform plan.
-    const uint64_t own = st->slots * (S->mx ? 8ull * k : S->fd ? 48ull * n + 4ull * k : S->wide ? 100ull * n : 0) +
-                         (S->wide ? std::min(st->slots, fdw::GROUP) * fdw::SCRATCH : 0);
+    // What the step at L = 65,536 takes beyond its transform plan, which mul and run_bare use; a batch that
+    // fits only without it, by the device's memory or the context's limit, is stepped by that plan.
+    const uint64_t own = S->wide ? st->slots * 100ull * n + std::min(st->slots, fdw::GROUP) * fdw::SCRATCH : 0;
     size_t freeb = 0, total = 0;
     if (hipMemGetInfo(&freeb, &total) != hipSuccess) return fail("hipMemGetInfo failed");
     if (need > freeb) return fail("batch needs " + std::to_string(need) + " bytes, " + std::to_string(freeb) + " free");
-    if (need + own > freeb) S->mx = S->fd = S->wide = false;
-    if (get_tables(C, n, &S->tab)) return 1;
-    if (wrap && get_tables(C, n / 2, &S->half)) return 1;
+    if (own > C->step_memory || need + own > freeb) S->wide = false;
     const size_t sl = st->slots;
     if (dalloc(&S->d_ones, sl * 2 * k) || dalloc(&S->d_ones_list, sl) || dalloc(&S->d_ones_out, sl)) return 1;
     S->ones_set.assign(sl, 0);
-    if (dalloc(&S->d_x, sl * k) || dalloc(&S->d_nbits, sl) || dalloc(&S->d_pos, sl) || dalloc(&S->d_err, sl) ||
-        dalloc(&S->d_nphat1, sl * n) || dalloc(&S->d_nphat2, sl * n) || dalloc(&S->d_nhat1, sl * n) ||
-        dalloc(&S->d_nhat2, sl * n) || dalloc(&S->d_exp, sl))
+    if (dalloc(&S->d_x, sl * k) || dalloc(&S->d_nbits, sl) || dalloc(&S->d_pos, sl) || dalloc(&S->d_err, sl) || dalloc(&S->d_exp, sl))
         return 1;
     S->ew = 1;
     S->exp_cap = sl;
-    if ((S->global || tune) && (dalloc(&S->d_work1, sl * n) || dalloc(&S->d_work2, sl * n) || dalloc(&S->d_lim, sl * 3 * k)))
-        return 1;
+    if ((S->fd || S->global || tune) && dalloc(&S->d_lim, sl * 3 * k)) return 1;
     if (S->mx && dalloc(&S->d_nl, sl * 2 * k)) return 1;
-    if (S->fd && (get_fd_tables(C, fd::length(k), &S->fd_tab) || dalloc(&S->d_fnp, sl * st->len) || dalloc(&S->d_fn, sl * (st->len / 2)) || dalloc(&S->d_spec, fd::mul_elems(k))))
+    if (S->fd && (get_fd_tables(C, fd::length(k), &S->fd_tab) || dalloc(&S->d_fnp, sl * st->len) || dalloc(&S->d_fn, sl * (st->len / 2)) ||
+                  (k == 16384 && (dalloc(&S->d_part, sl * k) || dalloc(&S->d_dig, sl * k)))))
         return 1;
     if (S->wide && (get_fd_tables(C, 4 * k, &S->fd_tab) || dalloc(&S->d_fnp, sl * 8 * fdw::H) || dalloc(&S->d_fn, sl * 4 * fdw::H) ||
                     dalloc(&S->d_wide, std::min<size_t>(sl, fdw::GROUP) * fdw::SCRATCH)))
         return 1;
-    if (v2ok) {
-        if (dalloc(&S->d_iwc1, n) || dalloc(&S->d_iwc2, n)) return 1;
-        if (n > 8192 && dalloc(&S->d_coef, sl * 6 * n)) return 1;
-        hipLaunchKernelGGL(k_scale_tab, dim3((n + 255) / 256), dim3(256), 0, C->stream, S->tab->vt.iw1, S->tab->vt.iw2,
-                           st->base, n, S->d_iwc1, S->d_iwc2);
-        HIPCHK(hipGetLastError());
+    if (S->transforms()) {
+        if (get_tables(C, n, &S->tab)) return 1;
+        if (wrap && get_tables(C, n / 2, &S->half)) return 1;
+        if (dalloc(&S->d_nphat1, sl * n) || dalloc(&S->d_nphat2, sl * n) || dalloc(&S->d_nhat1, sl * n) || dalloc(&S->d_nhat2, sl * n))
+            return 1;
+        if ((S->global || tune) && (dalloc(&S->d_work1, sl * n) || dalloc(&S->d_work2, sl * n))) return 1;
+        if (v2ok) {
+            if (dalloc(&S->d_iwc1, n) || dalloc(&S->d_iwc2, n)) return 1;
+            if (n > 8192 && dalloc(&S->d_coef, sl * 6 * n)) return 1;
+            hipLaunchKernelGGL(k_scale_tab, dim3((n + 255) / 256), dim3(256), 0, C->stream, S->tab->vt.iw1, S->tab->vt.iw2,
+                               st->base, n, S->d_iwc1, S->d_iwc2);
+            HIPCHK(hipGetLastError());
+        }
     }
     hipStream_t sm = C->stream;
     HIPCHK(hipMemsetAsync(S->d_x, 0, sl * k * 4, sm));
@@ -1683,20 +1709,23 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
     HIPCHK(hipMemsetAsync(S->d_nbits, 0, sl * 4, sm));
     HIPCHK(hipMemsetAsync(S->d_pos, 0, sl * 4, sm));
     HIPCHK(hipMemsetAsync(S->d_exp, 0, sl * 4, sm));
-    // Constants: N'-hat by a weighted forward transform; A|B (or N-hat) from N.
+    // Constants: the limbs of N' and N on the matrix cores, their spectra in double precision; for the
+    // transform kernels N'-hat by a weighted forward transform, A|B (or N-hat) from N.
     {
         uint32_t* limbs = S->d_nl;
-        if (!S->mx && dalloc(&limbs, sl * k * (S->fd || S->wide ? 2 : 1))) return 1;
+        if (!S->mx && dalloc(&limbs, sl * k * (S->direct(false) ? 2 : 1))) return 1;
         std::unique_ptr<uint32_t, void (*)(uint32_t*)> guard(S->mx ? nullptr : limbs, [](uint32_t* p) { hipFree(p); });
         const uint32_t tt = plan_threads(n);
         HIPCHK(hipMemcpyAsync(limbs, st->nprime, sl * k * 4, hipMemcpyHostToDevice, sm));
-        hipLaunchKernelGGL(k_load_forward, dim3(st->slots), dim3(tt), 0, sm, S->tab->t, limbs, k, S->d_nphat1, S->d_nphat2);
-        HIPCHK(hipGetLastError());
+        if (S->transforms()) {
+            hipLaunchKernelGGL(k_load_forward, dim3(st->slots), dim3(tt), 0, sm, S->tab->t, limbs, k, S->d_nphat1, S->d_nphat2);
+            HIPCHK(hipGetLastError());
+        }
         if (S->direct(false)) limbs += sl * k;  // N' stays
         HIPCHK(hipMemcpyAsync(limbs, st->n, sl * k * 4, hipMemcpyHostToDevice, sm));
         if (S->fd) HIPCHK(fd::launch_constants(S->fd_args(), k, st->slots, limbs - sl * k, limbs, S->d_fnp, S->d_fn, sm));
         if (S->wide) HIPCHK(fdw::launch_constants(S->fdw_args(), st->slots, limbs - sl * k, limbs, sm));
-        if (wrap) {
+        if (S->transforms() && wrap) {
             const uint32_t h = n / 2;
             F1 c1 = cinv(F1{mod1(8 * h), 0});
             F2 c2 = cinv(F2{(uint64_t)(8 * h), 0});
@@ -1713,7 +1742,7 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
             hipFree(t2);
             if (le != hipSuccess) return hip_fail("half factors launch", le);
             if (se != hipSuccess) return hip_fail("half factors", se);
-        } else {
+        } else if (S->transforms()) {
             hipLaunchKernelGGL(k_load_forward, dim3(st->slots), dim3(tt), 0, sm, S->tab->t, limbs, k, S->d_nhat1, S->d_nhat2);
             HIPCHK(hipGetLastError());
         }
@@ -1759,8 +1788,8 @@ int mm_set_exponent(void* st, size_t i, const uint32_t* words, size_t nwords, ui
     return 0;
 }
 
-// Device constants of one slot for a new modulus: N'-hat, and A|B (or N-hat), as mm_create
-// computes them for every slot. The exponent is cleared.
+// Device constants of one slot for a new modulus, as mm_create computes them for every slot. The
+// exponent is cleared.
 int mm_set_modulus(void* st, size_t i, const uint32_t* nl, const uint32_t* npl, const uint32_t* two_n) {
     State* S = (State*)st;
     Ctx* C = S->C;
@@ -1772,7 +1801,7 @@ int mm_set_modulus(void* st, size_t i, const uint32_t* nl, const uint32_t* npl, 
     const uint32_t k = S->k, n = S->n;
     hipStream_t sm = C->stream;
     if (!S->d_stage_lim && dalloc(&S->d_stage_lim, 2ull * k)) return 1;
-    if (S->wrap && ((!S->d_stage1 && dalloc(&S->d_stage1, n)) || (!S->d_stage2 && dalloc(&S->d_stage2, n)))) return 1;
+    if (S->transforms() && S->wrap && ((!S->d_stage1 && dalloc(&S->d_stage1, n)) || (!S->d_stage2 && dalloc(&S->d_stage2, n)))) return 1;
     uint32_t* lim = S->d_stage_lim;
     F1* t1 = S->d_stage1;
     F2* t2 = S->d_stage2;
@@ -1788,18 +1817,20 @@ int mm_set_modulus(void* st, size_t i, const uint32_t* nl, const uint32_t* npl, 
         A.first = (uint32_t)i;
         HIPCHK(fdw::launch_constants(A, 1, lim, lim + k, sm));
     }
-    const uint32_t tt = plan_threads(n);
-    hipLaunchKernelGGL(k_load_forward, dim3(1), dim3(tt), 0, sm, S->tab->t, lim, k, S->d_nphat1 + i * n, S->d_nphat2 + i * n);
-    HIPCHK(hipGetLastError());
-    if (S->wrap) {
-        const uint32_t h = n / 2;
-        F1 c1 = cinv(F1{mod1(8 * h), 0});
-        F2 c2 = cinv(F2{(uint64_t)(8 * h), 0});
-        hipLaunchKernelGGL(k_half_factors, dim3(1), dim3(plan_threads(h)), 0, sm, S->half->ht, lim + k, k, t1, t2,
-                           S->d_nhat1 + i * n, S->d_nhat2 + i * n, c1, c2);
-    } else {
-        hipLaunchKernelGGL(k_load_forward, dim3(1), dim3(tt), 0, sm, S->tab->t, lim + k, k, S->d_nhat1 + i * n,
-                           S->d_nhat2 + i * n);
+    if (S->transforms()) {
+        const uint32_t tt = plan_threads(n);
+        hipLaunchKernelGGL(k_load_forward, dim3(1), dim3(tt), 0, sm, S->tab->t, lim, k, S->d_nphat1 + i * n, S->d_nphat2 + i * n);
+        HIPCHK(hipGetLastError());
+        if (S->wrap) {
+            const uint32_t h = n / 2;
+            F1 c1 = cinv(F1{mod1(8 * h), 0});
+            F2 c2 = cinv(F2{(uint64_t)(8 * h), 0});
+            hipLaunchKernelGGL(k_half_factors, dim3(1), dim3(plan_threads(h)), 0, sm, S->half->ht, lim + k, k, t1, t2,
+                               S->d_nhat1 + i * n, S->d_nhat2 + i * n, c1, c2);
+        } else {
+            hipLaunchKernelGGL(k_load_forward, dim3(1), dim3(tt), 0, sm, S->tab->t, lim + k, k, S->d_nhat1 + i * n,
+                               S->d_nhat2 + i * n);
+        }
     }
     hipError_t le = hipGetLastError();
     hipError_t se = hipStreamSynchronize(sm);  // the staging buffers are reused by the next call
@@ -1862,20 +1893,21 @@ size_t read_window(const State* S, size_t i, bool plain, size_t* rows) {
 }
 
 // x[out] <- x[a] x[b] R^-1 on the context's stream, by the kernel that steps the batch where that is
-// the matrix-core or the double-precision one, else by the radix-4 kernel in `scratch`, or in the
-// batch's own (allocated once) when that is null.
+// the matrix-core or the double-precision one, else by the radix-4 kernel; the latter two in `scratch`
+// (MulScratch's bytes, of which the double-precision product uses 40 k of 60 k), or in the batch's own
+// (allocated once) when that is null.
 hipError_t launch_mul(State* S, uint32_t out, uint32_t a, uint32_t b, unsigned char* scratch) {
     hipStream_t sm = S->C->stream;
     if (S->mx) return mx::launch_mul(S->mx_args(false), S->k, out, a, b, sm);
-    if (S->fd) return fd::launch_mul(S->fd_args(), S->k, out, a, b, S->d_spec, sm);
     const MulScratch M(S->n, S->k);
     if (!scratch) {
         if (!S->d_mul) {
-            const hipError_t e = hipMalloc((void**)&S->d_mul, M.bytes);
+            const hipError_t e = hipMalloc((void**)&S->d_mul, S->fd ? fd::mul_elems(S->k) * sizeof(double2) : M.bytes);
             if (e != hipSuccess) return e;
         }
         scratch = S->d_mul;
     }
+    if (S->fd) return fd::launch_mul(S->fd_args(), S->k, out, a, b, (double2*)scratch, sm);
     auto kern = S->wrap ? k_mul<true> : k_mul<false>;
     hipLaunchKernelGGL(kern, dim3(1), dim3(S->threads), lds_scratch_bytes(S->threads), sm, S->args(), out, a, b, (F1*)scratch,
                        (F2*)(scratch + M.mb2), (F1*)(scratch + M.w1), (F2*)(scratch + M.w2), (uint32_t*)(scratch + M.lim));

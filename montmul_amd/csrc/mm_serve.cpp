@@ -135,6 +135,8 @@ struct Pool {
         if (!be_open) {
             if (S->open(S->user, &be)) return fail("cannot open a backend for length " + std::to_string(len));
             be_open = true;
+            // Under a budget a slot takes what it is counted at (other backends have no such limit).
+            if (S->opt.hbm_bytes) mm_hip_step_memory(&be, 0);
         }
         uint32_t cnt = std::max<uint32_t>(1, S->opt.pool_slots);
         const uint64_t per = mm_server_slot_bytes(len);
@@ -365,13 +367,10 @@ void hip_close(void* user, mm_backend* be) {
 
 extern "C" {
 
-// At L = 32,768 the register-transform step also stages its coefficients in HBM (24 n = 12 L). The step
-// kernels' own constants: the limbs of N' and N (4 L) on the matrix cores, their spectra (24 L) in double
-// precision, at L = 65,536 50 L and the scratch of a slot that runs (44 L and 8).
-uint64_t mm_server_slot_bytes(uint32_t len) {
-    const uint64_t own = len < 16 ? 0 : len <= 1024 ? 4ull * len : len <= 32768 ? 24ull * len : len == 65536 ? 94ull * len + 8 : 0;
-    return 50ull * len + 24 + (len == 32768 ? 12ull * len : 0) + own;
-}
+// What a transform plan holds in global mode (at L = 32,768 the register-transform step also stages its
+// coefficients in HBM: 24 n = 12 L); the matrix-core step (up to 18 L + 24) and the double-precision step (38 L + 24, 48 L + 24
+// at L = 32,768) hold less.
+uint64_t mm_server_slot_bytes(uint32_t len) { return 50ull * len + 24 + (len == 32768 ? 12ull * len : 0); }
 
 int mm_server_new(const mm_server_options* o, mm_open_fn open, mm_close_fn close, void* user, mm_server** out) {
     *out = nullptr;

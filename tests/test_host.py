@@ -170,6 +170,14 @@ def test_server_memory_budget_on_oracle():
         srv.close()
 
 
+@pytest.mark.parametrize("log_len", range(3, 18))
+def test_server_slot_bytes(log_len):
+    """A pool slot counts as what a transform plan holds, at every length: a budget admits the slots and
+    lengths that this allows."""
+    length = 1 << log_len
+    assert mm.Server.slot_bytes(length) == 50 * length + 24 + (12 * length if length == 32768 else 0)
+
+
 def test_cli_arguments():
     """The command line's option rules (main.rs:32-66): unknown, repeated and value-less keys
     are errors; values parse as numbers where needed."""
