@@ -41,8 +41,8 @@ constexpr size_t WEIGHTS = 48 * (H / 16) + 8 * 16 + 4 * 16 + 8 * 8 + 4 * 4;
 constexpr size_t TABLE = H + H / 256 + 32 + WEIGHTS;
 void make_tables(double2* out);
 hipError_t set_lds_limit();
-// Up to `bits` steps on slots [0, slots).
-hipError_t launch(Args A, u32 slots, u32 bits, hipStream_t sm);
+// Up to steps[g] steps on the slots [g GROUP, (g + 1) GROUP) of [0, slots).
+hipError_t launch(Args A, u32 slots, const u32* steps, hipStream_t sm);
 // The spectra of `count` slots from A.first on, from their limbs (npl, nl: K words per slot).
 hipError_t launch_constants(Args A, u32 count, const u32* npl, const u32* nl, hipStream_t sm);
 

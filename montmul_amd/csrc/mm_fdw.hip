@@ -319,9 +319,10 @@ template <int M> static void product(const Args& A, u32 slots, hipStream_t sm) {
     hipLaunchKernelGGL(k_sums<M>, dim3(slots * 16), dim3(256), 0, sm, A);
     hipLaunchKernelGGL(k_carry<M>, dim3(slots), dim3(T), M == WRAP ? 4 * K : 0, sm, A);
 }
-hipError_t launch(Args A, u32 slots, u32 bits, hipStream_t sm) {
+hipError_t launch(Args A, u32 slots, const u32* steps, hipStream_t sm) {
     for (A.first = 0; A.first < slots; A.first += GROUP) {
-        const u32 c = std::min(GROUP, slots - A.first);
+        const u32 c = std::min(GROUP, slots - A.first), bits = steps[A.first / GROUP];
+        if (bits == 0) continue;
         hipLaunchKernelGGL(k_digits, dim3(c), dim3(T), 0, sm, A, A.x + (size_t)A.first * K, 0u);
         for (u32 i = 0; i < bits; i++) {
             product<SQUARE>(A, c, sm);

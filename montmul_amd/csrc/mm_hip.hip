@@ -770,6 +770,12 @@ struct State {
         A.base = base;
         return A;
     }
+    // The most steps left in a slot of [first, end).
+    uint32_t most_left(uint32_t first, uint32_t end) const {
+        uint32_t r = 0;
+        for (uint32_t i = first; i < end; i++) r = std::max(r, nbits[i] - pos[i]);
+        return r;
+    }
     // A kernel of its own steps this batch, not a transform kernel.
     bool direct(bool bare) const { return mx || fd || (wide && !bare); }
     // The transform kernels run on this batch too, and their constants and work vectors are held (the
@@ -1052,10 +1058,16 @@ template <class Launch> int run_chunks(Ctx* C, uint64_t reps, Launch&& launch, f
     return 0;
 }
 
-// Up to `s` steps of one batch by the kernel that steps it alone (matrix-core or double-precision).
+// Up to `s` steps of one batch by the kernel that steps it alone (matrix-core or double-precision). At
+// L = 65,536 each of the groups of slots that run together takes nine launches a step: no more of them
+// than its own slots have steps left (enough for every replay, where these launches are captured).
 hipError_t launch_direct(State* S, uint32_t s, bool bare, hipStream_t sm) {
     if (S->mx) return mx::launch(S->mx_args(bare), S->k, S->slots, s, bare, sm);
-    if (S->wide) return fdw::launch(S->fdw_args(), S->slots, s, sm);
+    if (S->wide) {
+        std::vector<uint32_t> steps;
+        for (uint32_t f = 0; f < S->slots; f += fdw::GROUP) steps.push_back(std::min(s, S->most_left(f, std::min(S->slots, f + fdw::GROUP))));
+        return fdw::launch(S->fdw_args(), S->slots, steps.data(), sm);
+    }
     return fd::launch(S->fd_args(), S->k, S->slots, s, bare, sm);
 }
 
@@ -1063,8 +1075,7 @@ hipError_t launch_direct(State* S, uint32_t s, bool bare, hipStream_t sm) {
 int64_t steps(State* S, uint64_t bits, bool bare) {
     Ctx* C = S->C;
     if (hipSetDevice(C->device) != hipSuccess) { fail("hipSetDevice failed"); return MM_EFAULT; }
-    uint64_t most = 0;
-    for (uint32_t i = 0; i < S->slots; i++) most = std::max<uint64_t>(most, S->nbits[i] - S->pos[i]);
+    const uint64_t most = S->most_left(0, S->slots);
     uint64_t left = std::min(bits, most);
     S->last_ms = 0;
     S->last_launches = 0;
@@ -1349,7 +1360,7 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
     for (size_t g = 0; g < count; g++) {
         const State* S = G[g];
         (S->direct(false) ? direct : queued).push_back(g);
-        for (uint32_t i = 0; i < S->slots; i++) most = std::max<uint64_t>(most, S->nbits[i] - S->pos[i]);
+        most = std::max<uint64_t>(most, S->most_left(0, S->slots));
         if (!S->direct(false) && S->v2 && S->n <= 8192 && S->n / 8 > nt) nt = S->n / 8;
         G[g]->last_ms = 0;
         G[g]->last_launches = 0;
@@ -1378,7 +1389,7 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
     const uint32_t per_cu = nt == 1024 ? 1 : (2 * lds <= C->max_lds ? 2 : 1);
     hipStream_t sm = C->stream;
     std::vector<MixItem> items;
-    std::vector<uint32_t> list;
+    std::vector<uint32_t> list, direct_steps(count, 0);
     std::vector<double> cost;
     while (left > 0) {
         uint64_t s = left;
@@ -1408,14 +1419,15 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
             }
         }
         // The direct batches' streams (0: the context's), the longest first and each to the least
-        // loaded: a step takes about as long as the modulus is long, times the rounds of slots.
+        // loaded: a step takes about as long as the modulus is long, times the rounds of slots. A batch
+        // takes part with the steps it has left, not with the group's.
         std::vector<std::pair<double, size_t>> by_time;
         for (size_t g : direct) {
             const State* S = G[g];
-            uint64_t r = 0;
-            for (uint32_t i = 0; i < S->slots; i++) r = std::max<uint64_t>(r, S->nbits[i] - S->pos[i]);
+            direct_steps[g] = (uint32_t)std::min<uint64_t>(S->most_left(0, S->slots), s);
+            if (direct_steps[g] == 0) continue;
             const double per_cu = S->mx ? std::min(32.0, 4096.0 / S->k) : S->wide ? 0.125 : std::max(1.0, 8192.0 / S->k);
-            by_time.push_back({(double)std::min<uint64_t>(r, s) * S->k * std::max(1.0, S->slots / (per_cu * C->cus)), g});
+            by_time.push_back({(double)direct_steps[g] * S->k * std::max(1.0, S->slots / (per_cu * C->cus)), g});
         }
         std::stable_sort(by_time.begin(), by_time.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
         std::vector<size_t> lane[4];
@@ -1471,7 +1483,7 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
                            auto enqueue = [&](bool wide) {
                                for (int l = 3; l >= 0 && fe == hipSuccess; l--)
                                    for (size_t i = 0; i < lane[l].size() && fe == hipSuccess; i++)
-                                       if (G[lane[l][i]]->wide == wide) fe = launch_direct(G[lane[l][i]], (uint32_t)s, false, l ? C->side[l - 1] : sm);
+                                       if (G[lane[l][i]]->wide == wide) fe = launch_direct(G[lane[l][i]], direct_steps[lane[l][i]], false, l ? C->side[l - 1] : sm);
                            };
                            enqueue(false);
                            if (fe == hipSuccess && !queue.empty()) {
