@@ -127,8 +127,10 @@ typedef struct mm_options {
     int32_t autotune;        /* time every plan that can run a new batch's length (radix-8
                               * register kernel or radix-4 kernel, global mode with LDS tiles or
                               * LDS-resident, the register kernel's exchange tile, one or as many
-                              * slots per CU as fit) for 16 steps on the batch's own slots and keep
-                              * the fastest; the choice is cached per length and slot-count octave */
+                              * slots per CU as fit; and without prefer_lds the default step
+                              * kernel) for 16 steps on the batch's own slots and keep
+                              * the fastest; the choice is cached per length and slot-count octave.
+                              * mm_plan reports the fastest transform plan, mm_step_kernel what runs */
     uint32_t tile;           /* without autotune, global mode: the register kernel's exchange tile
                               * in elements (0: the default, half the vector at L = 1,024 .. 4,096,
                               * 2,048 at L = 8,192 and 4,096 at 16,384; also built: the whole

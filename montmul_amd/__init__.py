@@ -297,7 +297,8 @@ class Hip(Backend):
     def __init__(self, device=0, force_global=False, wraparound=True, max_launch_ms=0, prefer_lds=False,
                  autotune=False, tile=0, slots_per_cu=0):
         """autotune: time every plan that fits each new batch's length (16 steps on its own
-        slots) and keep the fastest, cached per length and slot-count octave. Without it, `tile`
+        slots), the default step kernel among them unless prefer_lds is given, and keep the
+        fastest, cached per length and slot-count octave. Without it, `tile`
         (the register kernel's exchange tile in global mode, in elements; 0 = default) and
         `slots_per_cu` (1 = one slot per CU; 0 = as many as fit) fix those choices."""
         self.options = Options(device, int(bool(force_global)), int(bool(wraparound)), max_launch_ms,

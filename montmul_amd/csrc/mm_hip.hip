@@ -493,10 +493,12 @@ struct FdTables {
 
 // A launch plan the autotuner can choose: kernel (register radix-8 or radix-4), mode (global or
 // LDS-resident), the register kernel's exchange tile in global mode (1: its default) and slots
-// per CU (0: as many as fit; 1: one, by padding the workgroup's LDS past half a CU's).
+// per CU (0: as many as fit; 1: one, by padding the workgroup's LDS past half a CU's). step: the
+// matrix-core or the double-precision step runs instead, where the batch can have it.
 struct PlanChoice {
     bool v2 = false, global = false;
     uint32_t tile = 1, slots_per_cu = 0;
+    bool step = false;
 };
 
 struct Ctx {
@@ -517,8 +519,8 @@ struct Ctx {
     unsigned char* mix_buf = nullptr;
     size_t mix_cap = 0;
     double mix_ms_per_step = 0;
-    // Autotuner choices: (n, wraparound, slot-count octave) -> (register kernel, global mode).
-    std::map<std::tuple<uint32_t, bool, uint32_t>, PlanChoice> tuned;
+    // Autotuner choices: (n, wraparound, whether a step kernel was among them, slot-count octave).
+    std::map<std::tuple<uint32_t, bool, bool, uint32_t>, PlanChoice> tuned;
     std::string name;
     std::mutex mu;
     std::map<uint32_t, std::shared_ptr<DevTables>> tabs;
@@ -1211,80 +1213,72 @@ bool plan_fits(const State* S, bool v2, bool global) {
     return plan_fits(S, p);
 }
 
-// Times every plan that fits for 16 steps on the batch's own slots and keeps the fastest:
-// kernel × mode × (register kernel in global mode) exchange tile × slots per CU. The slots hold
-// x = 0 and a 16-bit zero exponent for the timing (every kernel's work is the same for any data,
-// and 0 stays 0), and are cleared afterwards. The choice is cached per (n, wraparound,
-// slot-count octave), so later batches of that shape take it without timing.
-int autotune(State* S, bool v2ok) {
+// The steps that the autotuner times a candidate for.
+constexpr uint32_t TUNE_STEPS = 16;
+
+// The faster of two timed runs of TUNE_STEPS steps on the batch's own slots (the first also loads the code).
+// The slots hold x = 0 and a zero exponent (the kernels' work does not depend on the data, but for a
+// sign or two that take longer to find, and 0 stays 0), and are cleared afterwards.
+template <class Launch> int time_steps(State* S, double* ms, Launch&& launch) {
     Ctx* C = S->C;
-    const auto key = std::make_tuple(S->n, S->wrap, ilog2(S->slots));
-    bool have = false;
-    PlanChoice best;
-    best.v2 = S->v2;
-    best.global = S->global;
-    {
-        std::lock_guard<std::mutex> g(C->mu);
-        auto it = C->tuned.find(key);
-        if (it != C->tuned.end()) {
-            have = true;
-            best = it->second;
-        }
+    hipStream_t sm = C->stream;
+    const std::vector<uint32_t> nb(S->slots, TUNE_STEPS);
+    HIPCHK(hipMemcpyAsync(S->d_nbits, nb.data(), S->slots * 4ull, hipMemcpyHostToDevice, sm));
+    *ms = 1e300;
+    for (int rep = 0; rep < 2; rep++) {
+        HIPCHK(hipMemsetAsync(S->d_pos, 0, S->slots * 4ull, sm));
+        HIPCHK(hipEventRecord(C->ev0, sm));
+        HIPCHK(launch());
+        HIPCHK(hipEventRecord(C->ev1, sm));
+        HIPCHK(hipEventSynchronize(C->ev1));
+        float t = 0;
+        hipEventElapsedTime(&t, C->ev0, C->ev1);
+        *ms = std::min(*ms, (double)t);
     }
-    if (!have) {
-        const uint32_t T = 16;
-        hipStream_t sm = C->stream;
-        std::vector<uint32_t> nb(S->slots, T);
-        HIPCHK(hipMemcpyAsync(S->d_nbits, nb.data(), S->slots * 4ull, hipMemcpyHostToDevice, sm));
-        double best_ms = 1e300;
-        std::vector<PlanChoice> cands;
-        for (int v = v2ok ? 1 : 0; v >= 0; v--)
-            for (int g = 1; g >= 0; g--)
-                for (uint32_t tile : {1u, V2_WIDE_TILE, V1_TILE, S->n / 2})
-                    for (uint32_t spc : {0u, 1u}) {
-                        PlanChoice p;
-                        p.v2 = v;
-                        p.global = g;
-                        p.tile = v && g ? v2_tile_norm(S->n, tile) : tile;
-                        p.slots_per_cu = spc;
-                        bool seen = false;
-                        for (const PlanChoice& q : cands)
-                            seen |= q.v2 == p.v2 && q.global == p.global && q.tile == p.tile && q.slots_per_cu == p.slots_per_cu;
-                        if (!seen && plan_fits(S, p)) cands.push_back(p);
-                    }
-        for (const PlanChoice& p : cands) {
-            set_plan(S, p);
-            double t = 1e300;
-            for (int rep = 0; rep < 2; rep++) {  // the first launch also loads the code
-                HIPCHK(hipMemsetAsync(S->d_pos, 0, S->slots * 4ull, sm));
-                HIPCHK(hipEventRecord(C->ev0, sm));
+    HIPCHK(hipMemsetAsync(S->d_nbits, 0, S->slots * 4ull, sm));
+    HIPCHK(hipMemsetAsync(S->d_pos, 0, S->slots * 4ull, sm));
+    HIPCHK(hipMemsetAsync(S->d_err, 0, S->slots * 4ull, sm));
+    HIPCHK(hipStreamSynchronize(sm));
+    return 0;
+}
+
+// Times every transform plan that fits: kernel × mode × (register kernel in global mode) exchange
+// tile × slots per CU. The fastest to *best, its time to *best_ms.
+int time_plans(State* S, bool v2ok, PlanChoice* best, double* best_ms) {
+    std::vector<PlanChoice> cands;
+    for (int v = v2ok ? 1 : 0; v >= 0; v--)
+        for (int g = 1; g >= 0; g--)
+            for (uint32_t tile : {1u, V2_WIDE_TILE, V1_TILE, S->n / 2})
+                for (uint32_t spc : {0u, 1u}) {
+                    PlanChoice p;
+                    p.v2 = v;
+                    p.global = g;
+                    p.tile = v && g ? v2_tile_norm(S->n, tile) : tile;
+                    p.slots_per_cu = spc;
+                    bool seen = false;
+                    for (const PlanChoice& q : cands)
+                        seen |= q.v2 == p.v2 && q.global == p.global && q.tile == p.tile && q.slots_per_cu == p.slots_per_cu;
+                    if (!seen && plan_fits(S, p)) cands.push_back(p);
+                }
+    *best_ms = 1e300;
+    for (const PlanChoice& p : cands) {
+        set_plan(S, p);
+        double t;
+        if (time_steps(S, &t, [&] {
                 if (p.v2)
                     hipLaunchKernelGGL(pick_step_v2(ilog2(S->n), p.global, false, S->tile), dim3(S->slots), dim3(S->threads),
-                                       S->lds, sm, S->vargs(), 0u, T);
+                                       S->lds, S->C->stream, S->vargs(), 0u, TUNE_STEPS);
                 else
-                    hipLaunchKernelGGL(pick_step(p.global, S->wrap, false), dim3(S->slots), dim3(S->threads), S->lds, sm,
-                                       S->step_args(), 0u, T);
-                HIPCHK(hipGetLastError());
-                HIPCHK(hipEventRecord(C->ev1, sm));
-                HIPCHK(hipEventSynchronize(C->ev1));
-                float ms = 0;
-                hipEventElapsedTime(&ms, C->ev0, C->ev1);
-                t = std::min(t, (double)ms);
-            }
-            if (t < best_ms) {
-                best_ms = t;
-                best = p;
-            }
+                    hipLaunchKernelGGL(pick_step(p.global, S->wrap, false), dim3(S->slots), dim3(S->threads), S->lds,
+                                       S->C->stream, S->step_args(), 0u, TUNE_STEPS);
+                return hipGetLastError();
+            }))
+            return 1;
+        if (t < *best_ms) {
+            *best_ms = t;
+            *best = p;
         }
-        HIPCHK(hipMemsetAsync(S->d_nbits, 0, S->slots * 4ull, sm));
-        HIPCHK(hipMemsetAsync(S->d_pos, 0, S->slots * 4ull, sm));
-        HIPCHK(hipMemsetAsync(S->d_err, 0, S->slots * 4ull, sm));
-        HIPCHK(hipStreamSynchronize(sm));
-        std::lock_guard<std::mutex> g(C->mu);
-        C->tuned[key] = best;
     }
-    set_plan(S, best);
-    S->tuned = true;
     return 0;
 }
 
@@ -1524,99 +1518,33 @@ int64_t group_steps(State* const* G, size_t count, uint64_t bits, size_t* which)
     return MM_OK;
 }
 
-}  // namespace
-
-// ---- C ABI -------------------------------------------------------------------------------------
-extern "C" {
-
-const char* mm_last_error(void) { return g_err.c_str(); }
-
-int mm_device_count(void) {
-    int n = 0;
-    if (hipGetDeviceCount(&n) != hipSuccess) { fail("hipGetDeviceCount failed"); return -1; }
-    return n;
+// ---- Batches --------------------------------------------------------------------------------------
+// Whether the register-transform kernel may be planned at all.
+bool kernel_v1_asked() {
+    const char* e = getenv("MONTMUL_KERNEL");
+    return e && strcmp(e, "v1") == 0;
 }
 
-int mm_hip_open(const mm_options* opts, mm_backend* out) {
-    memset(out, 0, sizeof(*out));
-    auto C = new Ctx();
-    C->opts = opts ? *opts : mm_options{0, 0, 1, 0, 0, 0};
-    C->device = C->opts.device;
-    int count = 0;
-    if (hipGetDeviceCount(&count) != hipSuccess || C->device < 0 || C->device >= count) {
-        delete C;
-        return fail("no HIP device " + std::to_string(opts ? opts->device : 0));
+// The step kernel that runs a batch whose options name no transform kernel, mode or tile of its own
+// (force_global at n >= 512 is the default plan). The matrix-core step's work grows as n^2: at L = 1,024 it
+// does 91 M squarings/s, where the double-precision one would do 75 M by its work; at 2,048 30 M against 36 M.
+// At L = 65,536 a slot takes several workgroups: 148 K squarings/s at 64 slots against the radix-4
+// kernel's 32 K, at 256 148 K against 86 K, at 1,024 155 K against 88 K.
+struct StepKernels {
+    bool mx = false, fd = false, wide = false;
+    StepKernels(const Ctx* C, uint32_t k, uint32_t n, uint32_t base) {
+        const bool v2_length = n >= 512 && n <= 16384;
+        if (!C->opts.wraparound || C->opts.prefer_lds || kernel_v1_asked() || (!v2_length && C->opts.force_global)) return;
+        mx = mx::fits(k, base);
+        fd = !mx && fd::fits(k, base);
+        wide = !mx && !fd && fdw::fits(k, base);
     }
-    hipDeviceProp_t p;
-    if (hipSetDevice(C->device) != hipSuccess || hipGetDeviceProperties(&p, C->device) != hipSuccess) {
-        delete C;
-        return fail("cannot query HIP device");
-    }
-    C->cus = p.multiProcessorCount;
-    C->max_lds = p.sharedMemPerBlock;
-    // Marketing name with the architecture (e.g. "AMD Instinct MI355X (gfx950)").
-    C->name = p.name[0] ? std::string(p.name) + " (" + std::string(p.gcnArchName).substr(0, 6) + ")" : std::string(p.gcnArchName);
-    if (hipStreamCreateWithFlags(&C->stream, hipStreamNonBlocking) != hipSuccess || hipEventCreate(&C->ev0) != hipSuccess ||
-        hipEventCreate(&C->ev1) != hipSuccess || set_lds_limit(C)) {
-        delete C;
-        return 1;
-    }
-    // The fixed product scratch's address on this device (taken on the device's first open).
-    // Only mm_mul_noalloc needs it: a failure is reported there.
-    if (scratch_address(C->device, &C->scratch)) C->scratch_err = g_err;
-    out->self = C;
-    out->set_modulus = mm_set_modulus;
-    out->run_group = mm_run_group;
-    out->create = mm_create;
-    out->destroy = mm_destroy;
-    out->load = mm_load;
-    out->set_exponent = mm_set_exponent;
-    out->run = mm_run;
-    out->mul = mm_mul;
-    out->read = mm_read;
-    out->remaining = mm_remaining;
-    out->failed_slots = mm_failed_slots;
-    out->last_error = mm_last_error;
-    out->set_ones = mm_set_ones;
-    out->is_one_many = mm_is_one_many;
-    // Limits (gpu/mod.rs:272-283): bound Q = P1 * P2, lengths 2^3..2^24, full_k = wraparound.
-    u128 Q = (u128)P1 * P2;
-    out->bound_lo = (uint64_t)Q;
-    out->bound_hi = (uint64_t)(Q >> 64);
-    out->min_len = 8;
-    out->max_len = 1u << 24;
-    out->full_k = C->opts.wraparound ? 1 : 0;
-    return 0;
-}
+    bool any() const { return mx || fd || wide; }
+};
 
-void mm_hip_close(mm_backend* be) {
-    Ctx* C = (Ctx*)be->self;
-    if (!C) return;
-    hipSetDevice(C->device);
-    C->tabs.clear();
-    C->fd_tabs.clear();
-    if (C->mix_buf) hipFree(C->mix_buf);
-    for (hipStream_t sd : C->side)
-        if (sd) hipStreamDestroy(sd);
-    for (hipEvent_t e : {C->fork, C->join[0], C->join[1], C->join[2]})
-        if (e) hipEventDestroy(e);
-    if (C->ev0) hipEventDestroy(C->ev0);
-    if (C->ev1) hipEventDestroy(C->ev1);
-    if (C->stream) hipStreamDestroy(C->stream);
-    delete C;
-    be->self = nullptr;
-}
-
-int mm_hip_step_memory(mm_backend* be, uint64_t bytes) {
-    if (be->create != mm_create) return fail("not a HIP backend");
-    ((Ctx*)be->self)->step_memory = bytes;
-    return 0;
-}
-
-// Backend::create (reference: Gpu::create, gpu/mod.rs:325-370).
-int mm_create(void* self, const mm_batch_setup* st, void** out) {
-    Ctx* C = (Ctx*)self;
-    *out = nullptr;
+// A batch: by the context's options, by a plan that the autotuner chose, or (tune) with the state of every
+// transform plan, for the autotuner to time.
+int make_batch(Ctx* C, const mm_batch_setup* st, const PlanChoice* plan, bool tune, std::unique_ptr<State>* out) {
     if (hipSetDevice(C->device) != hipSuccess) return fail("hipSetDevice failed");
     if (st->len < 8 || (st->len & (st->len - 1)) || st->len > (1u << 24)) return fail("unsupported transform length");
     if (st->slots == 0) return fail("empty batch");
@@ -1628,9 +1556,11 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
     S->C = C;
     S->device = C->device;
     S->k = k; S->len = st->len; S->n = n; S->base = st->base; S->slots = st->slots; S->wrap = wrap;
-    const char* kenv = getenv("MONTMUL_KERNEL");
-    const bool v2ok = plan_fits(S.get(), true, true) && !(kenv && strcmp(kenv, "v1") == 0);
-    if (v2ok) {
+    const bool v2ok = plan_fits(S.get(), true, true) && !kernel_v1_asked();
+    if (plan) {
+        set_plan(S.get(), *plan);
+        S->tuned = true;
+    } else if (v2ok) {
         // Global mode unless LDS is preferred: its smaller LDS footprint (T in HBM, exchange
         // tiles of at most 2,048 elements) fits more workgroups per CU, and that wins at every
         // length of this kernel (squarings x bits per second, 4,096 slots: L = 1,024: 3.73e11
@@ -1640,8 +1570,7 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
     } else {
         set_plan(S.get(), false, C->opts.force_global || !plan_fits(S.get(), false, false));
     }
-    const bool tune = C->opts.autotune && !C->opts.force_global;
-    if (!tune && (C->opts.tile != 0 || C->opts.slots_per_cu != 0)) {
+    if (!plan && !tune && (C->opts.tile != 0 || C->opts.slots_per_cu != 0)) {
         PlanChoice p;
         p.v2 = S->v2;
         p.global = S->global;
@@ -1652,17 +1581,12 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
                         " is not a plan for L = " + std::to_string(st->len));
         set_plan(S.get(), p);
     }
-    // The matrix-core step and the double-precision step run every plan that names no transform
-    // kernel, mode or tile of its own
-    // (force_global at n >= 512 is the default plan). The first one's work grows as n^2: at L = 1,024 it
-    // does 91 M squarings/s, where the second would do 75 M by its work; at 2,048 30 M against 36 M.
-    // At L = 65,536 a slot takes several workgroups: 148 K squarings/s at 64 slots against the radix-4
-    // kernel's 32 K, at 256 148 K against 86 K.
-    const bool unnamed = wrap && !tune && !C->opts.prefer_lds && C->opts.tile == 0 && C->opts.slots_per_cu == 0 &&
-                         (v2ok || (!C->opts.force_global && !(kenv && strcmp(kenv, "v1") == 0)));
-    S->mx = unnamed && mx::fits(k, st->base);
-    S->fd = unnamed && !S->mx && S->global && fd::fits(k, st->base);  // T goes through HBM
-    S->wide = unnamed && !S->mx && !S->fd && S->global && fdw::fits(k, st->base);
+    if (!tune && (plan ? plan->step : C->opts.tile == 0 && C->opts.slots_per_cu == 0)) {
+        const StepKernels f(C, k, n, st->base);
+        S->mx = f.mx;
+        S->fd = f.fd;
+        S->wide = f.wide;
+    }
     // Device memory. Of every slot: x, the exponent of up to k words, the words of its state, the two raw
     // values of 1 with a list word and a flag. By the transform kernels: N'-hat, N-hat or A|B, work
     // vectors and limbs in global mode. By the matrix-core step: the limbs of N' and N (and of T, for
@@ -1760,7 +1684,6 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
         }
         HIPCHK(hipStreamSynchronize(sm));
     }
-    if (tune && autotune(S.get(), v2ok)) return 1;
     S->h_x.assign(sl * k, 0);
     S->x_fresh.assign(sl, 1);
     S->x_dirty.assign(sl, 0);
@@ -1768,6 +1691,150 @@ int mm_create(void* self, const mm_batch_setup* st, void** out) {
     S->e_dirty.assign(sl, 0);
     S->nbits.assign(sl, 0);
     S->pos.assign(sl, 0);
+    *out = std::move(S);
+    return 0;
+}
+
+// The autotuner: times every transform plan that can run the batch, and the step kernel where one can, each
+// for TUNE_STEPS steps on the batch's own slots, and makes the batch with the fastest. The choice is
+// cached per (n, wraparound, step kernel or not, slot-count octave), so later batches of that shape take it
+// without timing. The candidates' state is not held at once: the step kernel is timed on a batch of its own.
+int autotune(Ctx* C, const mm_batch_setup* st, std::unique_ptr<State>* out) {
+    const uint32_t n = st->len / 2;
+    const auto key = std::make_tuple(n, C->opts.wraparound != 0, StepKernels(C, st->k, n, st->base).any(), ilog2(std::max<uint64_t>(st->slots, 1)));
+    {
+        PlanChoice p;
+        bool have = false;
+        {
+            std::lock_guard<std::mutex> g(C->mu);
+            auto it = C->tuned.find(key);
+            if ((have = it != C->tuned.end())) p = it->second;
+        }
+        if (have) return make_batch(C, st, &p, false, out);
+    }
+    PlanChoice best;
+    double best_ms, step_ms;
+    if (make_batch(C, st, nullptr, true, out)) return 1;
+    if (time_plans(out->get(), plan_fits(out->get(), true, true) && !kernel_v1_asked(), &best, &best_ms)) return 1;
+    if (std::get<2>(key)) {
+        out->reset();
+        best.step = true;
+        if (make_batch(C, st, &best, false, out)) return 1;
+        State* S = out->get();
+        if (!S->direct(false)) return 0;  // no memory for the step kernel's own state this time
+        S->nbits.assign(S->slots, TUNE_STEPS);
+        if (time_steps(S, &step_ms, [&] { return launch_direct(S, TUNE_STEPS, false, C->stream); })) return 1;
+        S->nbits.assign(S->slots, 0);
+        if (step_ms > best_ms) {
+            out->reset();
+            best.step = false;
+            if (make_batch(C, st, &best, false, out)) return 1;
+        }
+    } else {
+        set_plan(out->get(), best);
+        (*out)->tuned = true;
+    }
+    std::lock_guard<std::mutex> g(C->mu);
+    C->tuned[key] = best;
+    return 0;
+}
+
+
+}  // namespace
+
+// ---- C ABI -------------------------------------------------------------------------------------
+extern "C" {
+
+const char* mm_last_error(void) { return g_err.c_str(); }
+
+int mm_device_count(void) {
+    int n = 0;
+    if (hipGetDeviceCount(&n) != hipSuccess) { fail("hipGetDeviceCount failed"); return -1; }
+    return n;
+}
+
+int mm_hip_open(const mm_options* opts, mm_backend* out) {
+    memset(out, 0, sizeof(*out));
+    auto C = new Ctx();
+    C->opts = opts ? *opts : mm_options{0, 0, 1, 0, 0, 0};
+    C->device = C->opts.device;
+    int count = 0;
+    if (hipGetDeviceCount(&count) != hipSuccess || C->device < 0 || C->device >= count) {
+        delete C;
+        return fail("no HIP device " + std::to_string(opts ? opts->device : 0));
+    }
+    hipDeviceProp_t p;
+    if (hipSetDevice(C->device) != hipSuccess || hipGetDeviceProperties(&p, C->device) != hipSuccess) {
+        delete C;
+        return fail("cannot query HIP device");
+    }
+    C->cus = p.multiProcessorCount;
+    C->max_lds = p.sharedMemPerBlock;
+    // Marketing name with the architecture (e.g. "AMD Instinct MI355X (gfx950)").
+    C->name = p.name[0] ? std::string(p.name) + " (" + std::string(p.gcnArchName).substr(0, 6) + ")" : std::string(p.gcnArchName);
+    if (hipStreamCreateWithFlags(&C->stream, hipStreamNonBlocking) != hipSuccess || hipEventCreate(&C->ev0) != hipSuccess ||
+        hipEventCreate(&C->ev1) != hipSuccess || set_lds_limit(C)) {
+        delete C;
+        return 1;
+    }
+    // The fixed product scratch's address on this device (taken on the device's first open).
+    // Only mm_mul_noalloc needs it: a failure is reported there.
+    if (scratch_address(C->device, &C->scratch)) C->scratch_err = g_err;
+    out->self = C;
+    out->set_modulus = mm_set_modulus;
+    out->run_group = mm_run_group;
+    out->create = mm_create;
+    out->destroy = mm_destroy;
+    out->load = mm_load;
+    out->set_exponent = mm_set_exponent;
+    out->run = mm_run;
+    out->mul = mm_mul;
+    out->read = mm_read;
+    out->remaining = mm_remaining;
+    out->failed_slots = mm_failed_slots;
+    out->last_error = mm_last_error;
+    out->set_ones = mm_set_ones;
+    out->is_one_many = mm_is_one_many;
+    // Limits (gpu/mod.rs:272-283): bound Q = P1 * P2, lengths 2^3..2^24, full_k = wraparound.
+    u128 Q = (u128)P1 * P2;
+    out->bound_lo = (uint64_t)Q;
+    out->bound_hi = (uint64_t)(Q >> 64);
+    out->min_len = 8;
+    out->max_len = 1u << 24;
+    out->full_k = C->opts.wraparound ? 1 : 0;
+    return 0;
+}
+
+void mm_hip_close(mm_backend* be) {
+    Ctx* C = (Ctx*)be->self;
+    if (!C) return;
+    hipSetDevice(C->device);
+    C->tabs.clear();
+    C->fd_tabs.clear();
+    if (C->mix_buf) hipFree(C->mix_buf);
+    for (hipStream_t sd : C->side)
+        if (sd) hipStreamDestroy(sd);
+    for (hipEvent_t e : {C->fork, C->join[0], C->join[1], C->join[2]})
+        if (e) hipEventDestroy(e);
+    if (C->ev0) hipEventDestroy(C->ev0);
+    if (C->ev1) hipEventDestroy(C->ev1);
+    if (C->stream) hipStreamDestroy(C->stream);
+    delete C;
+    be->self = nullptr;
+}
+
+int mm_hip_step_memory(mm_backend* be, uint64_t bytes) {
+    if (be->create != mm_create) return fail("not a HIP backend");
+    ((Ctx*)be->self)->step_memory = bytes;
+    return 0;
+}
+
+// Backend::create (reference: Gpu::create, gpu/mod.rs:325-370).
+int mm_create(void* self, const mm_batch_setup* st, void** out) {
+    Ctx* C = (Ctx*)self;
+    *out = nullptr;
+    std::unique_ptr<State> S;
+    if (C->opts.autotune && !C->opts.force_global ? autotune(C, st, &S) : make_batch(C, st, nullptr, false, &S)) return 1;
     *out = S.release();
     return 0;
 }
