@@ -7,14 +7,21 @@
 // zeta^j, zeta = exp(i pi / 2C), cyclic length C, gives products modulo X^2C + 1. Coefficients are
 // integers and are rounded to the nearest one.
 //
-// Exactness. With u = 2^-53, in the 2-norm a radix-16 pass adds at most 4 u (four levels of sums) and
-// 2 x 3 u (its inner rotations), each of the four twiddle factors between passes and the weights
-// 3.3 u (tables within u / 2), the last radix-2 or 4 stage 2 u: 49 u a transform. The two transforms
-// of a product, its pointwise step and the inverse make at most 150 u, and a coefficient of a b is
-// off by at most |a| |b| 150 u <= C 2^30 150 2^-53: 0.04, 0.07, 0.15 and 0.29 at L = 2,048, 4,096,
-// 8,192 and 16,384, below the 0.5 that rounding needs, for any digits (SplitSlot counts L = 32,768). Measured,
-// the farthest from an integer at L = 4,096 / 8,192 / 16,384 / 32,768: 6e-5 / 9e-5 / 1.2e-4 / 2.7e-4 on random
-// moduli, 0.003 / 0.006 / 0.012 / 0.024 on digits of the largest size with equal or alternating signs.
+// Exactness. With u = 2^-53, along each path from an input to an output of a transform a radix-16 pass
+// adds a relative error of at most 4 u (four levels of sums) and 2 x 3 u (its inner rotations), each of
+// the four twiddle factors between passes and the weights 3.3 u (tables within u / 2), the last
+// radix-2 or 4 stage 2 u: e = 49 u a transform. What that makes of a coefficient of a b, with A and B the
+// spectra, of length n and of 2-norms sqrt(n) |a| and sqrt(n) |b|:
+//   - the forward transforms' errors, at most e sqrt(n) |a| in the 2-norm (every pass is a multiple of a unitary
+//     one), reach a coefficient as 1/n sum |dA_j| |B_j| <= e |a| |b| each (Cauchy and Schwarz);
+//   - the inverse's error at an output is at most e times the sum of what its paths bring there,
+//     1/n sum |A_j B_j| <= |a| |b|, and so is the pointwise product's, with 3 u. (A bound by the 2-norm of a b would
+//     not do: that can be sqrt(C) |a| |b|.)
+// In all 150 u |a| |b| <= C 2^30 150 2^-53: 0.04, 0.07, 0.15 and 0.29 at L = 2,048, 4,096,
+// 8,192 and 16,384, below the 0.5 that rounding needs, for any digits (SplitSlot counts L = 32,768). The
+// farthest from an integer that a copy of these kernels that keeps the largest distance found:
+// L = 2,048 / 4,096 / 8,192 / 16,384 / 32,768: 5e-5 / 6e-5 / 9e-5 / 1.2e-4 / 2.4e-4 on random moduli, 0.0012 / 0.0024 /
+// 0.006 / 0.012 / 0.023 on digits of the largest size with equal, alternating and other periodic signs.
 //
 // A step, R = 2^(32k) = 2^(16 C):
 //     T = c x^2                  transform of length C, square, inverse
@@ -49,8 +56,17 @@ typedef int64_t i64;
 typedef uint16_t u16;
 
 constexpr u32 SGN = 0x80008000u;
-constexpr u64 BETA = 0x7fffffffu;  // |limb sums| < BETA (2^32 - 1): c C <= 2^16
+constexpr u64 BETA = 0x7fffffffu;  // |limb sums| < BETA (2^32 - 1): c C < 2^17 (fits)
 constexpr u64 BIAS = BETA * 0xffffffffull;
+// A limb's sum is c (v + 2^16 w), v and w coefficients: of C + 1 digits, the highest 0 or 1, so at most
+// C 2^30 + 2^16. Biased (and with T's limbs, for x) it stays below 2^64 with a carry from below.
+constexpr bool sums_fit(u64 c, u64 C) {
+    const unsigned __int128 most = (unsigned __int128)c * ((C << 30) + 65536) * 65537;
+    return most < BIAS && most + BIAS + SGN + BETA + 0xffffffffull < (unsigned __int128)1 << 64;
+}
+static_assert(sums_fit(131071 / 2048, 2048) && sums_fit(131071 / 4096, 4096) && sums_fit(131071 / 8192, 8192) &&
+                  sums_fit(131071 / 16384, 16384) && sums_fit(131071 / 32768, 32768),
+              "c C < 2^17");
 constexpr double MAGIC = 6755399441055744.0;  // 1.5 2^52: integers appear in the low bits of the sum
 constexpr u64 MAGIC_BITS = 0x4338000000000000ull;
 
@@ -454,8 +470,8 @@ __device__ __forceinline__ void inverse(Z* v, const Tables& W, unsigned char* ld
 }
 
 // ---- Carries over the workgroup: 8 limb sums per thread, thread 0 lowest ----------------------
-// Sums < 2^63; limbs in l. Returns the carry out. `sc`: 32 words of scratch, another for the next
-// call.
+// Sums (biased: not negative) that stay below 2^64 with a carry of 32 bits added; limbs in l. Returns the
+// carry out. `sc`: 32 words of scratch, another for the next call.
 template <u32 WAVES> __device__ __forceinline__ u32 bcarry(const u64* v, u32* l, u32* sc, u32 t) {
     const u32 lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
     u32 c = 0;

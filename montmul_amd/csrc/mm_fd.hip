@@ -60,7 +60,7 @@ __global__ __launch_bounds__(LOGC == 15 ? 1024 : Geo<LOGC == 15 ? 14 : LOGC>::T)
         plain<LOGC>(A, first + blockIdx.x, out + row * k, T + row * 2 * k, lds);
 }
 
-// k = 1,024 .. 16,384 limbs; c C < 2^17 keeps the limb sums of T below BETA (2^32 - 1).
+// k = 1,024 .. 16,384 limbs; c C < 2^17 keeps the limb sums of T below BETA (2^32 - 1) (sums_fit).
 bool fits(u32 k, u32 base) { return k >= 1024 && k <= 16384 && (k & (k - 1)) == 0 && (u64)base * 2 * k < 131072; }
 
 double2 unit(u64 num, u64 den) {

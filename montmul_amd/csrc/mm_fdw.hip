@@ -1,7 +1,7 @@
 // mm_fdw.hip - the double-precision step at L = 65,536, several workgroups to a slot.
 //
 // Digits of 16 bits would leave no proof of exactness at this length (C 2^30 127 2^-53 = 0.99), so a
-// residue is 131,072 signed digits in base 256: 131,072 2^14 130 2^-53 = 3e-5. As in SplitSlot (mm_fd.h),
+// residue is 131,072 signed digits in base 256: 131,072 2^14 130 2^-53 = 3e-5 (2e-6 found, as in mm_fd.h). As in SplitSlot (mm_fd.h),
 // X^C - i is a product of eight X^H - z_p, H = 16,384, z_p = exp(2 pi i (4p + 1) / 32), and the last product,
 // right-angled at half the length, of four: z_p = exp(2 pi i (4p + 1) / 16). The parts are independent
 // weighted transforms of length H, one workgroup each; the coefficients follow from the parts' results by
@@ -283,7 +283,8 @@ __global__ __launch_bounds__(1024) void k_limbs(Args A) {
     }
 }
 
-// Limb sums stay below BETA (2^32 - 1) = 2^63: c 2^31 (2^24 + 2^16 + 2^8 + 1), c < 128.
+// Limb sums stay below BETA (2^32 - 1): c (2^31 + 2^8) (2^24 + 2^16 + 2^8 + 1) with c < 128.
+static_assert((unsigned __int128)127 * ((1ull << 31) + 256) * 0x1010101u < BIAS, "c < 128");
 bool fits(u32 k, u32 base) { return k == K && base < 128; }
 
 void make_tables(double2* out) {

@@ -48,6 +48,7 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 constexpr u32 SGN = 0x80808080u;   // 128 in every byte
 constexpr u64 BETA = 1u << 27;     // |column sums| < BETA (2^32 - 1): base * n <= 2^20
 constexpr u64 BIAS = BETA * 0xffffffffull;
+static_assert((u64)(1u << 20) * ((1u << 14) + 1) * 0x1010101u < BIAS, "base * n <= 2^20");
 
 // The steps' arguments, per batch.
 struct Args {
