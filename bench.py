@@ -45,6 +45,8 @@ PROFILE = {8192: "profiles/k_steps_fd_100kbit_4096slots.md",
 TRAFFIC_PER_SLOT_STEP = {8192: 261_363, 32768: 3_550_055}
 VALU_PER_SLOT_STEP = {8192: 43_132, 32768: 233_944}
 KERNELS = {4: "k_steps (radix-4)", 8: "k_steps_v2", 32: "k_steps_mx (matrix cores)", 64: "k_steps_fd (double precision)"}
+ARITHMETIC = {4: "integer (M31 x M61)", 8: "integer (M31 x M61)", 32: "int8 matrix cores, 32-bit sums",
+              64: "float64 transforms, every coefficient rounded to its exact integer"}
 REF_5090 = 1_536_441.0     # reference, RTX 5090, 170 slots (README.md:14)
 
 
@@ -286,7 +288,8 @@ def main():
         "scaling": "weak",
         "vs_baseline": round(value / REF_5090, 4) if args.bits == 100_000 else None,
         "vs_baseline_ref": "reference Gpu backend, RTX 5090, 170 slots, 1,536,441 squarings/s (README.md:14)",
-        "dtype": "u32",
+        "dtype": "u32",  # the limbs; the arithmetic on them:
+        "arithmetic": ARITHMETIC[head["kernel"]],
         "data": "synthetic (GMP generator seeded 2026, as the reference's score workload)",
         "config": {"workload": f"{args.bits:,}-bit moduli, L={L}, k={head['k']}, base 3, top {ebits:,} bits of N-1, " +
                                ("global mode (T and constants in HBM; transform exchanges through LDS)"

@@ -204,10 +204,12 @@ uint64_t mm_max_lds(void *self);
 int mm_device_name(void *self, char *buf, size_t len);
 /* The Hip table's set_modulus (see mm_backend): device constants of one slot rebuilt. */
 int mm_set_modulus(void *state, size_t slot, const uint32_t *n, const uint32_t *nprime, const uint32_t *two_n);
-/* The Hip table's run_group (see mm_backend): the states' slots are stepped by one persistent
- * launch of the mixed-length kernel per chunk. Its workgroups take per-slot descriptors (length
- * class, slot) from a queue in device memory, longest work first, and step each slot at its own
- * length. Every state must come from the same mm_hip_open. */
+/* The Hip table's run_group (see mm_backend). States that have a step kernel of their own
+ * (mm_step_kernel 32 or 64) are stepped by it, side by side on up to four streams, each for the steps it
+ * has left. The others' slots are stepped by one persistent launch of the mixed-length kernel per chunk:
+ * its workgroups take per-slot descriptors (length class, slot) from a queue in device memory,
+ * longest work first, and step each slot at its own length. Every state must come from the same
+ * mm_hip_open. */
 int64_t mm_run_group(void *const *states, size_t count, uint64_t bits, size_t *which);
 /* Device time of the step kernel launches of the latest run, in milliseconds (HIP events on
  * the batch's stream), and the number of launches. No reference counterpart: measurement. */

@@ -1,8 +1,10 @@
-"""Mixed-length batch benchmark: moduli of many sizes stepped by one persistent launch against
-the same moduli run as plain per-length batches, one length after another.
+"""Mixed-length batch benchmark: moduli of many sizes stepped together against the same moduli run
+as plain per-length batches, one length after another. Together each length runs its own step
+kernel, side by side on up to four streams; with --transforms (the modular transforms, as
+Hip(prefer_lds=True)) all of them share one persistent launch of the mixed-length kernel.
 
     python -m montmul_amd.mixed [--count 1000] [--seed 11] [--min-bits 2048] [--max-bits 200000] \
-        [--ebits 4000] [--check 16] [--parts]
+        [--ebits 4000] [--check 16] [--parts] [--transforms]
 
 Moduli: `count` random odd numbers whose bit sizes are log-uniform in [min-bits, max-bits]
 (Python `random` seeded `seed`), each at the transform length of its own size (L = 256 ..
@@ -14,13 +16,13 @@ and one run(ebits) of every per-length ModBatch in turn. Checks: every slot's ra
 both forms, and read == pow(3, e, N) (GMP) on `check` slots spread over the lengths.
 
 Prints one JSON line: squarings/s of both forms (squarings = sum of exponent bits), the mixed
-launch's kernel milliseconds (HIP events), slots per length, and the check counts.
+run's milliseconds on the device (HIP events), slots per length, and the check counts.
 
-`--parts` also times the mixed launch on parts of the workload, to show what bounds it: the
-longest length's slots (plus one shortest-length slot of 16 steps, so that they run in the mixed
-kernel rather than their own), every other slot alone, and every other slot plus one slot of the
-longest length with a 16-bit exponent (which puts the others in that length's workgroup size
-while adding almost no work). Their kernel milliseconds go into the line as "parts_ms".
+`--parts` also times the mixed run on parts of the workload, to show what bounds it: the
+longest length's slots (plus one shortest-length slot of 16 steps, so that with --transforms they
+run in the mixed kernel), every other slot alone, and every other slot plus one slot of the
+longest length with a 16-bit exponent (which with --transforms puts the others in that length's
+workgroup size while adding almost no work). Their milliseconds go into the line as "parts_ms".
 """
 
 import argparse
@@ -64,10 +66,11 @@ def main():
     ap.add_argument("--check", type=int, default=16)
     ap.add_argument("--device", type=int, default=0)
     ap.add_argument("--parts", action="store_true", help="also time the longest length and the rest apart")
+    ap.add_argument("--transforms", action="store_true", help="step by the modular transforms (one mixed launch)")
     args = ap.parse_args()
     moduli, exps = workload(args.count, args.seed, args.min_bits, args.max_bits, args.ebits)
     squarings = sum(e.bit_length() for e in exps)
-    hip = mm.Hip(device=args.device)
+    hip = mm.Hip(device=args.device, prefer_lds=args.transforms)
     t0 = time.perf_counter()
     mix = mm.MixBatch(hip, moduli, 3)
     setup_s = time.perf_counter() - t0
@@ -118,7 +121,8 @@ def main():
         sample.add(rng.randrange(len(moduli)))
     powm_mismatch = sum(0 if mix.check_pow(i, 3, exps[i]) else 1 for i in sorted(sample))
     line = {
-        "metric": "mixed-length squarings/s: one persistent launch vs per-length batches",
+        "metric": "mixed-length squarings/s: lengths together vs one after another",
+        "steps": "modular transforms, one launch" if args.transforms else "each length's step kernel, side by side",
         "workload": f"{len(moduli)} moduli, bits log-uniform in [{args.min_bits}, {args.max_bits}] (seed {args.seed}), "
                     f"base 3, e = top min({args.ebits}, bits) bits of N-1",
         "squarings": squarings,
@@ -144,7 +148,7 @@ def main():
 
 
 def parts(hip, moduli, exps, by_len, ebits):
-    """Kernel milliseconds of the mixed launch on parts of the workload (one untimed pass each)."""
+    """Milliseconds of the mixed run on parts of the workload (one untimed pass each)."""
     longest, shortest = max(by_len), min(by_len)
     big = by_len[longest]
     rest = [i for length, idx in sorted(by_len.items()) if length != longest for i in idx]
@@ -153,8 +157,8 @@ def parts(hip, moduli, exps, by_len, ebits):
     def short(i):  # the top 16 bits of slot i's exponent: 16 steps
         return exps[i] >> max(0, exps[i].bit_length() - 16)
 
-    # One length alone would run its own kernel, so the longest length gets one slot of the
-    # shortest beside it, which keeps it in the mixed launch at the cost of 16 short steps.
+    # The longest length gets one slot of the shortest beside it: with --transforms one length alone
+    # would run its own kernel, and 16 short steps keep it in the mixed launch.
     cases = {
         f"L={longest} ({len(big)} slots) + one L={shortest} slot of 16 steps": (
             [moduli[i] for i in big] + [moduli[tiny]], [exps[i] for i in big] + [short(tiny)]),
